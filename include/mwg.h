@@ -50,7 +50,7 @@ typedef struct mwg_predictor_s *mwg_predictor;
 #define MWG_APPLY_MIXED 1u    /* MFMA slice contractions with split-FP16 operands (hi + lo, 22
                                  significand bits) on f16 MFMA: k = 7 FP32 sums over <= 64 slices,
                                  FP64 beyond; k = 9 every slice's FP32 result summed in FP64.
-                                 Slices with large bounds run as FP64 tuples.  k = 7 and k = 9 only
+                                 Slices with large bounds run in FP64.  k = 7 and k = 9 only
                                  (MWG_ERR_ARG at other orders) */
 #define MWG_APPLY_PREDICT 2u  /* learned refinement predictor (norm test stays the judge; the output
                                  tree can differ from the plain one, see mwg_predictor_create) */
@@ -72,7 +72,8 @@ typedef struct mwg_apply_stats {
     double t_apply;          /* seconds: work-list build + contraction + refine + transforms */
     double t_contract;       /* seconds spent in contraction kernels (device clock: first contraction
                                 workgroup to last reduction workgroup, summed over the iterations) */
-    double flops;            /* flops issued: FP64 tuples * 6 (k+1)^4 + MFMA flops of the slices
+    double flops;            /* FP64 tuples * 6 (k+1)^4 (three passes each; the FP64 contraction shares
+                                passes between tuples and issues fewer) + MFMA flops of the slices
                                 (f16 16x16x32 MFMAs as issued, padding included: k = 7 28 per slice,
                                 2*16*16*32*28, a skipped z half counted; k = 9 90, 2*16*16*32*90) */
     int64_t device_loop;     /* 1: the refinement loop ran on the device (split tests and work lists
@@ -89,8 +90,9 @@ int mwg_ctx_destroy(mwg_ctx ctx);
 const char *mwg_last_error(mwg_ctx ctx);
 int mwg_sync(mwg_ctx ctx);
 /* contraction task granularity (no reference counterpart: MRCPP threads over output
- * nodes with OpenMP): at most this many tuples per FP64 wave task (1..4096; an iteration
- * with fewer than 4096 tasks' worth of tuples uses smaller tasks, down to 16) and MFMA slices per
+ * nodes with OpenMP): at most this many FP64 slices per workgroup task (1..4096; an iteration
+ * with fewer than 2048 tasks' worth of slices uses smaller tasks, down to 8; a task size is
+ * raised where the slots of an iteration would exceed 8 GiB) and MFMA slices per
  * workgroup task (0..4096, 0 = automatic; k = 7 uses at most 256, 128 when automatic;
  * k = 9 sizes automatic tasks from each refinement iteration's slice total, 16 to 128
  * slices, and raises a task size, automatic or set, where the FP64 node slots of an

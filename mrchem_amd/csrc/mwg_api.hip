@@ -272,13 +272,10 @@ struct Ctx {
     DBuf<char> rbd;
     DBuf<int> moves;  // tree compaction: (from, to) node-group pairs
     DBuf<char> iterbuf;  // per-iteration tables (work items, job tables, box requests)
-    DBuf<SegRec> segs;
-    DBuf<int> segcnt;        // per work-list segment: count over all parts
-    DBuf<long long> gslice;  // per output node: first slice
-    TaskCaps caps{1 << 20, 1 << 18, 1 << 15, 1 << 13, 1 << 15, 1 << 15, 1 << 13};
+    DBuf<NodeSched> nodes;  // per output node: its slices and tasks
+    TaskCaps caps{1 << 18, 1 << 18, 1 << 12, 1 << 13};
     DBuf<int> thread_off, gtotal;
     DBuf<long long> gofs;
-    DBuf<Tuple> tuples;
     DBuf<uint64_t> genKeys;
     DBuf<int> genJob, genCount, genOverflow;
     DBuf<double> genPool, genNorm;
@@ -289,17 +286,16 @@ struct Ctx {
     DBuf<TransformItem> titems;
     DBuf<MulItem> mitems;  // batched products: items and work lists of all jobs
     DBuf<int> mwork;
-    DBuf<ContractTask> tasks;
-    DBuf<ReduceItem> reds;
-    DBuf<double> partials, nodeslots;
-    DBuf<Slice> slices;
-    DBuf<SliceTask> stasks;
+    // FP64 slices, tasks and slots; the same for the MFMA slices
+    DBuf<Slice> slices64, slices;
+    DBuf<SliceTask> tasks, stasks;
+    DBuf<double> slots64, nodeslots;
     // refinement traces (features, split label) and the learned predictor
     bool tracing = false;
     std::vector<float> trace_X, trace_y;
     struct PredH *pred = nullptr;
     float pred_thr = 0.5f;
-    int chunk = 64;        // tuples per FP64 contraction task
+    int chunk = 64;        // slices per FP64 contraction task (at most)
     int slice_chunk = 0;   // slices per MFMA task (at most MAX_SLICE_CHUNK; 0: from each iteration's total)
 };
 
@@ -1425,7 +1421,7 @@ static double slice_flops(int K) {
     return 0.0;
 }
 
-// device memory for the FP64 partial slots of one refinement iteration
+// device memory for the task slots of one refinement iteration (per kind of task)
 constexpr double SLOT_BUDGET = 8.0 * (1ull << 30);
 
 // gen_shift: the generated-node tables hold 4 << gen_shift entries per input node, and at
@@ -1631,6 +1627,16 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
     // the same order; the running norm sums the same squares in another order).
     const int njobs = (int)jobs.size();
     bool dl_done = false;
+    auto alloc_schedule = [&]() {  // buffers of the schedule's capacities
+        C.slices64.alloc((size_t)std::max<long long>(C.caps.slices64, 1));
+        C.tasks.alloc((size_t)std::max(C.caps.tasks, 1));
+        C.slots64.alloc((size_t)std::max(C.caps.tasks, 1) * 8 * K3);
+        if (mixed) {
+            C.slices.alloc((size_t)std::max<long long>(C.caps.slices, 1));
+            C.stasks.alloc((size_t)std::max(C.caps.stasks, 1));
+            C.nodeslots.alloc((size_t)std::max(C.caps.stasks, 1) * 8 * K3);
+        }
+    };
 
     auto device_loop = [&]() -> bool {
         const int nr = (int)jobs[0].out->roots.size();
@@ -1685,14 +1691,12 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                 off += cap;
             }
         }
-        const int nseg = mixed ? 9 : 8;
+        const int nseg = mixed ? 2 : 1;
         const size_t eb = (size_t)ENUM_BLOCKS + (size_t)WCAP;  // >= work nodes x parts for any list <= WCAP
-        C.thread_off.alloc(eb * nseg * 256);
+        if (mixed) C.thread_off.alloc(eb * nseg * 256);
         C.gtotal.alloc(eb * nseg);
         C.gofs.alloc(eb * nseg);
-        C.segs.alloc((size_t)WCAP * 8);
-        C.segcnt.alloc((size_t)WCAP * nseg);
-        C.gslice.alloc((size_t)WCAP);
+        C.nodes.alloc((size_t)WCAP);
         C.lwork[0].alloc((size_t)WCAP);
         C.lwork[1].alloc((size_t)WCAP);
         C.lcidx.alloc((size_t)WCAP);
@@ -1717,15 +1721,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                           : (C.slice_chunk > 0 ? std::max(C.slice_chunk, C.hw_schunk[d])
                                                : (C.hw_schunk[d] > 0 ? C.hw_schunk[d] : -2048));
         };
-        C.tuples.alloc((size_t)std::max<long long>(C.caps.tuples, 1));
-        C.tasks.alloc((size_t)std::max(C.caps.tasks, 1));
-        C.reds.alloc((size_t)std::max(C.caps.reds, 1));
-        C.partials.alloc((size_t)std::max(C.caps.slots, 1) * K3);
-        if (mixed) {
-            C.slices.alloc((size_t)std::max<long long>(C.caps.slices, 1));
-            C.stasks.alloc((size_t)std::max(C.caps.stasks, 1));
-            C.nodeslots.alloc((size_t)std::max(C.caps.nnslots, 1) * 8 * K3);
-        }
+        alloc_schedule();
         // schedule summary | table counts | work-node norms
         const size_t o_tab = 256;
         const size_t o_wn = (o_tab + 4 * (size_t)njobs * sizeof(long long) + 255) & ~(size_t)255;
@@ -1826,36 +1822,31 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                 HC(launch_split16(s, genPoolCap, 0, C.genCount.p, K3, K, C.genPool.p, C.genPool16.p, C.genExp16.p, 1,
                                   gfirst));
             if (!mixed)
-                HC(launch_enum(s, 0, WCAP, 0, dw, djt, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, nullptr, nullptr,
-                               nullptr, nullptr, nwp, queue + 1));
+                HC(launch_enum(s, 0, K, WCAP, 0, dw, djt, C.tabs.p, gs, C.gtotal.p, nullptr, nullptr, nullptr, nullptr,
+                               nullptr, nwp, queue + 1));
             else
                 HC(launch_enum_mixed(s, 0, K, WCAP, 0, dw, djt, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, nullptr,
-                                     nullptr, nullptr, nullptr, nullptr, nullptr, nwp, queue + 1));
-            HC(launch_build_tasks(s, WCAP, nseg, 0, chunk_dl(d), schunk_dl(d), C.gtotal.p, C.caps, C.genCount.p, genPoolCap,
-                                  C.gofs.p, C.tasks.p, C.stasks.p, C.reds.p, dsum, C.segs.p, C.segcnt.p, C.gslice.p,
-                                  C.genOverflow.p, dw, dtab, njobs, nwp));
+                                     nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nwp, queue + 1));
+            HC(launch_build_tasks(s, WCAP, nseg, 0, chunk_dl(d), schunk_dl(d), C.gtotal.p, C.caps, C.genCount.p,
+                                  genPoolCap, C.gofs.p, C.nodes.p, dsum, C.genOverflow.p, nwp));
             if (!mixed)
-                HC(launch_enum(s, 1, WCAP, 0, dw, djt, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, C.gofs.p, C.tuples.p,
-                               dsum, C.segs.p, nwp, queue + 2));
+                HC(launch_enum(s, 1, K, WCAP, 0, dw, djt, C.tabs.p, gs, C.gtotal.p, C.gofs.p, C.slices64.p, dsum,
+                               C.nodes.p, C.tasks.p, nwp, queue + 2));
             else
                 HC(launch_enum_mixed(s, 1, K, WCAP, 0, dw, djt, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, C.gofs.p,
-                                     C.tuples.p, C.slices.p, dsum, C.segs.p, C.gslice.p, nwp, queue + 2));
-            const int grid64 = std::max(1, (C.caps.tasks + 3) / 4);
-            const int gridred = std::min(4096, std::max(1, C.caps.reds));
-            HC(launch_contract_fp64(s, K, 0, dsum, grid64, C.tasks.p, dw, djt, C.tabs.p, C.tuples.p, C.genPool.p,
-                                    C.partials.p, dts));
+                                     C.slices64.p, C.slices.p, dsum, C.nodes.p, C.tasks.p, C.stasks.p, nwp, queue + 2));
+            HC(launch_contract_slices64(s, K, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dw, djt, C.slices64.p,
+                                        C.genPool.p, C.slots64.p, dts));
             if (mixed) {
                 const int tpb = mfma_tasks_per_block(K);
                 const int gridmf = std::max(1, (C.caps.stasks + tpb - 1) / tpb);
                 HC(launch_contract_mfma(s, K, 0, dsum, gridmf, C.stasks.p, dw, djt, C.tabs.p, C.slices.p, C.genPool.p,
                                         C.nodeslots.p, dtab, C.genPool16.p, C.genExp16.p));
             }
-            HC(launch_reduce_partials(s, 0, dsum, gridred, C.reds.p, dw, djt, C.partials.p,
-                                      mixed ? C.nodeslots.p : nullptr, K3, mixed ? dwn : nullptr));
+            HC(launch_reduce_slots(s, WCAP, nwp, dsum, C.nodes.p, dw, djt, C.slots64.p, C.nodeslots.p, K3, dwn));
             // (the kernel after the reduction stamps the contraction's end)
-            if (!mixed) HC(launch_work_norms(s, WCAP, dw, djt, K3, dwn, nwp, dts + 1));
             HC(launch_loop_split(s, njobs, C.ljobs.p, dw, dwn, M.maxDepth, C.lctl.p, C.lcidx.p, dtab,
-                                 mixed ? dts + 1 : nullptr));
+                                 dts + 1));
             HC(launch_loop_emit(s, njobs, C.ljobs.p, dw, nwp, C.lcidx.p, C.lwork[cur ^ 1].p, nwnext, WCAP, dsum,
                                 C.lctl.p, d, djt, C.titems.p, tcap, C.liter_d));
             HC(hipEventRecord(C.evIter[d], s));  // (k_loop_emit wrote the host's entry d)
@@ -2090,45 +2081,32 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         // the norms, the schedule sizes and the counts back once.  When a capacity (or
         // the generated-node pool) was too small, nothing of the schedule ran: grow and
         // run it again.
-        const int nseg = mixed ? 9 : 8;
+        const int nseg = mixed ? 2 : 1;
         // few output nodes (the roots): several workgroups share each node's candidates
         const int nparts = enum_parts(nw);
-        C.thread_off.alloc((size_t)nw * nseg * nparts * 256);
+        if (mixed) C.thread_off.alloc((size_t)nw * nseg * nparts * 256);
         C.gtotal.alloc((size_t)nw * nseg * nparts);
         C.gofs.alloc((size_t)nw * nseg * nparts);
-        C.segs.alloc((size_t)nw * 8);
-        C.segcnt.alloc((size_t)nw * nseg);
-        C.gslice.alloc((size_t)nw);
+        C.nodes.alloc((size_t)nw);
         auto launch_count = [&]() {
             if (!mixed)
-                HC(launch_enum(s, 0, nw, nparts, dwork, djobs, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, nullptr,
-                               nullptr, nullptr, nullptr));
+                HC(launch_enum(s, 0, K, nw, nparts, dwork, djobs, C.tabs.p, gs, C.gtotal.p, nullptr, nullptr, nullptr,
+                               nullptr, nullptr));
             else
                 HC(launch_enum_mixed(s, 0, K, nw, nparts, dwork, djobs, C.tabs.p, gs, C.thread_off.p, C.gtotal.p,
-                                     nullptr, nullptr, nullptr, nullptr, nullptr, nullptr));
+                                     nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr));
         };
         auto ensure_caps = [&](const TaskSummary *need) {
             auto grow = [](long long have, long long want) {
                 return want <= have ? have : std::max<long long>(want + want / 4, 1024);
             };
             if (need) {
-                C.caps.tuples = grow(C.caps.tuples, need->ntuples);
+                C.caps.slices64 = grow(C.caps.slices64, need->nslices64);
                 C.caps.slices = grow(C.caps.slices, need->nslices);
                 C.caps.tasks = (int)grow(C.caps.tasks, need->ntasks);
                 C.caps.stasks = (int)grow(C.caps.stasks, need->nstasks);
-                C.caps.reds = (int)grow(C.caps.reds, need->nreds);
-                C.caps.slots = (int)grow(C.caps.slots, need->nslots);
-                C.caps.nnslots = (int)grow(C.caps.nnslots, need->nnslots);
             }
-            C.tuples.alloc((size_t)std::max<long long>(C.caps.tuples, 1));
-            C.tasks.alloc((size_t)std::max(C.caps.tasks, 1));
-            C.reds.alloc((size_t)std::max(C.caps.reds, 1));
-            C.partials.alloc((size_t)std::max(C.caps.slots, 1) * K3);
-            if (mixed) {
-                C.slices.alloc((size_t)std::max<long long>(C.caps.slices, 1));
-                C.stasks.alloc((size_t)std::max(C.caps.stasks, 1));
-                C.nodeslots.alloc((size_t)std::max(C.caps.nnslots, 1) * 8 * K3);
-            }
+            alloc_schedule();
         };
         std::vector<double> wn((size_t)nw * 8);
         std::vector<long long> tabcnt(4 * jt.size());
@@ -2136,7 +2114,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         std::vector<float> cfeat(C.tracing ? (size_t)nw * 8 * MLP_FEATURES : 0);
         TaskSummary hsum;
         unsigned long long hts[2] = {0ull, 0ull};
-        int chunk_it = C.chunk;  // FP64 task size of this iteration (raised when partial slots would not fit)
+        int chunk_it = C.chunk;  // FP64 task size of this iteration (raised when its slots would not fit)
         // slices per MFMA task (a workgroup task).  k = 7: at most MFMA8_TASK_SLICES (the
         // waves sum a quarter of them each in FP32), MFMA8_TASK_DEFAULT when automatic;
         // k = 9: about 2048 tasks per iteration when automatic (16 to 128 slices each),
@@ -2146,32 +2124,26 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         auto launch_schedule = [&]() {
             ensure_caps(nullptr);
             HC(launch_build_tasks(s, nw, nseg, nparts, chunk_it, schunk_it, C.gtotal.p, C.caps, C.genCount.p,
-                                  genPoolCap, C.gofs.p, C.tasks.p, C.stasks.p, C.reds.p, dsum, C.segs.p,
-                                  C.segcnt.p, C.gslice.p, C.genOverflow.p, dwork, dtab, (int)jt.size()));
+                                  genPoolCap, C.gofs.p, C.nodes.p, dsum, C.genOverflow.p));
             if (!mixed)
-                HC(launch_enum(s, 1, nw, nparts, dwork, djobs, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, C.gofs.p,
-                               C.tuples.p, dsum, C.segs.p));
+                HC(launch_enum(s, 1, K, nw, nparts, dwork, djobs, C.tabs.p, gs, C.gtotal.p, C.gofs.p, C.slices64.p,
+                               dsum, C.nodes.p, C.tasks.p));
             else
                 HC(launch_enum_mixed(s, 1, K, nw, nparts, dwork, djobs, C.tabs.p, gs, C.thread_off.p, C.gtotal.p,
-                                     C.gofs.p, C.tuples.p, C.slices.p, dsum, C.segs.p, C.gslice.p));
-            const int grid64 = std::max(1, (C.caps.tasks + 3) / 4);
-            const int gridred = std::min(4096, std::max(1, C.caps.reds));
+                                     C.gofs.p, C.slices64.p, C.slices.p, dsum, C.nodes.p, C.tasks.p, C.stasks.p));
             // contraction time: the device clock at the first workgroup of the first and the
             // last workgroup of the last contraction kernel
-            HC(launch_contract_fp64(s, K, 0, dsum, grid64, C.tasks.p, dwork, djobs, C.tabs.p, C.tuples.p,
-                                    C.genPool.p, C.partials.p, dts));
+            HC(launch_contract_slices64(s, K, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dwork, djobs,
+                                        C.slices64.p, C.genPool.p, C.slots64.p, dts));
             if (mixed) {
                 const int tpb = mfma_tasks_per_block(K);
                 const int gridmf = std::max(1, (C.caps.stasks + tpb - 1) / tpb);
                 HC(launch_contract_mfma(s, K, 0, dsum, gridmf, C.stasks.p, dwork, djobs, C.tabs.p, C.slices.p,
                                         C.genPool.p, C.nodeslots.p, dtab, C.genPool16.p, C.genExp16.p));
             }
-            // (mixed: the reduce items cover every output component and write the norms)
-            HC(launch_reduce_partials(s, 0, dsum, gridred, C.reds.p, dwork, djobs, C.partials.p,
-                                      mixed ? C.nodeslots.p : nullptr, K3, mixed ? dwn : nullptr));
-            // (the contraction's end: stamped by the next kernel on the stream)
-            if (!mixed) HC(launch_work_norms(s, nw, dwork, djobs, K3, dwn, nullptr, dts + 1));
-            else HC(launch_stamp(s, dts + 1));
+            HC(launch_reduce_slots(s, nw, nullptr, dsum, C.nodes.p, dwork, djobs, C.slots64.p, C.nodeslots.p, K3,
+                                   dwn));
+            HC(launch_stamp(s, dts + 1));  // the contraction's end
             // refinement predictor: features of every work node's children and their split
             // probabilities, read back with the norms (no extra round trip)
             if (want_feat) {
@@ -2220,18 +2192,19 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                                       C.genPool16.p, C.genExp16.p, 1));
                 }
                 genPoolCap = want;
+                // (the counts are taken anew; entries 4 t + 3 hold the generated nodes: kept)
+                HC(hipMemset2DAsync(dtab, 4 * sizeof(long long), 0, 3 * sizeof(long long), jt.size(), s));
                 launch_count();
             }
             TaskSummary need = hsum;
-            if ((double)need.nslots * K3 * sizeof(double) > SLOT_BUDGET && chunk_it < 4096) {
-                // twice the task size; the slot capacity stays, the next schedule tells
-                chunk_it *= 2;
-                need.nslots = 0;
+            if ((double)need.ntasks * 8 * K3 * sizeof(double) > SLOT_BUDGET && chunk_it < 4096) {
+                // twice the task size; the capacity stays, the next schedule tells
+                chunk_it = std::min(4096, 2 * chunk_it);
+                need.ntasks = 0;
             }
-            if (K != 8 && (double)need.nnslots * 8 * K3 * sizeof(double) > SLOT_BUDGET &&
+            if (K != 8 && (double)need.nstasks * 8 * K3 * sizeof(double) > SLOT_BUDGET &&
                 hsum.schunk < MAX_SLICE_CHUNK) {
-                schunk_it = 2 * hsum.schunk;  // the same for the MFMA tasks' node slots
-                need.nnslots = 0;
+                schunk_it = 2 * hsum.schunk;  // the same for the MFMA tasks
                 need.nstasks = 0;
             }
             ensure_caps(&need);
@@ -2255,9 +2228,9 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                 cand += pre[(size_t)T.tab0 + work[i].job + T.ntab];
             }
             fprintf(stderr,
-                    "[mwg timing] iteration %d: %d work nodes, %lld candidates, %lld tuples, %lld slices, %d generated "
+                    "[mwg timing] iteration %d: %d work nodes, %lld candidates, %lld FP64 slices, %lld MFMA slices, %d generated "
                     "(pool %d)\n",
-                    iter, nw, cand, hsum.ntuples, hsum.nslices, genLastNew, genPoolCap);
+                    iter, nw, cand, hsum.nslices64, hsum.nslices, genLastNew, genPoolCap);
         }
         for (size_t q = 0; q < jt.size(); q++) {
             JobH &J = jobs[jt_job[q]];

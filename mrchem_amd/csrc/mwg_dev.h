@@ -53,22 +53,11 @@ struct TermTab {
     unsigned long long bm[3][BM];
 };
 
-// one surviving (g, f, ft, gt, term) tuple
-struct Tuple {
-    int g;          // index into the work list
-    int f;          // input node index (>= 0) or -(generated index + 1)
-    uint8_t term;   // index into the TermTab array
-    uint8_t combo;  // gt * 8 + ft
-    int16_t dx, dy, dz;
-};
-static_assert(sizeof(Tuple) == 16, "tuple record is 16 bytes");
-
-// one (g, f, ft, term) slice of the mixed-precision apply: all 8 output
-// components at once (mask: which gt are accumulated)
-// one MFMA slice (g, f, ft, term): every output component gt of node g from component ft
-// of input node f, with the operator blocks already resolved: xo, yo, zo are the offsets
-// (in block values) of the (gt_d = 0, ft_d) block of each dimension in the level's block
-// array (the gt_d = 1 block follows 2 (k+1)^2 values later)
+// one slice (g, f, ft, term): every surviving output component gt of node g (mask) from
+// component ft of input node f, with the operator blocks already resolved: xo, yo, zo are the
+// (gt_d = 0, ft_d) block of each dimension in the level's block array (the gt_d = 1 block
+// follows two blocks later): its index in FP64 slices, the offset of its first value in MFMA
+// slices.  Every surviving (g, f, ft, gt, term) combination (tuple) is one mask bit.
 struct Slice {
     double w;      // term weight
     int f;         // input node index (>= 0) or -(generated index + 1)
@@ -79,7 +68,7 @@ struct Slice {
 };
 static_assert(sizeof(Slice) == 32, "slice record is 32 bytes");
 
-// a slice is contracted in FP64 (as tuples) when its largest bound exceeds
+// a slice is contracted in FP64 when its largest bound exceeds
 // ROUTE_FP64 = 2^21 times the screening threshold thr: the FP32 rounding of a slice
 // (~8 * 2^-24 of its bound) then stays below thr, the size of every tuple the
 // screening drops

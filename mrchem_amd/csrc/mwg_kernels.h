@@ -6,6 +6,19 @@
 #include "mwg_core.h"
 #include "mwg_dev.h"
 
+// CALL with KK = K as a constant, for the orders the library is built for
+#define MWG_DISPATCH_K(K, CALL)                                       \
+    switch (K) {                                                      \
+        case 4: { constexpr int KK = 4; CALL; } break;                \
+        case 5: { constexpr int KK = 5; CALL; } break;                \
+        case 6: { constexpr int KK = 6; CALL; } break;                \
+        case 7: { constexpr int KK = 7; CALL; } break;                \
+        case 8: { constexpr int KK = 8; CALL; } break;                \
+        case 9: { constexpr int KK = 9; CALL; } break;                \
+        case 10: { constexpr int KK = 10; CALL; } break;              \
+        default: return hipErrorInvalidValue;                         \
+    }
+
 namespace mwg {
 
 constexpr double GAUSS_CUT_D = GAUSS_CUT;
@@ -70,15 +83,22 @@ struct JobTab {
 // generated-node pool did not hold every generated node, and then no kernel of the
 // schedule runs).
 struct TaskSummary {
-    long long ntuples, nslices;
-    int ntasks, nstasks, nreds, nslots, nnslots;
+    long long nslices64, nslices;  // FP64 and MFMA slices
+    int ntasks, nstasks;           // their tasks (one slot of 8 K^3 doubles each)
     int overflow;  // bit 0: a capacity below, bit 1: generated-node pool
     int gen_count, gen_overflow;  // generated-node counter and table-overflow flag, for the host
-    int schunk;                   // slices per MFMA task used by the schedule (mixed)
+    int chunk, schunk;            // slices per FP64 and MFMA task used by the schedule
 };
 struct TaskCaps {
-    long long tuples, slices;
-    int tasks, stasks, reds, slots, nnslots;
+    long long slices64, slices;
+    int tasks, stasks;
+};
+// an output node's slices and tasks: FP64 (64) and split-FP16 MFMA (16); a task's slot has its
+// index
+struct NodeSched {
+    long long start64, start16;
+    int count64, count16;
+    int task64, task16;  // first tasks
 };
 
 // one Gaussian term of one operator level, as the screening-box kernel reads it
@@ -175,23 +195,26 @@ hipError_t launch_gen_mark(hipStream_t s, int nw, const WorkItem *work, const Jo
 // firstp: first read on the device)
 hipError_t launch_gen_compute(hipStream_t s, int first, int cap, const JobTab *jobs, const GenState &gs,
                               const double *W, int K, const int *firstp = nullptr);
-// per tuple segment (output node, component): first tuple, count, first FP64 task, first
-// partial slot (-1: its single task writes the output directly)
-struct SegRec {
+// A task: a run of slices of one output node (one workgroup, one slot of 8 K^3 doubles)
+struct SliceTask {
     long long start;
     int count;
-    int task0;
-    int slot0;
-    int pad_stask0;  // on component 0 of a node: its first slice task (mixed)
+    int g;     // work index
+    int slot;
 };
 // nparts workgroups share each output node's candidates (counts and offsets per
-// (node, segment, part))
-hipError_t launch_enum(hipStream_t s, int mode, int nw, int nparts, const WorkItem *work, const JobTab *jobs,
-                       const TermTab *tabs, const GenState &gs, int *thread_off, int *seg_total,
-                       const long long *seg_ofs, Tuple *out, const TaskSummary *sum, const SegRec *segs,
-                       const int *nwp = nullptr, int *queue = nullptr);
-hipError_t launch_work_norms(hipStream_t s, int nw, const WorkItem *work, const JobTab *jobs, int K3,
-                             double *compact, const int *nwp = nullptr, unsigned long long *ts_end = nullptr);
+// (node, segment, part)); mode 0 counts (and adds the jobs' statistics), mode 1 writes the
+// slices and tasks.  Plain method: one segment, the FP64 slices.
+hipError_t launch_enum(hipStream_t s, int mode, int K, int nw, int nparts, const WorkItem *work, const JobTab *jobs,
+                       const TermTab *tabs, const GenState &gs, int *seg_total, const long long *seg_ofs, Slice *out,
+                       const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks, const int *nwp = nullptr,
+                       int *queue = nullptr);
+// FP64 slice contraction (mwg_fp64.hip).  With sum: the task count is read on the device; grid
+// (tasks) covers the capacity.  With ts: an extra first workgroup stamps the start.
+hipError_t launch_contract_slices64(hipStream_t s, int K, int ntask, const TaskSummary *sum, int grid,
+                                    const SliceTask *tasks, const WorkItem *work, const JobTab *jobs,
+                                    const Slice *slices, const double *genPool, double *slots,
+                                    unsigned long long *ts = nullptr);
 // the device clock into *t (one thread; marks the end of the kernels before it on the stream)
 hipError_t launch_stamp(hipStream_t s, unsigned long long *t);
 struct TransformItem {
@@ -201,30 +224,11 @@ struct TransformItem {
     int first_child;
 };
 hipError_t launch_transform(hipStream_t s, int mode, int n, const TransformItem *items, const double *M, int K);
-// one wavefront task: a chunk of the tuples of segment (g, gt)
-struct ContractTask {
-    long long start;
-    int count;
-    int g;     // work index
-    int gt;
-    int slot;  // partial slot, -1 = write the output node directly
-};
-struct ReduceItem {
-    int g, gt, slot0, nslots;  // K^3 slots of FP64 tuple tasks
-    int nslot0, nnslots;       // 8 K^3 node slots of mixed-precision slice tasks
-};
-struct SliceTask {
-    long long start;
-    int count;
-    int g;
-    int slot;  // node slot (8 K^3 doubles)
-};
 hipError_t launch_enum_mixed(hipStream_t s, int mode, int K, int nw, int nparts, const WorkItem *work,
-                             const JobTab *jobs,
-                             const TermTab *tabs, const GenState &gs, int *thread_off, int *seg_total,
-                             const long long *seg_ofs, Tuple *out, Slice *sout, const TaskSummary *sum,
-                             const SegRec *segs, const long long *gslice, const int *nwp = nullptr,
-                             int *queue = nullptr);
+                             const JobTab *jobs, const TermTab *tabs, const GenState &gs, int *thread_off,
+                             int *seg_total, const long long *seg_ofs, Slice *out64, Slice *out16,
+                             const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks, SliceTask *stasks,
+                             const int *nwp = nullptr, int *queue = nullptr);
 // Split-FP16 copies of FP64 blocks (mwg_mfma.hip): block b (values src[b bvals ..]) as rows
 // of K values, scaled by 2^exp[b] so that the block's largest magnitude lies in [0.5, 1)
 // (exp 0 for a zero block); x 2^e = hi + lo up to about 2^-23 of it.  K = 8: each row
@@ -267,14 +271,12 @@ hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const Pro
                            double coef, const double *acoef, const double *bcoef, double *out);
 hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const DevBasis &B, double ca, const double *acoef,
                       double cb, const double *bcoef, double *out);
-// from the per-segment counts (nseg = 8: plain FP64, 9: mixed): segment offsets, FP64
-// tasks (full chunks first), MFMA slice tasks, reduce items, slot numbering.  wchunk:
-// slices per MFMA task, or (<= 0) about -wchunk tasks over the iteration's slices.
+// from the per-(node, segment, part) counts (nseg = 1: plain FP64, 2: mixed): part offsets,
+// task sizes, every node's first slices and tasks.  wchunk: slices per MFMA task, or (<= 0)
+// about -wchunk tasks over the iteration's slices.
 hipError_t launch_build_tasks(hipStream_t s, int nw, int nseg, int nparts, int chunk, int wchunk, const int *tot,
-                              TaskCaps caps, const int *gen_count, int gen_pcap, long long *ofs, ContractTask *tasks,
-                              SliceTask *stasks, ReduceItem *reds, TaskSummary *sum, SegRec *segs, int *segcnt,
-                              long long *gslice, const int *gen_overflow, const WorkItem *work, long long *tabcnt,
-                              int ntab, const int *nwp = nullptr);
+                              TaskCaps caps, const int *gen_count, int gen_pcap, long long *ofs, NodeSched *nodes,
+                              TaskSummary *sum, const int *gen_overflow, const int *nwp = nullptr);
 // ---- device-resident refinement (mwg_kernels.hip)
 // The plain method's refinement loop without a host round trip: every job of the batch has
 // one job table per iteration (table index = job index, all work nodes of iteration d at
@@ -327,14 +329,10 @@ hipError_t launch_loop_emit(hipStream_t s, int njobs, LoopJob *lj, const WorkIte
 // input tree around each child
 hipError_t launch_child_features(hipStream_t s, int nw, const WorkItem *work, const JobTab *jobs,
                                  const double *wnorms, float *feat);
-// with sum: the task count is read on the device; grid (blocks) covers the capacity
-hipError_t launch_contract_fp64(hipStream_t s, int K, int ntask, const TaskSummary *sum, int grid,
-                                const ContractTask *tasks, const WorkItem *work, const JobTab *jobs,
-                                const TermTab *tabs, const Tuple *tuples, const double *genPool, double *partials,
-                                unsigned long long *ts = nullptr);
 hipError_t launch_move_groups(hipStream_t s, int npairs, const int *from_to, double *coef, double *norm, int nb);
-hipError_t launch_reduce_partials(hipStream_t s, int n, const TaskSummary *sum, int grid, const ReduceItem *items,
-                                  const WorkItem *work, const JobTab *jobs, const double *partials,
-                                  const double *nodeslots, int K3, double *wnorm = nullptr);
+// output components (and their norms, also to wnorm) from the task slots
+hipError_t launch_reduce_slots(hipStream_t s, int nw, const int *nwp, const TaskSummary *sum, const NodeSched *nodes,
+                               const WorkItem *work, const JobTab *jobs, const double *slots64, const double *slots16,
+                               int K3, double *wnorm);
 
 }  // namespace mwg

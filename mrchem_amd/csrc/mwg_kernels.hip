@@ -908,13 +908,16 @@ __device__ inline void term_prefix(CandTerms &ct, const JobTab &J, const TermTab
     (void)tabs;
 }
 
+// the candidates of part of nparts workgroups that share an output node
+__device__ inline void part_range(int total, int part, int nparts, int &k0, int &k1) {
+    k0 = (int)((long long)total * part / nparts);
+    k1 = (int)((long long)total * (part + 1) / nparts);
+}
+
 template <class Visit>
 __device__ inline void walk_candidates(const CandTerms &ct, const int *fcache, const FCache &fc, const WorkItem &wi,
-                                       const JobTab &J, const TermTab *tabs, const GenState &gs, int part, int nparts,
+                                       const JobTab &J, const TermTab *tabs, const GenState &gs, int k0, int k1,
                                        Visit &&visit) {
-    const int total = ct.start[J.ntab];
-    // part of nparts workgroups that share this output node: a contiguous candidate range
-    const int k0 = (int)((long long)total * part / nparts), k1 = (int)((long long)total * (part + 1) / nparts);
     for (int k = k0 + threadIdx.x; k < k1; k += blockDim.x) {
         int lo = 0, hi = J.ntab - 1;  // last t with start[t] <= k
         while (lo < hi) {
@@ -932,14 +935,12 @@ __device__ inline void walk_candidates(const CandTerms &ct, const int *fcache, c
         const int f = lookup_f(fcache, fc, wi, J, gs, dx, dy, dz);
         if (f == INT_MIN) continue;
         double fn[8];
-        int nft = 8;
         if (f >= 0) {
             for (int q = 0; q < 8; q++) fn[q] = J.inNorm[(size_t)f * 8 + q];
         } else {
             // an entry past the allocated pool (its count is redone after the pool grows)
             fn[0] = -f - 1 < gs.pcap ? gs.norm[-f - 1] : 0.0;
             for (int q = 1; q < 8; q++) fn[q] = 0.0;  // (no wavelet part: no bound above thr >= 0)
-            nft = 1;
         }
         const double *nrm = J.operNorms + tb.nrm;
         double nx[4], ny[4], nz[4];
@@ -948,7 +949,7 @@ __device__ inline void walk_candidates(const CandTerms &ct, const int *fcache, c
             ny[q] = nrm[(dy + tb.band) * 4 + q];
             nz[q] = nrm[(dz + tb.band) * 4 + q];
         }
-        visit(t, tb, dx, dy, dz, f, fn, nft, nx, ny, nz);
+        visit(k, t, tb, dx, dy, dz, f, fn, nx, ny, nz);
     }
 }
 
@@ -1134,98 +1135,183 @@ __global__ void __launch_bounds__(64) k_job_route(int nbj, const BoxJob *bjs, co
 
 // ----------------------------------------------------------------- apply: work list
 
-// Enumerates, for one output node, every (term, delta, ft, gt) candidate inside the
-// screened boxes and keeps those whose bound |w| prod_d ||X_d|| ||f_ft|| exceeds the
-// job threshold.  Tuples are laid out by segment (g, gt):
-//   mode 0 counts per (thread, gt), scans over the block and writes per-thread
-//          offsets inside each segment and the segment totals;
-//   mode 1 writes every tuple at the segment's start (from the schedule) + the part's
-//          offset inside the segment + thread offset + running index.
+// Enumerates, for one output node, every (term, delta, ft, gt) candidate inside the screened
+// boxes and keeps the combinations whose bound |w| prod_d ||X_d|| ||f_ft|| exceeds the job
+// threshold; the surviving gt of a (term, delta, ft) make one slice.
+//   mode 0 counts the slices of the part (and the job's tuples);
+//   mode 1 writes them from the node's start (from the schedule) + the part's offset, and
+//          the node's tasks (part 0).
+// The contraction shares its y and z passes between neighbours in the list, so the slices of
+// a term go in the order (dz, ft_z, dy, ft_y, dx, ft_x).  Candidates come in the order (term, dz,
+// dy, dx), every one with its 8 ft: ENUM_CHUNK of them at a time are screened into LDS (8 masks
+// each), their slices counted per (candidate, ft_z, ft_y) in the order of the list, and the
+// prefix of these counts gives every slice its place.  (A plane (term, dz) that a chunk or a
+// part cuts is ordered within each piece: the runs are shorter there.)
+constexpr int ENUM_CHUNK = 1024;
+
+// the node's tasks: at most chunk slices each (slot = task index)
+__device__ __forceinline__ void emit_tasks(int g, long long start, int count, int chunk, int task0, SliceTask *tasks) {
+    const int n = (count + chunk - 1) / chunk;
+    for (int h = threadIdx.x; h < n; h += blockDim.x)
+        tasks[task0 + h] = SliceTask{start + (long long)h * chunk, min(chunk, count - h * chunk), g, task0 + h};
+}
+
+__device__ inline int block_sum_256i(int v, int *wsum) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+}
+
 template <int MODE>
-__device__ __forceinline__ void enum_node(int g, int part, int nparts, const WorkItem *work, const JobTab *jobs,
-                                          const TermTab *tabs, const GenState &gs, int *thread_off,
-                                          int *seg_total, const long long *seg_ofs, Tuple *out,
-                                          const SegRec *segs) {
+__device__ __forceinline__ void enum_node(int g, int part, int nparts, int K2, const WorkItem *work,
+                                          const JobTab *jobs, const TermTab *tabs, const GenState &gs, int *seg_total,
+                                          const long long *seg_ofs, Slice *out, const TaskSummary *sum,
+                                          const NodeSched *nodes, SliceTask *tasks) {
     const WorkItem wi = work[g];
     const JobTab &J = jobs[wi.job];
-    __shared__ int scan[8][256];
     __shared__ int fcache[FCACHE];
     __shared__ CandTerms ct;
+    __shared__ int wsum[4];
+    __shared__ uint2 smask[MODE == 1 ? ENUM_CHUNK : 1];
+    __shared__ __align__(16) unsigned short place[MODE == 1 ? 4 * ENUM_CHUNK : 1];
     const FCache fc = fill_fcache(fcache, wi, J, tabs, gs);
     term_prefix(ct, J, tabs);
-    int cnt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    long long base[8];
-    if (MODE == 1)
-        for (int q = 0; q < 8; q++) {
-            const size_t sp = ((size_t)g * 8 + q) * nparts + part;  // (segment, part)
-            base[q] = segs[(size_t)g * 8 + q].start + (nparts > 1 ? seg_ofs[sp] : 0) +
-                      thread_off[sp * 256 + threadIdx.x];
-        }
-    walk_candidates(ct, fcache, fc, wi, J, tabs, gs, part, nparts,
-                    [&](int t, const TermTab &tb, int dx, int dy, int dz, int f, const double *fn, int nft,
-                        const double *nx, const double *ny, const double *nz) {
-                        const double aw = fabs(tb.w);
-                        const unsigned long long cm = combo_mask(tb, dx, dy, dz);
-                        unsigned surv[8];
-                        double maxb[8];
-                        screen_candidate<false>(aw, nx, ny, nz, fn, cm, J.thr, surv, maxb);
-                        (void)nft;
-                        if (MODE == 0) {
-#pragma unroll
-                            for (int ft = 0; ft < 8; ft++)
-#pragma unroll
-                                for (int gt = 0; gt < 8; gt++) cnt[gt] += (surv[ft] >> gt) & 1u;
-                        } else {
-                            // per gt (static index of base and cnt) its surviving ft, in order
-#pragma unroll
-                            for (int gt = 0; gt < 8; gt++) {
-                                unsigned sg = 0u;
-#pragma unroll
-                                for (int ft = 0; ft < 8; ft++) sg |= ((surv[ft] >> gt) & 1u) << ft;
-                                for (unsigned m = sg; m; m &= m - 1) {
-                                    const int ft = __builtin_ctz(m);
-                                    Tuple tp;
-                                    tp.g = g;
-                                    tp.f = f;
-                                    tp.term = (uint8_t)t;
-                                    tp.combo = (uint8_t)(gt * 8 + ft);
-                                    tp.dx = (int16_t)dx;
-                                    tp.dy = (int16_t)dy;
-                                    tp.dz = (int16_t)dz;
-                                    out[base[gt] + cnt[gt]] = tp;
-                                    cnt[gt]++;
-                                }
-                            }
-                        }
-                    });
+    int k0, k1;
+    part_range(ct.start[J.ntab], part, nparts, k0, k1);
     if (MODE == 0) {
-        for (int q = 0; q < 8; q++) scan[q][threadIdx.x] = cnt[q];
-        __syncthreads();
-        for (int off = 1; off < 256; off <<= 1) {
-            int v[8];
-            for (int q = 0; q < 8; q++) v[q] = threadIdx.x >= off ? scan[q][threadIdx.x - off] : 0;
-            __syncthreads();
-            for (int q = 0; q < 8; q++) scan[q][threadIdx.x] += v[q];
-            __syncthreads();
+        int ns = 0, nt = 0;
+        walk_candidates(ct, fcache, fc, wi, J, tabs, gs, k0, k1,
+                        [&](int k, int t, const TermTab &tb, int dx, int dy, int dz, int f, const double *fn,
+                            const double *nx, const double *ny, const double *nz) {
+                            unsigned surv[8];
+                            double maxb[8];
+                            screen_candidate<false>(fabs(tb.w), nx, ny, nz, fn, combo_mask(tb, dx, dy, dz), J.thr, surv,
+                                                    maxb);
+#pragma unroll
+                            for (int ft = 0; ft < 8; ft++) {
+                                ns += surv[ft] ? 1 : 0;
+                                nt += __popc(surv[ft]);
+                            }
+                        });
+        ns = block_sum_256i(ns, wsum);
+        nt = block_sum_256i(nt, wsum);
+        if (threadIdx.x == 0) {
+            seg_total[(size_t)g * nparts + part] = ns;
+            if (nt) atomicAdd((unsigned long long *)&gs.tabcnt[4 * wi.job], (unsigned long long)nt);
         }
-        for (int q = 0; q < 8; q++)
-            thread_off[(((size_t)g * 8 + q) * nparts + part) * 256 + threadIdx.x] = scan[q][threadIdx.x] - cnt[q];
-        if (threadIdx.x == 255)
-            for (int q = 0; q < 8; q++) seg_total[((size_t)g * 8 + q) * nparts + part] = scan[q][255];
+        return;
+    }
+    const NodeSched nd = nodes[g];
+    if (part == 0) emit_tasks(g, nd.start64, nd.count64, sum->chunk, nd.task64, tasks);
+    long long base = nd.start64 + (nparts > 1 ? seg_ofs[(size_t)g * nparts + part] : 0);
+    for (int kc = k0; kc < k1; kc += ENUM_CHUNK) {
+        const int ke = min(k1, kc + ENUM_CHUNK), n = ke - kc;
+        for (int q = threadIdx.x; q < n; q += 256) smask[q] = make_uint2(0u, 0u);
+        for (int q = threadIdx.x; q < ENUM_CHUNK / 2; q += 256) ((uint4 *)place)[q] = make_uint4(0u, 0u, 0u, 0u);
+        __syncthreads();
+        walk_candidates(ct, fcache, fc, wi, J, tabs, gs, kc, ke,
+                        [&](int k, int t, const TermTab &tb, int dx, int dy, int dz, int f, const double *fn,
+                            const double *nx, const double *ny, const double *nz) {
+                            unsigned surv[8];
+                            double maxb[8];
+                            screen_candidate<false>(fabs(tb.w), nx, ny, nz, fn, combo_mask(tb, dx, dy, dz), J.thr, surv,
+                                                    maxb);
+                            smask[k - kc] = make_uint2(surv[0] | surv[1] << 8 | surv[2] << 16 | surv[3] << 24,
+                                                       surv[4] | surv[5] << 8 | surv[6] << 16 | surv[7] << 24);
+                        });
+        // a candidate's places: f(ft_z, ft_y) -> index of its counter in the order of the list
+        auto visit = [&](auto &&fn) {
+            for (int k = kc + threadIdx.x; k < ke; k += 256) {
+                const uint2 m = smask[k - kc];
+                if (!(m.x | m.y)) continue;
+                int lo = 0, hi = J.ntab - 1;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (ct.start[mid] <= k) lo = mid;
+                    else hi = mid - 1;
+                }
+                const TermTab &tb = tabs[J.tab0 + lo];
+                const int nx = 2 * tb.ub[0] + 1, ny = 2 * tb.ub[1] + 1;
+                const int c = k - ct.start[lo], iz = c / (nx * ny), e = c - iz * nx * ny, iy = e / nx;
+                const int ps = ct.start[lo] + iz * nx * ny;  // the plane's and the row's first candidates
+                const int a = max(ps, kc), b = min(ps + nx * ny, ke);
+                const int ra = max(ps + iy * nx, a), rb = min(ps + (iy + 1) * nx, b);
+                const int p0 = 4 * (a - kc) + 2 * (ra - a) + (k - ra);
+                fn(k, m, tb, e - iy * nx - tb.ub[0], iy - tb.ub[1], iz - tb.ub[2], p0, 2 * (b - a), rb - ra);
+            }
+        };
+        __syncthreads();
+        visit([&](int k, const uint2 m, const TermTab &tb, int dx, int dy, int dz, int p0, int sz, int sy) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {  // c = ft_y + 2 ft_z: the bytes ft = 2 c, 2 c + 1
+                const unsigned w = (c < 2 ? m.x : m.y) >> (16 * (c & 1));
+                place[p0 + (c >> 1) * sz + (c & 1) * sy] = (unsigned short)(((w & 0xffu) ? 1 : 0) + ((w & 0xff00u) ? 1 : 0));
+            }
+        });
+        __syncthreads();
+        // exclusive prefix of the counters: 16 of them per thread
+        constexpr int PER = 4 * ENUM_CHUNK / 256;
+        unsigned short v[PER];
+#pragma unroll
+        for (int q = 0; q < PER; q++) v[q] = place[threadIdx.x * PER + q];
+        int tsum = 0;
+#pragma unroll
+        for (int q = 0; q < PER; q++) tsum += v[q];
+        const int incl = wave_incl_scan(tsum);
+        if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = incl;
+        __syncthreads();
+        int run = incl - tsum, total = 0;
+        for (int w = 0; w < 4; w++) {
+            if (w < (int)(threadIdx.x >> 6)) run += wsum[w];
+            total += wsum[w];
+        }
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            place[threadIdx.x * PER + q] = (unsigned short)run;
+            run += v[q];
+        }
+        __syncthreads();
+        visit([&](int k, const uint2 m, const TermTab &tb, int dx, int dy, int dz, int p0, int sz, int sy) {
+            const int f = lookup_f(fcache, fc, wi, J, gs, dx, dy, dz);
+            const unsigned long long wb = (unsigned long long)__double_as_longlong(tb.w);
+            const int blk = (int)(tb.blk / K2);
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const unsigned w2 = (c < 2 ? m.x : m.y) >> (16 * (c & 1));
+                if (!(w2 & 0xffffu)) continue;
+                Slice *dst = out + base + place[p0 + (c >> 1) * sz + (c & 1) * sy];
+#pragma unroll
+                for (int fx = 0; fx < 2; fx++) {
+                    const unsigned surv = (w2 >> (8 * fx)) & 0xffu;
+                    if (!surv) continue;
+                    const int ft = 2 * c + fx;
+                    const int xo = blk + (dx + tb.band) * 4 + (ft & 1), yo = blk + (dy + tb.band) * 4 + ((ft >> 1) & 1);
+                    const int zo = blk + (dz + tb.band) * 4 + (ft >> 2);
+                    ((uint4 *)dst)[0] = make_uint4((unsigned)wb, (unsigned)(wb >> 32), (unsigned)f, (unsigned)xo);
+                    ((uint4 *)dst)[1] = make_uint4((unsigned)yo, (unsigned)zo, (unsigned)ft | (surv << 8), 0u);
+                    dst++;
+                }
+            }
+        });
+        base += total;
+        __syncthreads();
     }
 }
 
 // one workgroup per (work node, part) (grid-stride; nwp: the node count on the device, the
 // parts then follow from it as on the host)
 template <int MODE>
-__global__ void __launch_bounds__(256) k_enum(int nw, const int *nwp, int *queue, int nparts, const WorkItem *work,
-                                              const JobTab *jobs, const TermTab *tabs, GenState gs, int *thread_off,
-                                              int *seg_total, const long long *seg_ofs, Tuple *out,
-                                              const TaskSummary *sum, const SegRec *segs) {
+__global__ void __launch_bounds__(256) k_enum(int nw, const int *nwp, int *queue, int nparts, int K2,
+                                              const WorkItem *work, const JobTab *jobs, const TermTab *tabs,
+                                              GenState gs, int *seg_total, const long long *seg_ofs, Slice *out,
+                                              const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks) {
     if (MODE == 1 && sum->overflow) return;
     const int n = nwp ? *nwp : nw, np = nwp ? enum_parts(n) : nparts;
     for_items(n * np, queue, [&](int b) {
-        enum_node<MODE>(b / np, b % np, np, work, jobs, tabs, gs, thread_off, seg_total, seg_ofs, out, segs);
+        enum_node<MODE>(b / np, b % np, np, K2, work, jobs, tabs, gs, seg_total, seg_ofs, out, sum, nodes, tasks);
     });
 }
 
@@ -1369,390 +1455,129 @@ __device__ inline void block_excl_scan_1024_n(long long (&v)[NV], long long (*ws
 }
 
 
-// One workgroup.  Phase 0 (several parts per node): segment counts and the parts'
-// offsets inside their segment.  Phase 1: per thread (a range of output nodes) the
-// totals of tuples, slices, FP64 tasks, slots, slice tasks and reduce items; one block
-// scan of the six gives each thread's offsets.  Phase 2: per segment (node, component)
-// its record (start, count, first task, first slot), reduce items, and the tasks of
-// segments with few tasks; segments (and nodes' slice runs) with many tasks go to a list
-// in LDS.  Phase 3: one wave per listed segment writes its tasks.  Every task has a fixed
-// position, so the schedule does not depend on the order of the list.
-constexpr int BT_FEW = 32, BT_LIST = 2048, BT_TABS = 256;
-constexpr long long FP64_TASKS = 4096;  // FP64 tasks an iteration aims at (task size permitting)
+// One workgroup.  Per node the slices of its (one or two) segments over all parts, and the parts'
+// offsets inside them; from the totals the task sizes; one block scan of slices and tasks gives
+// every node its first slices and tasks.  The fill kernels write the tasks themselves.
+constexpr long long FP64_TASKS = 2048;  // FP64 tasks an iteration aims at (task size permitting)
+constexpr int FP64_TASK_MIN = 8;        // ... of at least this many slices
 
-// (one workgroup: the pointers never alias, so that loads of later iterations can be
-// issued ahead of the stores of earlier ones)
 __global__ void __launch_bounds__(1024)
     k_build_tasks(int nw, const int *nwp, int nseg, int nparts, int chunk, int wchunk, const int *__restrict__ tot,
-                  TaskCaps caps,
-                  const int *__restrict__ gen_count, int gen_pcap, long long *__restrict__ ofs,
-                  ContractTask *__restrict__ tasks, SliceTask *__restrict__ stasks, ReduceItem *__restrict__ reds,
-                  TaskSummary *__restrict__ sum, SegRec *__restrict__ segs, int *__restrict__ segcnt,
-                  long long *__restrict__ gslice, const int *__restrict__ gen_overflow,
-                  const WorkItem *__restrict__ work, long long *__restrict__ tabcnt, int ntab) {
-    __shared__ long long wsum6[17][6];
-    __shared__ int big[BT_LIST];     // segment ids (>= 0) or -(node + 1) for slice runs
-    __shared__ int nbig;
+                  TaskCaps caps, const int *__restrict__ gen_count, int gen_pcap, long long *__restrict__ ofs,
+                  NodeSched *__restrict__ nodes, TaskSummary *__restrict__ sum,
+                  const int *__restrict__ gen_overflow) {
+    __shared__ long long wsum4[17][4];
     if (nwp) {  // the work list's size on the device (its parts as the enumeration derived them)
         nw = *nwp;
         nparts = enum_parts(nw);
     }
-    const bool mixed = nseg == 9;
-    // FP64 tasks of a tuple segment with c tuples (plain: always one, even empty, so that
-    // every output component is written; mixed: the reduce item writes the component)
-    auto ntasks_of = [&](int c) { return mixed ? (c + chunk - 1) / chunk : (c <= chunk ? 1 : (c + chunk - 1) / chunk); };
-    auto nslots_of = [&](int c) { return mixed ? (c + chunk - 1) / chunk : (c <= chunk ? 0 : (c + chunk - 1) / chunk); };
-    if (threadIdx.x == 0) nbig = 0;
-    // per job table: tuples and slices of its output nodes (statistics for the host),
-    // summed in LDS for the first BT_TABS tables, in global memory beyond
-    __shared__ unsigned long long lcnt[2 * BT_TABS];
-    // (entries 4 t + 3 hold the generated-node counts of the iteration: kept)
-    for (int q = threadIdx.x; q < 3 * ntab; q += blockDim.x) tabcnt[4 * (q / 3) + q % 3] = 0;
-    for (int q = threadIdx.x; q < 2 * BT_TABS; q += blockDim.x) lcnt[q] = 0;
-    // phase 0: segment counts (sum over the parts) and per-part offsets inside the segment
-    // (relative to the segment's start)
-    // (one part per node: the counts are the totals and every part offset is 0, which
-    // the fill kernels know)
-    const int nsg = nw * nseg;  // (work lists stay far below 2^31 / 9 nodes)
-    if (nparts > 1) {
-#pragma unroll 4
-        for (int sg = threadIdx.x; sg < nsg; sg += blockDim.x) {
-            int c = 0;
-            for (int p = 0; p < nparts; p++) {
-                ofs[sg * nparts + p] = c;
-                c += tot[sg * nparts + p];
-            }
-            segcnt[sg] = c;
-        }
-    }
-    const int *sc = nparts > 1 ? segcnt : tot;
-    __syncthreads();
-    // phase 1: this thread's totals (a contiguous range of output nodes)
+    const bool mixed = nseg == 2;
     const int g0 = (int)((long long)nw * threadIdx.x / 1024), g1 = (int)((long long)nw * (threadIdx.x + 1) / 1024);
-    {
-        // task sizes from the iteration's totals.  FP64 tasks: at most chunk tuples, fewer
-        // (down to 16) when the iteration has fewer than FP64_TASKS x chunk tuples, so that a
-        // coarse iteration still spreads over the GPU.  Slices per MFMA task when automatic
-        // (wchunk <= 0): about -wchunk tasks, at least 16 and at most 128 slices each (larger
-        // tasks leave too few to balance the k = 9 slices over the CUs)
-        long long tu1 = 0, sl1 = 0;
-        for (int g = g0; g < g1; g++) {
-            for (int q = 0; q < 8; q++) tu1 += sc[(size_t)g * nseg + q];
-            if (mixed) sl1 += sc[(size_t)g * 9 + 8];
+    long long v2[2] = {0, 0}, t2[2];
+    for (int g = g0; g < g1; g++) {
+        int c[2] = {0, 0};
+        for (int q = 0; q < nseg; q++) {
+            const size_t sg = ((size_t)g * nseg + q) * nparts;
+            if (nparts == 1) {  // (the fill kernels know that the only part's offset is 0)
+                c[q] = tot[sg];
+                continue;
+            }
+            for (int p = 0; p < nparts; p++) {
+                ofs[sg + p] = c[q];
+                c[q] += tot[sg + p];
+            }
         }
-        long long v2[2] = {tu1, sl1}, t2[2];
-        block_excl_scan_1024_n<2>(v2, (long long(*)[2])wsum6, t2);
-        chunk = (int)min((long long)chunk, max(16LL, (t2[0] + FP64_TASKS - 1) / FP64_TASKS));
+        nodes[g].count64 = c[0];
+        nodes[g].count16 = c[1];
+        v2[0] += c[0];
+        v2[1] += c[1];
+    }
+    // task sizes from the iteration's totals.  FP64 tasks: at most chunk slices, fewer (down
+    // to FP64_TASK_MIN) when the iteration has fewer than FP64_TASKS x chunk of them, so that a
+    // coarse iteration still spreads over the GPU.  Slices per MFMA task when automatic
+    // (wchunk <= 0): about -wchunk tasks, at least 16 and at most 128 slices each (larger
+    // tasks leave too few to balance the k = 9 slices over the CUs)
+    {
+        long long w2[2] = {v2[0], v2[1]};
+        block_excl_scan_1024_n<2>(w2, (long long(*)[2])wsum4, t2);
+        chunk = (int)min((long long)chunk, max((long long)FP64_TASK_MIN, (t2[0] + FP64_TASKS - 1) / FP64_TASKS));
         if (mixed && wchunk <= 0) {
             const long long want = (t2[1] + (-wchunk) - 1) / (-wchunk);
             wchunk = (int)min(128LL, max(16LL, want));
         }
         __syncthreads();
     }
-    long long tup = 0, sl = 0, nt = 0, nst = 0, slots = 0, nred = 0;
+    long long nt64 = 0, nt16 = 0;
     for (int g = g0; g < g1; g++) {
-        if (mixed) {
-            const int cs = sc[(size_t)g * 9 + 8];
-            sl += cs;
-            nst += (cs + wchunk - 1) / wchunk;
-        }
-        for (int q = 0; q < 8; q++) {
-            const int c = sc[(size_t)g * nseg + q];
-            tup += c;
-            nt += ntasks_of(c);
-            slots += nslots_of(c);
-            if (!mixed && c > chunk) nred++;
-        }
+        nt64 += (nodes[g].count64 + chunk - 1) / chunk;
+        if (mixed) nt16 += (nodes[g].count16 + wchunk - 1) / wchunk;
     }
-    long long pv[6] = {tup, sl, nt, nst, slots, nred}, pt[6];
-    block_excl_scan_1024_n<6>(pv, wsum6, pt);
-    long long btup = pv[0], bsl = pv[1], bnt = pv[2], bnst = pv[3], bslots = pv[4], bnred = pv[5];
-    long long Ttup = pt[0], Tsl = pt[1], Tnt = pt[2], Tnst = pt[3], Tslots = pt[4], Tnred = pt[5];
-    if (mixed) Tnred = 8LL * nw;
+    long long pv[4] = {v2[0], v2[1], nt64, nt16}, pt[4];
+    block_excl_scan_1024_n<4>(pv, wsum4, pt);
     int overflow = 0;
-    if (Ttup > caps.tuples || Tsl > caps.slices || Tnt > caps.tasks || Tnst > caps.stasks || Tnred > caps.reds ||
-        Tslots > caps.slots || Tnst > caps.nnslots)
-        overflow |= 1;
+    if (pt[0] > caps.slices64 || pt[1] > caps.slices || pt[2] > caps.tasks || pt[3] > caps.stasks) overflow |= 1;
     if (*(volatile const int *)gen_count > gen_pcap) overflow |= 2;
     if (threadIdx.x == 0) {
-        sum->ntuples = Ttup;
-        sum->nslices = Tsl;
-        sum->ntasks = (int)Tnt;
-        sum->nstasks = (int)Tnst;
-        sum->nreds = (int)Tnred;
-        sum->nslots = (int)Tslots;
-        sum->nnslots = (int)Tnst;
+        sum->nslices64 = pt[0];
+        sum->nslices = pt[1];
+        sum->ntasks = (int)pt[2];
+        sum->nstasks = (int)pt[3];
         sum->overflow = overflow;
         sum->gen_count = *(volatile const int *)gen_count;
         sum->gen_overflow = *(volatile const int *)gen_overflow;
-        sum->schunk = mixed ? wchunk : 0;
+        sum->chunk = chunk;
+        sum->schunk = mixed ? wchunk : 1;
     }
     if (overflow) return;
-    auto emit_task = [&](const SegRec &r, int sgi, int h) {
-        const int cnt = r.slot0 < 0 ? r.count : min(chunk, r.count - h * chunk);
-        tasks[r.task0 + h] = ContractTask{r.start + (long long)h * chunk, cnt, sgi >> 3, sgi & 7,
-                                          r.slot0 < 0 ? -1 : r.slot0 + h};
-    };
-    auto emit_stask = [&](int g, int h) {
-        const int cs = sc[(size_t)g * 9 + 8], nn0 = segs[(size_t)g * 8].pad_stask0;
-        stasks[nn0 + h] = SliceTask{gslice[g] + (long long)h * wchunk, min(wchunk, cs - h * wchunk), g, nn0 + h};
-    };
-    // phase 2: segment records, reduce items, tasks of small segments
-    int run_jt = -1;  // table statistics: one add per run of nodes of the same table
-    unsigned long long run_t = 0, run_s = 0;
-    auto flush_run = [&]() {
-        if (run_jt < 0) return;
-        if (run_jt < BT_TABS) {
-            atomicAdd(&lcnt[2 * run_jt], run_t);
-            atomicAdd(&lcnt[2 * run_jt + 1], run_s);
-        } else {
-            atomicAdd((unsigned long long *)&tabcnt[4 * run_jt], run_t);
-            atomicAdd((unsigned long long *)&tabcnt[4 * run_jt + 1], run_s);
-        }
-    };
     for (int g = g0; g < g1; g++) {
-        {
-            const int jt = work[g].job;
-            if (jt != run_jt) {
-                flush_run();
-                run_jt = jt;
-                run_t = run_s = 0;
-            }
-            for (int q = 0; q < 8; q++) run_t += (unsigned long long)sc[(size_t)g * nseg + q];
-            if (mixed) run_s += (unsigned long long)sc[(size_t)g * 9 + 8];
-        }
-        int nn0 = (int)bnst, nns = 0;
-        if (mixed) {
-            const int cs = sc[(size_t)g * 9 + 8];
-            nns = (cs + wchunk - 1) / wchunk;
-            gslice[g] = bsl;
-            segs[(size_t)g * 8].pad_stask0 = nn0;  // first slice task of node g
-            int slot_ = -1;
-            if (nns > BT_FEW) {
-                slot_ = atomicAdd(&nbig, 1);
-                if (slot_ < BT_LIST) big[slot_] = -(g + 1);
-            }
-            if (slot_ < 0 || slot_ >= BT_LIST)
-                for (int h = 0; h < nns; h++)
-                    stasks[nn0 + h] = SliceTask{bsl + (long long)h * wchunk, min(wchunk, cs - h * wchunk), g, nn0 + h};
-            bnst += nns;
-            bsl += cs;
-        }
-        for (int q = 0; q < 8; q++) {
-            const int c = sc[(size_t)g * nseg + q];
-            const int k = ntasks_of(c), ns = nslots_of(c);
-            const int sgi = g * 8 + q;
-            const SegRec r{btup, c, (int)bnt, ns ? (int)bslots : -1, 0};
-            segs[sgi].start = r.start;
-            segs[sgi].count = r.count;
-            segs[sgi].task0 = r.task0;
-            segs[sgi].slot0 = r.slot0;
-            if (mixed) reds[(size_t)g * 8 + q] = ReduceItem{g, q, (int)bslots, ns, nn0, nns};
-            else if (ns) reds[bnred++] = ReduceItem{g, q, (int)bslots, ns, 0, 0};
-            int slot_ = -1;
-            if (k > BT_FEW) {
-                slot_ = atomicAdd(&nbig, 1);
-                if (slot_ < BT_LIST) big[slot_] = sgi;
-            }
-            if (slot_ < 0 || slot_ >= BT_LIST)
-                for (int h = 0; h < k; h++) emit_task(r, sgi, h);
-            bnt += k;
-            bslots += ns;
-            btup += c;
-        }
-    }
-    flush_run();
-    __syncthreads();
-    for (int q = threadIdx.x; q < 2 * min(ntab, BT_TABS); q += blockDim.x)
-        tabcnt[4 * (q >> 1) + (q & 1)] = (long long)lcnt[q];
-    // phase 3: the listed segments, one wave per segment with the lanes over its tasks
-    // (the fill kernels add the segment starts to the per-part offsets themselves)
-    const int nb = min(nbig, BT_LIST);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int b = wave; b < nb; b += 16) {
-        const int id = big[b];
-        if (id >= 0) {
-            const SegRec r = segs[id];
-            const int k = ntasks_of(r.count);
-            for (int h = lane; h < k; h += 64) emit_task(r, id, h);
-        } else {
-            const int g = -id - 1;
-            const int nns = (sc[(size_t)g * 9 + 8] + wchunk - 1) / wchunk;
-            for (int h = lane; h < nns; h += 64) emit_stask(g, h);
-        }
+        const int c64 = nodes[g].count64, c16 = nodes[g].count16;
+        NodeSched nd;
+        nd.start64 = pv[0];
+        nd.start16 = pv[1];
+        nd.count64 = c64;
+        nd.count16 = c16;
+        nd.task64 = (int)pv[2];
+        nd.task16 = (int)pv[3];
+        nodes[g] = nd;
+        pv[0] += c64;
+        pv[1] += c16;
+        pv[2] += (c64 + chunk - 1) / chunk;
+        if (mixed) pv[3] += (c16 + wchunk - 1) / wchunk;
     }
 }
 
-// ----------------------------------------------------------------- apply: FP64 contraction
-
-// One wavefront per task = a chunk of the tuples of one segment (g, gt):
-//   out_gt[c][b][a] += w * sum X[a][i] Y[b][j] Z[c][l] f_ft[l][j][i]
-// Pass 1 keeps a row of f per lane (X by scalar loads), passes 2 and 3 exchange
-// through the wave's LDS slice.  The result goes to the output node when the
-// segment has one chunk, else to a partial slot summed by k_reduce_partials.
-template <int K>
-__device__ inline void contract_fp64_task(const ContractTask task, const WorkItem *work, const JobTab *jobs,
-                                          const TermTab *tabs, const Tuple *tuples, const double *genPool,
-                                          double *partials, double *B, int lane) {
-    constexpr int K2 = K * K, K3 = K2 * K;
-    constexpr int NP = (K2 + 63) / 64;
-    const WorkItem wi = work[task.g];
-    const JobTab &J = jobs[wi.job];
-    const int gt = task.gt;
-    const gdouble *blocks = (const gdouble *)J.operBlocks;
-    const gdouble *inCoef = (const gdouble *)J.inCoef;
-    const gdouble *gen = (const gdouble *)genPool;
-    double acc[NP][K];
-#pragma unroll
-    for (int p = 0; p < NP; p++)
-#pragma unroll
-        for (int c = 0; c < K; c++) acc[p][c] = 0.0;
-    for (int it = 0; it < task.count; it++) {
-        const Tuple tp = tuples[task.start + it];
-        const int ft = tp.combo & 7;
-        const TermTab &tb = tabs[J.tab0 + tp.term];
-        const int tx = 2 * (gt & 1) + (ft & 1);
-        const int ty = 2 * ((gt >> 1) & 1) + ((ft >> 1) & 1);
-        const int tz = 2 * ((gt >> 2) & 1) + ((ft >> 2) & 1);
-        const long long band = tb.band, blk = tb.blk;
-        const gdouble *X = blocks + blk + ((tp.dx + band) * 4 + tx) * K2;
-        const gdouble *Y = blocks + blk + ((tp.dy + band) * 4 + ty) * K2;
-        const gdouble *Z = blocks + blk + ((tp.dz + band) * 4 + tz) * K2;
-        const gdouble *f = tp.f >= 0 ? inCoef + (size_t)tp.f * 8 * K3 + ft * K3 : gen + (size_t)(-tp.f - 1) * K3;
-        const double w = tb.w;
-        // The operator rows come through scalar loads.  Up to K = 8 a whole K x K block fits
-        // the scalar registers and the loops unroll fully; beyond, two rows (pass 3: two
-        // columns) are live at a time — the same sums in the same order.
-        constexpr bool ROWWISE = K > 8;
-        constexpr int RU = ROWWISE ? 2 : K;
-        for (int r = lane; r < K2; r += 64) {
-            double fr[K];
-#pragma unroll
-            for (int i = 0; i < K; i++) fr[i] = f[r * K + i];
-#pragma unroll RU
-            for (int a = 0; a < K; a++) {
-                double s = 0.0;
-#pragma unroll
-                for (int i = 0; i < K; i++) s += X[a * K + i] * fr[i];
-                B[r * K + a] = s;
-            }
-        }
-        wave_sync();
-        for (int col = lane; col < K2; col += 64) {
-            const int l = col / K, a = col % K;
-            double tc[K];
-#pragma unroll
-            for (int j = 0; j < K; j++) tc[j] = B[(l * K + j) * K + a];
-#pragma unroll RU
-            for (int b = 0; b < K; b++) {
-                double s = 0.0;
-#pragma unroll
-                for (int j = 0; j < K; j++) s += Y[b * K + j] * tc[j];
-                B[(l * K + b) * K + a] = s;
-            }
-        }
-        wave_sync();
-#pragma unroll
-        for (int p = 0; p < NP; p++) {
-            const int ba = lane + 64 * p;
-            if (ba < K2) {
-                if constexpr (ROWWISE) {
-                    double s[K];
-#pragma unroll
-                    for (int c = 0; c < K; c++) s[c] = 0.0;
-#pragma unroll 2
-                    for (int l = 0; l < K; l++) {
-                        const double t = B[l * K2 + ba];
-#pragma unroll
-                        for (int c = 0; c < K; c++) s[c] += Z[c * K + l] * t;
-                    }
-#pragma unroll
-                    for (int c = 0; c < K; c++) acc[p][c] += w * s[c];
-                } else {
-                    double tc[K];
-#pragma unroll
-                    for (int l = 0; l < K; l++) tc[l] = B[l * K2 + ba];
-#pragma unroll
-                    for (int c = 0; c < K; c++) {
-                        double s = 0.0;
-#pragma unroll
-                        for (int l = 0; l < K; l++) s += Z[c * K + l] * tc[l];
-                        acc[p][c] += w * s;
-                    }
-                }
-            }
-        }
-        wave_sync();
-    }
-    double *dst = task.slot >= 0 ? partials + (size_t)task.slot * K3
-                                 : J.outCoef + (size_t)wi.node * 8 * K3 + gt * K3;
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-        const int ba = lane + 64 * p;
-        if (ba < K2) {
-#pragma unroll
-            for (int c = 0; c < K; c++) dst[c * K2 + ba] = acc[p][c];
-        }
-    }
-}
-
-// The task count comes from the device-built schedule (sum) when given; the grid
-// covers the schedule's capacity and waves past the count exit.
-template <int K>
-__global__ void __launch_bounds__(256) k_contract_fp64(int ntask_arg, const TaskSummary *sum,
-                                                       const ContractTask *tasks, const WorkItem *work,
-                                                       const JobTab *jobs, const TermTab *tabs,
-                                                       const Tuple *tuples, const double *genPool,
-                                                       double *partials, unsigned long long *ts) {
-    // (no stores or clock reads on the way to the task loop: the operator rows are read
-    // through scalar loads, which the compiler only uses for memory nothing before them may
-    // have changed.  With ts, block 0, dispatched first, only stamps the contraction's start
-    // and the tasks start at block 1.)
-    constexpr int K3 = K * K * K;
-    __shared__ double buf[4][K3];
-    if (ts && blockIdx.x == 0) {
-        if (threadIdx.x == 0) *ts = (unsigned long long)wall_clock64();
-        return;
-    }
-    const int wave = wave_id(), lane = threadIdx.x & 63;
-    const int ntask = sum ? (sum->overflow ? 0 : sum->ntasks) : ntask_arg;
-    const int ti = ((int)blockIdx.x - (ts ? 1 : 0)) * 4 + wave;
-    if (ti >= ntask) return;
-    contract_fp64_task<K>(tasks[ti], work, jobs, tabs, tuples, genPool, partials, buf[wave], lane);
-}
-
-
-// sums, per segment (g, gt), the FP64 tuple slots and the gt part of the mixed
-// node slots in slot order (deterministic)
-// Sums the partial results of an output component in a fixed order.  With wnorm
-// (mixed path: every component of every work node has an item) the component's norm
-// goes to the tree and to the compact per-work-node array as well.
-__global__ void __launch_bounds__(256) k_reduce_partials(int n_arg, const TaskSummary *sum, const ReduceItem *items,
-                                                         const WorkItem *work, const JobTab *jobs,
-                                                         const double *partials, const double *nodeslots, int K3,
-                                                         double *wnorm) {
+// Sums the task slots of an output component in a fixed order (FP64 tasks, then MFMA tasks)
+// into the node, and its norm into the tree and the compact per-work-node array.  One
+// workgroup per (work node, component).
+__global__ void __launch_bounds__(256) k_reduce_slots(int nw, const int *nwp, const TaskSummary *sum,
+                                                      const NodeSched *nodes, const WorkItem *work, const JobTab *jobs,
+                                                      const double *slots64, const double *slots16, int K3,
+                                                      double *wnorm) {
     __shared__ double wsum[4];
-    const int n = sum ? (sum->overflow ? 0 : sum->nreds) : n_arg;
+    if (sum->overflow) return;
+    const int n = 8 * (nwp ? *nwp : nw), chunk = sum->chunk, wchunk = sum->schunk;
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const ReduceItem it = items[i];
-        const WorkItem wi = work[it.g];
+        const int g = i >> 3, gt = i & 7;
+        const NodeSched nd = nodes[g];
+        const WorkItem wi = work[g];
         const JobTab &J = jobs[wi.job];
-        double *dst = J.outCoef + (size_t)wi.node * 8 * K3 + it.gt * K3;
+        const int n64 = (nd.count64 + chunk - 1) / chunk, n16 = (nd.count16 + wchunk - 1) / wchunk;
+        double *dst = J.outCoef + (size_t)wi.node * 8 * K3 + gt * K3;
+        const double *p64 = slots64 + ((size_t)nd.task64 * 8 + gt) * K3;
+        const double *p16 = slots16 + ((size_t)nd.task16 * 8 + gt) * K3;
         double ss = 0.0;
         for (int e = threadIdx.x; e < K3; e += blockDim.x) {
             double s = 0.0;
-            for (int q = 0; q < it.nslots; q++) s += partials[(size_t)(it.slot0 + q) * K3 + e];
-            for (int q = 0; q < it.nnslots; q++) s += nodeslots[((size_t)(it.nslot0 + q) * 8 + it.gt) * K3 + e];
+            for (int q = 0; q < n64; q++) s += p64[(size_t)q * 8 * K3 + e];
+            for (int q = 0; q < n16; q++) s += p16[(size_t)q * 8 * K3 + e];
             dst[e] = s;
             ss += s * s;
         }
-        if (wnorm) {
-            ss = block_sum_256(ss, wsum);
-            if (threadIdx.x == 0) {
-                const double v = sqrt(ss);
-                J.outNorm[(size_t)wi.node * 8 + it.gt] = v;
-                wnorm[(size_t)it.g * 8 + it.gt] = v;
-            }
+        ss = block_sum_256(ss, wsum);
+        if (threadIdx.x == 0) {
+            const double v = sqrt(ss);
+            J.outNorm[(size_t)wi.node * 8 + gt] = v;
+            wnorm[(size_t)g * 8 + gt] = v;
         }
     }
 }
@@ -1760,95 +1585,91 @@ __global__ void __launch_bounds__(256) k_reduce_partials(int n_arg, const TaskSu
 
 // ----------------------------------------------------------------- apply: mixed-precision work list
 
-// Same candidates and bounds as k_enum.  A candidate (term, delta, ft) whose
-// surviving combos all stay below ROUTE_FP64 * thr becomes one slice (all allowed
-// gt, split-FP16 MFMA); otherwise its surviving combos become FP64 tuples.  Counters per
-// thread: 8 tuple segments (per gt) + 1 slice segment; layout of thread_off and
-// seg_total: [g][9][...].
+// Same candidates and bounds as k_enum.  A slice (term, delta, ft) whose surviving combinations
+// all stay below the route bound is contracted on split-FP16 MFMA, the others in FP64.
+// Segments per node: 0 the FP64 slices, 1 the MFMA slices; layout of thread_off and
+// seg_total: [g][2][...].
 template <int MODE>
 __device__ __forceinline__ void enum_mixed_node(int g, int part, int nparts, int K2, const WorkItem *work,
                                                 const JobTab *jobs, const TermTab *tabs, const GenState &gs,
                                                 int *thread_off, int *seg_total, const long long *seg_ofs,
-                                                Tuple *out, Slice *sout, const SegRec *segs,
-                                                const long long *gslice) {
+                                                Slice *out64, Slice *out16, const TaskSummary *sum,
+                                                const NodeSched *nodes, SliceTask *tasks, SliceTask *stasks) {
     const WorkItem wi = work[g];
     const JobTab &J = jobs[wi.job];
-    __shared__ int scan[9][256];
+    __shared__ int scan[2][256];
     __shared__ int fcache[FCACHE];
     __shared__ CandTerms ct;
+    __shared__ int wsum[4];
     const FCache fc = fill_fcache(fcache, wi, J, tabs, gs);
     term_prefix(ct, J, tabs);
-    int cnt[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    long long base[9];
-    if (MODE == 1)
-        for (int q = 0; q < 9; q++) {
-            const size_t sp = ((size_t)g * 9 + q) * nparts + part;  // (segment, part)
-            base[q] = (q < 8 ? segs[(size_t)g * 8 + q].start : gslice[g]) + (nparts > 1 ? seg_ofs[sp] : 0) +
+    int cnt[2] = {0, 0}, nt64 = 0;
+    long long base[2] = {0, 0};
+    if (MODE == 1) {
+        const NodeSched nd = nodes[g];
+        if (part == 0) {
+            emit_tasks(g, nd.start64, nd.count64, sum->chunk, nd.task64, tasks);
+            emit_tasks(g, nd.start16, nd.count16, sum->schunk, nd.task16, stasks);
+        }
+        for (int q = 0; q < 2; q++) {
+            const size_t sp = ((size_t)g * 2 + q) * nparts + part;  // (segment, part)
+            base[q] = (q ? nd.start16 : nd.start64) + (nparts > 1 ? seg_ofs[sp] : 0) +
                       thread_off[sp * 256 + threadIdx.x];
         }
-    walk_candidates(ct, fcache, fc, wi, J, tabs, gs, part, nparts,
-                    [&](int t, const TermTab &tb, int dx, int dy, int dz, int f, const double *fn, int nft,
+    }
+    int k0, k1;
+    part_range(ct.start[J.ntab], part, nparts, k0, k1);
+    walk_candidates(ct, fcache, fc, wi, J, tabs, gs, k0, k1,
+                    [&](int k, int t, const TermTab &tb, int dx, int dy, int dz, int f, const double *fn,
                         const double *nx, const double *ny, const double *nz) {
                         const double aw = fabs(tb.w);
                         const unsigned long long cm = combo_mask(tb, dx, dy, dz);
                         unsigned survs[8];
                         double maxbs[8];
                         screen_candidate<true>(aw, nx, ny, nz, fn, cm, J.thr, survs, maxbs);
-                        (void)nft;  // (survs[ft] = 0 beyond the node's components)
 #pragma unroll
                         for (int ft = 0; ft < 8; ft++) {
-                            const int surv = (int)survs[ft];
-                            const double maxb = maxbs[ft];
+                            const unsigned surv = survs[ft];
                             if (!surv) continue;
-                            if (maxb > J.route) {
-#pragma unroll
-                                for (int gt = 0; gt < 8; gt++) {
-                                    if (!((surv >> gt) & 1)) continue;
-                                    if (MODE == 1) {
-                                        Tuple tp;
-                                        tp.g = g;
-                                        tp.f = f;
-                                        tp.term = (uint8_t)t;
-                                        tp.combo = (uint8_t)(gt * 8 + ft);
-                                        tp.dx = (int16_t)dx;
-                                        tp.dy = (int16_t)dy;
-                                        tp.dz = (int16_t)dz;
-                                        out[base[gt] + cnt[gt]] = tp;
-                                    }
-                                    cnt[gt]++;
-                                }
-                            } else {
-                                if (MODE == 1) {
-                                    // the record as two 16-byte stores (layout of Slice): weight,
-                                    // f, FP32 block offsets of the three dimensions, ft, and the
-                                    // surviving components only (the same tuples as the plain
-                                    // work list, FP32 in place of FP64)
-                                    const unsigned long long wb = (unsigned long long)__double_as_longlong(tb.w);
-                                    const int xo = (int)(tb.blk + ((dx + tb.band) * 4 + (ft & 1)) * K2);
-                                    const int yo = (int)(tb.blk + ((dy + tb.band) * 4 + ((ft >> 1) & 1)) * K2);
-                                    const int zo = (int)(tb.blk + ((dz + tb.band) * 4 + ((ft >> 2) & 1)) * K2);
-                                    uint4 *dst = (uint4 *)(sout + base[8] + cnt[8]);
-                                    dst[0] = make_uint4((unsigned)wb, (unsigned)(wb >> 32), (unsigned)f, (unsigned)xo);
-                                    dst[1] = make_uint4((unsigned)yo, (unsigned)zo, (unsigned)ft | ((unsigned)surv << 8), 0u);
-                                }
-                                cnt[8]++;
+                            const bool r64 = maxbs[ft] > J.route;
+                            if (MODE == 1) {
+                                // the record as two 16-byte stores (layout of Slice): weight, f,
+                                // block offsets of the three dimensions (MFMA: in values; FP64: in
+                                // blocks), ft and the surviving components
+                                const unsigned long long wb = (unsigned long long)__double_as_longlong(tb.w);
+                                const int unit = r64 ? 1 : K2, blk = (int)(r64 ? tb.blk / K2 : tb.blk);
+                                const int xo = blk + ((dx + tb.band) * 4 + (ft & 1)) * unit;
+                                const int yo = blk + ((dy + tb.band) * 4 + ((ft >> 1) & 1)) * unit;
+                                const int zo = blk + ((dz + tb.band) * 4 + ((ft >> 2) & 1)) * unit;
+                                uint4 *dst = (uint4 *)(r64 ? out64 + base[0] + cnt[0] : out16 + base[1] + cnt[1]);
+                                dst[0] = make_uint4((unsigned)wb, (unsigned)(wb >> 32), (unsigned)f, (unsigned)xo);
+                                dst[1] = make_uint4((unsigned)yo, (unsigned)zo, (unsigned)ft | (surv << 8), 0u);
+                            } else if (r64) {
+                                nt64 += __popc(surv);
                             }
+                            if (r64) cnt[0]++;
+                            else cnt[1]++;
                         }
                     });
     if (MODE == 0) {
-        for (int q = 0; q < 9; q++) scan[q][threadIdx.x] = cnt[q];
+        nt64 = block_sum_256i(nt64, wsum);
+        for (int q = 0; q < 2; q++) scan[q][threadIdx.x] = cnt[q];
         __syncthreads();
         for (int off = 1; off < 256; off <<= 1) {
-            int v[9];
-            for (int q = 0; q < 9; q++) v[q] = threadIdx.x >= off ? scan[q][threadIdx.x - off] : 0;
+            int v[2];
+            for (int q = 0; q < 2; q++) v[q] = threadIdx.x >= off ? scan[q][threadIdx.x - off] : 0;
             __syncthreads();
-            for (int q = 0; q < 9; q++) scan[q][threadIdx.x] += v[q];
+            for (int q = 0; q < 2; q++) scan[q][threadIdx.x] += v[q];
             __syncthreads();
         }
-        for (int q = 0; q < 9; q++)
-            thread_off[(((size_t)g * 9 + q) * nparts + part) * 256 + threadIdx.x] = scan[q][threadIdx.x] - cnt[q];
-        if (threadIdx.x == 255)
-            for (int q = 0; q < 9; q++) seg_total[((size_t)g * 9 + q) * nparts + part] = scan[q][255];
+        for (int q = 0; q < 2; q++)
+            thread_off[(((size_t)g * 2 + q) * nparts + part) * 256 + threadIdx.x] = scan[q][threadIdx.x] - cnt[q];
+        if (threadIdx.x == 255) {
+            for (int q = 0; q < 2; q++) seg_total[((size_t)g * 2 + q) * nparts + part] = scan[q][255];
+            if (nt64) atomicAdd((unsigned long long *)&gs.tabcnt[4 * wi.job], (unsigned long long)nt64);
+            if (scan[1][255])
+                atomicAdd((unsigned long long *)&gs.tabcnt[4 * wi.job + 1], (unsigned long long)scan[1][255]);
+        }
     }
 }
 
@@ -1856,42 +1677,15 @@ template <int MODE>
 __global__ void __launch_bounds__(256) k_enum_mixed(int nw, const int *nwp, int *queue, int nparts, int K2,
                                                     const WorkItem *work, const JobTab *jobs, const TermTab *tabs,
                                                     GenState gs, int *thread_off, int *seg_total,
-                                                    const long long *seg_ofs, Tuple *out, Slice *sout,
-                                                    const TaskSummary *sum, const SegRec *segs,
-                                                    const long long *gslice) {
+                                                    const long long *seg_ofs, Slice *out64, Slice *out16,
+                                                    const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks,
+                                                    SliceTask *stasks) {
     if (MODE == 1 && sum->overflow) return;
     const int n = nwp ? *nwp : nw, np = nwp ? enum_parts(n) : nparts;
     for_items(n * np, queue, [&](int b) {
-        enum_mixed_node<MODE>(b / np, b % np, np, K2, work, jobs, tabs, gs, thread_off, seg_total, seg_ofs, out,
-                              sout, segs, gslice);
+        enum_mixed_node<MODE>(b / np, b % np, np, K2, work, jobs, tabs, gs, thread_off, seg_total, seg_ofs, out64,
+                              out16, sum, nodes, tasks, stasks);
     });
-}
-
-
-// norms of the work nodes of all jobs, into their trees and into a compact array
-__device__ __forceinline__ void work_norms_node(int i, const WorkItem *work, const JobTab *jobs, int K3,
-                                                double *compact) {
-    const WorkItem wi = work[i];
-    const JobTab &J = jobs[wi.job];
-    const double *p = J.outCoef + (size_t)wi.node * 8 * K3;
-    for (int c = 0; c < 8; c++) {
-        double s = 0.0;
-        for (int e = threadIdx.x; e < K3; e += 64) s += p[c * K3 + e] * p[c * K3 + e];
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        if (threadIdx.x == 0) {
-            const double v = sqrt(s);
-            J.outNorm[(size_t)wi.node * 8 + c] = v;
-            compact[(size_t)i * 8 + c] = v;
-        }
-    }
-}
-
-__global__ void k_work_norms(int nw, const int *nwp, const WorkItem *work, const JobTab *jobs, int K3,
-                             double *compact, unsigned long long *ts_end) {
-    // (the contraction's end on the device clock: this kernel starts once the reduction is done)
-    if (ts_end && blockIdx.x == 0 && threadIdx.x == 0) *ts_end = (unsigned long long)wall_clock64();
-    const int n = nwp ? *nwp : nw;
-    for (int i = blockIdx.x; i < n; i += gridDim.x) work_norms_node(i, work, jobs, K3, compact);
 }
 
 // ----------------------------------------------------------------- apply: device-resident refinement
@@ -2287,18 +2081,6 @@ static hipError_t allow_smem(Kern *k, size_t sm) {
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
 }
 
-#define MWG_DISPATCH_K(K, CALL)                                       \
-    switch (K) {                                                      \
-        case 4: { constexpr int KK = 4; CALL; } break;                \
-        case 5: { constexpr int KK = 5; CALL; } break;                \
-        case 6: { constexpr int KK = 6; CALL; } break;                \
-        case 7: { constexpr int KK = 7; CALL; } break;                \
-        case 8: { constexpr int KK = 8; CALL; } break;                \
-        case 9: { constexpr int KK = 9; CALL; } break;                \
-        case 10: { constexpr int KK = 10; CALL; } break;              \
-        default: return hipErrorInvalidValue;                         \
-    }
-
 hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
                          double pre, const DevBasis &B, const double *gx, const double *gw, double *out) {
     if (n <= 0) return hipSuccess;
@@ -2410,26 +2192,17 @@ hipError_t launch_gen_compute(hipStream_t s, int first, int cap, const JobTab *j
     return hipGetLastError();
 }
 
-hipError_t launch_enum(hipStream_t s, int mode, int nw, int nparts, const WorkItem *work, const JobTab *jobs,
-                       const TermTab *tabs, const GenState &gs, int *thread_off, int *seg_total,
-                       const long long *seg_ofs, Tuple *out, const TaskSummary *sum, const SegRec *segs,
-                       const int *nwp, int *queue) {
+hipError_t launch_enum(hipStream_t s, int mode, int K, int nw, int nparts, const WorkItem *work, const JobTab *jobs,
+                       const TermTab *tabs, const GenState &gs, int *seg_total, const long long *seg_ofs, Slice *out,
+                       const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks, const int *nwp, int *queue) {
     if (nw <= 0) return hipSuccess;
     const unsigned nb = nwp ? (unsigned)DEVCOUNT_GRID : (unsigned)nw * (unsigned)nparts;
     if (mode == 0)
-        hipLaunchKernelGGL(k_enum<0>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, work, jobs, tabs, gs,
-                           thread_off, seg_total, seg_ofs, out, sum, segs);
+        hipLaunchKernelGGL(k_enum<0>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, K * K, work, jobs, tabs, gs,
+                           seg_total, seg_ofs, out, sum, nodes, tasks);
     else
-        hipLaunchKernelGGL(k_enum<1>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, work, jobs, tabs, gs,
-                           thread_off, seg_total, seg_ofs, out, sum, segs);
-    return hipGetLastError();
-}
-
-hipError_t launch_work_norms(hipStream_t s, int nw, const WorkItem *work, const JobTab *jobs, int K3,
-                             double *compact, const int *nwp, unsigned long long *ts_end) {
-    if (nw <= 0) return hipSuccess;
-    const int nb = nwp ? std::min(nw, DEVCOUNT_GRID) : nw;
-    hipLaunchKernelGGL(k_work_norms, dim3(nb), dim3(64), 0, s, nw, nwp, work, jobs, K3, compact, ts_end);
+        hipLaunchKernelGGL(k_enum<1>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, K * K, work, jobs, tabs, gs,
+                           seg_total, seg_ofs, out, sum, nodes, tasks);
     return hipGetLastError();
 }
 
@@ -2480,49 +2253,35 @@ hipError_t launch_transform(hipStream_t s, int mode, int n, const TransformItem 
 }
 
 hipError_t launch_build_tasks(hipStream_t s, int nw, int nseg, int nparts, int chunk, int wchunk, const int *tot,
-                              TaskCaps caps, const int *gen_count, int gen_pcap, long long *ofs, ContractTask *tasks,
-                              SliceTask *stasks, ReduceItem *reds, TaskSummary *sum, SegRec *segs, int *segcnt,
-                              long long *gslice, const int *gen_overflow, const WorkItem *work, long long *tabcnt,
-                              int ntab, const int *nwp) {
+                              TaskCaps caps, const int *gen_count, int gen_pcap, long long *ofs, NodeSched *nodes,
+                              TaskSummary *sum, const int *gen_overflow, const int *nwp) {
     hipLaunchKernelGGL(k_build_tasks, dim3(1), dim3(1024), 0, s, nw, nwp, nseg, nparts, chunk, wchunk, tot, caps,
-                       gen_count, gen_pcap, ofs, tasks, stasks, reds, sum, segs, segcnt, gslice, gen_overflow, work,
-                       tabcnt, ntab);
+                       gen_count, gen_pcap, ofs, nodes, sum, gen_overflow);
     return hipGetLastError();
 }
 
-hipError_t launch_contract_fp64(hipStream_t s, int K, int ntask, const TaskSummary *sum, int grid,
-                                const ContractTask *tasks, const WorkItem *work, const JobTab *jobs,
-                                const TermTab *tabs, const Tuple *tuples, const double *genPool, double *partials,
-                                unsigned long long *ts) {
-    const int nb = sum ? grid : (ntask + 3) / 4;
-    if (nb <= 0) return hipSuccess;
-    MWG_DISPATCH_K(K, hipLaunchKernelGGL(k_contract_fp64<KK>, dim3(nb + (ts ? 1 : 0)), dim3(256), 0, s, ntask, sum,
-                                         tasks, work, jobs, tabs, tuples, genPool, partials, ts));
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_partials(hipStream_t s, int n, const TaskSummary *sum, int grid, const ReduceItem *items,
-                                  const WorkItem *work, const JobTab *jobs, const double *partials,
-                                  const double *nodeslots, int K3, double *wnorm) {
-    const int nb = sum ? grid : n;
-    if (nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_partials, dim3(nb), dim3(256), 0, s, n, sum, items, work, jobs, partials, nodeslots,
+hipError_t launch_reduce_slots(hipStream_t s, int nw, const int *nwp, const TaskSummary *sum, const NodeSched *nodes,
+                               const WorkItem *work, const JobTab *jobs, const double *slots64, const double *slots16,
+                               int K3, double *wnorm) {
+    if (nw <= 0) return hipSuccess;
+    const int nb = (int)std::min<long long>(8LL * nw, 4096);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(nb), dim3(256), 0, s, nw, nwp, sum, nodes, work, jobs, slots64, slots16,
                        K3, wnorm);
     return hipGetLastError();
 }
 
 hipError_t launch_enum_mixed(hipStream_t s, int mode, int K, int nw, int nparts, const WorkItem *work, const JobTab *jobs,
                              const TermTab *tabs, const GenState &gs, int *thread_off, int *seg_total,
-                             const long long *seg_ofs, Tuple *out, Slice *sout, const TaskSummary *sum,
-                             const SegRec *segs, const long long *gslice, const int *nwp, int *queue) {
+                             const long long *seg_ofs, Slice *out64, Slice *out16, const TaskSummary *sum,
+                             const NodeSched *nodes, SliceTask *tasks, SliceTask *stasks, const int *nwp, int *queue) {
     if (nw <= 0) return hipSuccess;
     const unsigned nb = nwp ? (unsigned)DEVCOUNT_GRID : (unsigned)nw * (unsigned)nparts;
     if (mode == 0)
         hipLaunchKernelGGL(k_enum_mixed<0>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, K * K, work, jobs,
-                           tabs, gs, thread_off, seg_total, seg_ofs, out, sout, sum, segs, gslice);
+                           tabs, gs, thread_off, seg_total, seg_ofs, out64, out16, sum, nodes, tasks, stasks);
     else
         hipLaunchKernelGGL(k_enum_mixed<1>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, K * K, work, jobs,
-                           tabs, gs, thread_off, seg_total, seg_ofs, out, sout, sum, segs, gslice);
+                           tabs, gs, thread_off, seg_total, seg_ofs, out64, out16, sum, nodes, tasks, stasks);
     return hipGetLastError();
 }
 

@@ -44,7 +44,7 @@ class Context:
         check(lib().mwg_sync(self.h), self.h)
 
     def set_tuning(self, fp64_chunk: int, slice_chunk: int):
-        """Contraction task granularity: tuples per FP64 wave task, MFMA slices per wave task."""
+        """Contraction task granularity: slices per FP64 task, slices per MFMA task."""
         check(lib().mwg_ctx_set_tuning(self.h, int(fp64_chunk), int(slice_chunk)), self.h)
 
     def get_tuning(self) -> tuple[int, int]:
