@@ -284,8 +284,10 @@ struct Ctx {
     DBuf<unsigned long long> genHashKeys;
     DBuf<int> genHashVals;
     DBuf<TransformItem> titems;
-    DBuf<MulItem> mitems;  // batched products: items and work lists of all jobs
-    DBuf<int> mwork;
+    DBuf<MulItem> mitems;  // products, sums, projections: items of all jobs, and the jobs
+    DBuf<MulJobDev> mjobs;
+    DBuf<double> ppar;  // parameters of a projected function
+    DBuf<int> mwork;    // (quantum numbers)
     // FP64 slices, tasks and slots; the same for the MFMA slices
     DBuf<Slice> slices64, slices;
     DBuf<SliceTask> tasks, stasks;
@@ -351,10 +353,10 @@ struct MraH {
     int n0 = 0, corner[3] = {0, 0, 0}, boxes[3] = {1, 1, 1}, maxDepth = 16;
     double sfac = 1.0;
     Basis B;
-    DBuf<double> U, qx, qw, phiq, W, WT, ccoef;
+    DBuf<double> U, qx, qw, phiq, W, WT, E, C, ccoef;
     double lo(int d) const { return sfac * std::ldexp((double)corner[d], -n0); }
     double width(int d) const { return sfac * std::ldexp((double)boxes[d], -n0); }
-    DevBasis dev() const { return DevBasis{B.K, U.p, qx.p, qw.p, phiq.p, W.p}; }
+    DevBasis dev() const { return DevBasis{B.K, U.p, qx.p, qw.p, phiq.p, W.p, E.p, C.p}; }
     ProjGeom geom() const { return ProjGeom{{lo(0), lo(1), lo(2)}, sfac, n0}; }
 };
 
@@ -1151,30 +1153,79 @@ static void build_oper(OperH &O, MraH *mra, double mu, double prec) {
 
 // ------------------------------------------------------------------ projection
 
+// read-back of n doubles at the start of the context's device block, through pinned memory
+static const double *read_compact(Ctx &C, size_t n) {
+    C.rb.reserve(n * sizeof(double));
+    if (n) HC(hipMemcpyAsync(C.rb.h, C.rbd.p, n * sizeof(double), hipMemcpyDeviceToHost, C.stream));
+    stream_wait(C);
+    C.stage.off = 0;
+    return (const double *)C.rb.h;
+}
+
+// Bottom-up compression of finished trees (their leaves' norms already on the host): one launch
+// per depth for all of them, then the parents' new norms to the host in one transfer.
+static void compress_trees(Ctx &C, MraH &M, const std::vector<TreeH *> &trees) {
+    std::vector<std::vector<std::vector<int>>> L(trees.size());
+    int maxd = 0;
+    for (size_t j = 0; j < trees.size(); j++) {
+        L[j] = trees[j]->internal_by_depth();
+        maxd = std::max(maxd, (int)L[j].size());
+    }
+    std::vector<TransformItem> items;
+    std::vector<size_t> lofs(maxd + 1, 0);
+    for (int d = 0; d < maxd; d++) {
+        lofs[d] = items.size();
+        for (size_t j = 0; j < trees.size(); j++)
+            if (d < (int)L[j].size())
+                for (int p : L[j][d]) items.push_back({trees[j]->coef.p, trees[j]->norm.p, p, trees[j]->child[p]});
+    }
+    lofs[maxd] = items.size();
+    if (!items.empty()) {
+        upload_async(C, C.titems, items.data(), items.size());
+        C.rbd.alloc(8 * items.size() * sizeof(double));
+        double *cn = (double *)C.rbd.p;
+        for (int d = maxd - 1; d >= 0; d--)
+            HC(launch_transform(C.stream, 0, (int)(lofs[d + 1] - lofs[d]), C.titems.p + lofs[d], M.W.p, M.B.K,
+                                cn + 8 * lofs[d]));
+        const double *h = read_compact(C, 8 * items.size());
+        size_t q = 0;
+        for (int d = 0; d < maxd; d++)
+            for (size_t j = 0; j < trees.size(); j++)
+                if (d < (int)L[j].size())
+                    for (int p : L[j][d]) std::memcpy(&trees[j]->cnorm[8 * (size_t)p], h + 8 * q++, 8 * sizeof(double));
+    }
+    for (TreeH *T : trees) {
+        T->sqnorm_from_cnorm();
+        T->fit_dev();
+    }
+}
+
 template <class LaunchFn>
 static void project_adaptive(TreeH &T, double prec, LaunchFn launch, const std::vector<double> *gauss_alpha,
                              const std::vector<double> *gauss_center) {
     MraH &M = *T.mra;
     Ctx &C = *M.ctx;
-    hipStream_t s = C.stream;
     T.make_roots();
     std::vector<int> work = T.roots;
     double sNorm = 0.0, wNorm = 0.0;
     int iter = 0;
-    DBuf<int> dwork, ddepth, dlr;
+    std::vector<MulItem> items;
     while (!work.empty()) {
         T.ensure_dev(T.n());
-        dwork.upload(work.data(), work.size(), s);
-        ddepth.upload(T.depth.data(), T.depth.size(), s);
-        dlr.upload(T.lr.data(), T.lr.size(), s);
-        launch((int)work.size(), dwork.p, ddepth.p, dlr.p, T.coef.p);
-        HC(launch_norms(s, (int)work.size(), dwork.p, T.coef.p, T.norm.p, T.K3()));
-        std::vector<double> nrm(8 * (size_t)T.n());
-        T.norm.download(nrm.data(), nrm.size(), s);
-        for (int i : work) {
-            std::memcpy(&T.cnorm[8 * (size_t)i], &nrm[8 * (size_t)i], 8 * sizeof(double));
-            if (iter == 0) sNorm += nrm[8 * i] * nrm[8 * i];
-            for (int c = 1; c < 8; c++) wNorm += nrm[8 * i + c] * nrm[8 * i + c];
+        items.resize(work.size());
+        for (size_t w = 0; w < work.size(); w++) {
+            const int i = work[w];
+            items[w] = MulItem{i, T.depth[i], {T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2]}, 0, 0, 0, 0, 0};
+        }
+        upload_async(C, C.mitems, items.data(), items.size());
+        C.rbd.alloc(8 * work.size() * sizeof(double));
+        launch((int)work.size(), C.mitems.p, T.coef.p, T.norm.p, (double *)C.rbd.p);
+        const double *nrm = read_compact(C, 8 * work.size());
+        for (size_t w = 0; w < work.size(); w++) {
+            const double *p = nrm + 8 * w;
+            std::memcpy(&T.cnorm[8 * (size_t)work[w]], p, 8 * sizeof(double));
+            if (iter == 0) sNorm += p[0] * p[0];
+            for (int c = 1; c < 8; c++) wNorm += p[c] * p[c];
         }
         const double tnorm = std::sqrt(sNorm + wNorm);
         std::vector<int> next;
@@ -1209,17 +1260,7 @@ static void project_adaptive(TreeH &T, double prec, LaunchFn launch, const std::
         work.swap(next);
         iter++;
     }
-    // bottom-up compression of the internal nodes
-    auto L = T.internal_by_depth();
-    std::vector<TransformItem> items;
-    for (int d = (int)L.size() - 1; d >= 0; d--) {
-        items.clear();
-        for (int p : L[d]) items.push_back({T.coef.p, nullptr, p, T.child[p]});
-        C.titems.upload(items.data(), items.size(), s);
-        HC(launch_transform(s, 0, (int)items.size(), C.titems.p, M.W.p, M.B.K));
-    }
-    T.refresh_norms();
-    T.fit_dev();
+    compress_trees(C, M, {&T});
 }
 
 // ------------------------------------------------------------------ apply
@@ -2459,201 +2500,119 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
 
 // ------------------------------------------------------------------ multiplication
 
-// the node of T at (d, l) (steps 0) or its leaf ancestor and the levels between
-static void locate(const TreeH &T, int d, const int *l, int &src, int &steps) {
-    for (int dd = d; dd >= 0; dd--) {
-        const int sh = d - dd;
-        const int i = T.find(dd, l[0] >> sh, l[1] >> sh, l[2] >> sh);
-        if (i >= 0) {
-            src = i;
-            steps = sh;
-            return;
-        }
-    }
-    throw Error(MWG_ERR_STATE, "input tree does not cover the box");
-}
-
-static void multiply_trees(TreeH &out, double prec, double coef, TreeH &A, TreeH &B) {
-    MraH &M = *A.mra;
-    Ctx &C = *M.ctx;
-    hipStream_t s = C.stream;
-    if (A.n() == 0 || B.n() == 0) throw Error(MWG_ERR_STATE, "multiply: empty input tree");
-    out.make_roots();
-    // union grid
-    std::vector<int> order(out.roots.begin(), out.roots.end());
-    for (size_t w = 0; w < order.size(); w++) {
-        const int i = order[w];
-        const int d = out.depth[i], x = out.lr[3 * i], y = out.lr[3 * i + 1], z = out.lr[3 * i + 2];
-        const int ia = A.find(d, x, y, z), ib = B.find(d, x, y, z);
-        const bool sp = (ia >= 0 && A.child[ia] >= 0) || (ib >= 0 && B.child[ib] >= 0);
-        if (sp && d < M.maxDepth) {
-            out.split(i);
-            for (int a = 0; a < 8; a++) order.push_back(out.child[i] + a);
-        }
-    }
-    std::vector<int> work;
-    for (int i = 0; i < out.n(); i++) work.push_back(i);
-    double sNorm = 0.0, wNorm = 0.0;
-    bool first = true;
-    DBuf<MulItem> ditems;
-    DBuf<int> dwork;
-    while (!work.empty()) {
-        out.ensure_dev(out.n());
-        std::vector<MulItem> items(work.size());
-        for (size_t w = 0; w < work.size(); w++) {
-            const int i = work[w];
-            MulItem &it = items[w];
-            it.node = i;
-            it.depth = out.depth[i];
-            for (int q = 0; q < 3; q++) it.l[q] = out.lr[3 * i + q];
-            locate(A, it.depth, it.l, it.asrc, it.asteps);
-            locate(B, it.depth, it.l, it.bsrc, it.bsteps);
-        }
-        ditems.upload(items.data(), items.size(), s);
-        HC(launch_multiply(s, (int)items.size(), ditems.p, M.geom(), M.dev(), coef, A.coef.p, B.coef.p, out.coef.p));
-        dwork.upload(work.data(), work.size(), s);
-        HC(launch_norms(s, (int)work.size(), dwork.p, out.coef.p, out.norm.p, out.K3()));
-        std::vector<double> nrm(8 * (size_t)out.n());
-        out.norm.download(nrm.data(), nrm.size(), s);
-        for (int i : work) {
-            std::memcpy(&out.cnorm[8 * (size_t)i], &nrm[8 * (size_t)i], 8 * sizeof(double));
-            if (first && out.depth[i] == 0) sNorm += nrm[8 * i] * nrm[8 * i];
-            for (int c = 1; c < 8; c++) wNorm += nrm[8 * i + c] * nrm[8 * i + c];
-        }
-        first = false;
-        const double tnorm = std::sqrt(sNorm + wNorm);
-        std::vector<int> next;
-        for (int i : work) {
-            if (out.child[i] >= 0) continue;
-            const int d = out.depth[i];
-            if (d >= M.maxDepth) continue;
-            double wn = 0.0;
-            for (int c = 1; c < 8; c++) wn += out.cnorm[8 * i + c] * out.cnorm[8 * i + c];
-            if (split_check(M.n0 + d, std::sqrt(wn), prec, tnorm)) {
-                out.split(i);
-                for (int a = 0; a < 8; a++) next.push_back(out.child[i] + a);
-            }
-        }
-        work.swap(next);
-    }
-    auto L = out.internal_by_depth();
-    std::vector<TransformItem> titems;
-    for (int d = (int)L.size() - 1; d >= 0; d--) {
-        titems.clear();
-        for (int p : L[d]) titems.push_back({out.coef.p, nullptr, p, out.child[p]});
-        C.titems.upload(titems.data(), titems.size(), s);
-        HC(launch_transform(s, 0, (int)titems.size(), C.titems.p, M.W.p, M.B.K));
-    }
-    out.refresh_norms();
-    out.fit_dev();
-}
-
-// Many independent products as one: the same items, kernels and split tests as
-// multiply_trees for every job, with the launches of all jobs queued back to back and
-// one host round trip per refinement iteration (uploads through the staging ring, one
-// read-back of all jobs' norms).  Each output is identical to its single product.
+// Products and sums: out on the union grid of a and b (products are refined further).  For every
+// output node the input node that represents it (steps 0) or its leaf ancestor and the levels
+// between, known from the parent's as the nodes are made.
 struct MulJob {
     TreeH *out, *a, *b;
-    double prec, coef;
+    double prec, coef, coefb;
     std::vector<int> work;
     double sNorm = 0.0, wNorm = 0.0;
     bool first = true;
+    struct Src {
+        int a, at, b, bt;
+    };
+    std::vector<Src> src;
+    Src child_src(const Src &p, int c) const {
+        Src r;
+        const int ca = p.at == 0 ? a->child[p.a] : -1, cb = p.bt == 0 ? b->child[p.b] : -1;
+        r.a = ca >= 0 ? ca + c : p.a;
+        r.at = ca >= 0 ? 0 : p.at + 1;
+        r.b = cb >= 0 ? cb + c : p.b;
+        r.bt = cb >= 0 ? 0 : p.bt + 1;
+        return r;
+    }
+    void split(int i) {
+        out->split(i);
+        const Src p = src[i];
+        for (int c = 0; c < 8; c++) src.push_back(child_src(p, c));
+    }
+    void union_grid(int max_depth) {
+        if (a->n() == 0 || b->n() == 0) throw Error(MWG_ERR_STATE, "empty input tree");
+        out->make_roots();
+        src.clear();
+        for (int r : out->roots) {
+            const int ia = a->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+            const int ib = b->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+            if (ia < 0 || ib < 0) throw Error(MWG_ERR_STATE, "input tree does not cover the box");
+            src.push_back(Src{ia, 0, ib, 0});
+        }
+        for (int i = 0; i < out->n(); i++) {  // (breadth first: the nodes' own order)
+            const Src s = src[i];
+            const bool sp = (s.at == 0 && a->child[s.a] >= 0) || (s.bt == 0 && b->child[s.b] >= 0);
+            if (sp && out->depth[i] < max_depth) split(i);
+        }
+        work.resize(out->n());
+        for (int i = 0; i < out->n(); i++) work[i] = i;
+    }
+    void items_of(int job, MulItem *v) const {
+        for (size_t w = 0; w < work.size(); w++) {
+            const int i = work[w];
+            const Src &s = src[i];
+            v[w] = MulItem{i, out->depth[i], {out->lr[3 * i], out->lr[3 * i + 1], out->lr[3 * i + 2]},
+                           s.a, s.at, s.b, s.bt, job};
+        }
+    }
 };
 
+// f(j) for the jobs, on host threads where the work (nodes) is worth their start
+template <class F>
+static void for_jobs_of(size_t njobs, size_t nodes, F f) {
+    if (nodes < 4096)
+        for (size_t j = 0; j < njobs; j++) f(j);
+    else
+        for_each_job(njobs, f);
+}
+
+// the jobs' work nodes in one launch; their norms (8 per item, job by job from ofs[j]) on the host
+template <class LaunchFn>
+static const double *run_items(Ctx &C, std::vector<MulJob> &jobs, std::vector<size_t> &ofs, LaunchFn launch) {
+    std::vector<MulJobDev> jd(jobs.size());
+    ofs.assign(jobs.size() + 1, 0);
+    for (size_t j = 0; j < jobs.size(); j++) {
+        MulJob &J = jobs[j];
+        if (!J.work.empty()) J.out->ensure_dev(J.out->n());
+        jd[j] = MulJobDev{J.a->coef.p, J.b->coef.p, J.out->coef.p, J.out->norm.p, J.coef, J.coefb};
+        ofs[j + 1] = ofs[j] + J.work.size();
+    }
+    const size_t n = ofs[jobs.size()];
+    if (n == 0) return nullptr;
+    std::vector<MulItem> items(n);
+    for_jobs_of(jobs.size(), n, [&](size_t j) { jobs[j].items_of((int)j, items.data() + ofs[j]); });
+    upload_async(C, C.mitems, items.data(), n);
+    upload_async(C, C.mjobs, jd.data(), jd.size());
+    C.rbd.alloc(8 * n * sizeof(double));
+    launch((int)n, C.mitems.p, C.mjobs.p, (double *)C.rbd.p);
+    return read_compact(C, 8 * n);
+}
+
+// Independent products as one: all jobs' nodes of a refinement iteration in one launch (each
+// output identical to its single product) and one host round trip.
 static void multiply_batch(std::vector<MulJob> &jobs) {
     if (jobs.empty()) return;
     MraH &M = *jobs[0].a->mra;
     Ctx &C = *M.ctx;
-    hipStream_t s = C.stream;
-    for (MulJob &J : jobs)
+    size_t nodes = 0;
+    for (MulJob &J : jobs) {
         if (J.a->n() == 0 || J.b->n() == 0) throw Error(MWG_ERR_STATE, "multiply: empty input tree");
-    for_each_job(jobs.size(), [&](size_t j) {
-        MulJob &J = jobs[j];
-        TreeH &out = *J.out, &A = *J.a, &B = *J.b;
-        out.make_roots();
-        std::vector<int> order(out.roots.begin(), out.roots.end());
-        for (size_t w = 0; w < order.size(); w++) {
-            const int i = order[w];
-            const int d = out.depth[i], x = out.lr[3 * i], y = out.lr[3 * i + 1], z = out.lr[3 * i + 2];
-            const int ia = A.find(d, x, y, z), ib = B.find(d, x, y, z);
-            const bool sp = (ia >= 0 && A.child[ia] >= 0) || (ib >= 0 && B.child[ib] >= 0);
-            if (sp && d < M.maxDepth) {
-                out.split(i);
-                for (int a = 0; a < 8; a++) order.push_back(out.child[i] + a);
-            }
-        }
-        J.work.resize(out.n());
-        for (int i = 0; i < out.n(); i++) J.work[i] = i;
-    });
-    std::vector<MulItem> items;
-    std::vector<int> wl;
-    std::vector<size_t> ofs(jobs.size() + 1);
-    std::vector<std::vector<MulItem>> jitems(jobs.size());
-    while (true) {
-        for (MulJob &J : jobs)
-            if (!J.work.empty()) J.out->ensure_dev(J.out->n());
-        for_each_job(jobs.size(), [&](size_t j) {
-            MulJob &J = jobs[j];
-            std::vector<MulItem> &v = jitems[j];
-            v.resize(J.work.size());
-            for (size_t w = 0; w < J.work.size(); w++) {
-                const int i = J.work[w];
-                MulItem &it = v[w];
-                it.node = i;
-                it.depth = J.out->depth[i];
-                for (int q = 0; q < 3; q++) it.l[q] = J.out->lr[3 * i + q];
-                locate(*J.a, it.depth, it.l, it.asrc, it.asteps);
-                locate(*J.b, it.depth, it.l, it.bsrc, it.bsteps);
-            }
-        });
-        items.clear();
-        wl.clear();
-        for (size_t j = 0; j < jobs.size(); j++) {
-            ofs[j] = items.size();
-            items.insert(items.end(), jitems[j].begin(), jitems[j].end());
-            wl.insert(wl.end(), jobs[j].work.begin(), jobs[j].work.end());
-        }
-        ofs[jobs.size()] = items.size();
-        if (items.empty()) break;
-        upload_async(C, C.mitems, items.data(), items.size());
-        upload_async(C, C.mwork, wl.data(), wl.size());
-        size_t total = 0;
-        for (size_t j = 0; j < jobs.size(); j++) {
-            const int nj = (int)(ofs[j + 1] - ofs[j]);
-            if (!nj) continue;
-            MulJob &J = jobs[j];
-            HC(launch_multiply(s, nj, C.mitems.p + ofs[j], M.geom(), M.dev(), J.coef, J.a->coef.p, J.b->coef.p,
-                               J.out->coef.p));
-            HC(launch_norms(s, nj, C.mwork.p + ofs[j], J.out->coef.p, J.out->norm.p, J.out->K3()));
-            total += 8 * (size_t)J.out->n();
-        }
-        C.rb.reserve(total * sizeof(double));
-        double *h = (double *)C.rb.h;
-        size_t off = 0;
-        for (size_t j = 0; j < jobs.size(); j++) {
-            if (ofs[j + 1] == ofs[j]) continue;
-            const size_t m = 8 * (size_t)jobs[j].out->n();
-            HC(hipMemcpyAsync(h + off, jobs[j].out->norm.p, m * sizeof(double), hipMemcpyDeviceToHost, s));
-            off += m;
-        }
-        stream_wait(C);
-        C.stage.off = 0;
-        std::vector<size_t> hofs(jobs.size(), 0);
-        off = 0;
-        for (size_t j = 0; j < jobs.size(); j++) {
-            if (ofs[j + 1] == ofs[j]) continue;
-            hofs[j] = off;
-            off += 8 * (size_t)jobs[j].out->n();
-        }
-        for_each_job(jobs.size(), [&](size_t j) {
+        nodes += J.a->n() + J.b->n();
+    }
+    for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(M.maxDepth); });
+    std::vector<size_t> ofs;
+    while (const double *h = run_items(C, jobs, ofs, [&](int n, const MulItem *items, const MulJobDev *jd, double *cn) {
+               HC(launch_multiply(C.stream, n, items, jd, M.geom(), M.dev(), cn));
+           })) {
+        for_jobs_of(jobs.size(), ofs.back(), [&](size_t j) {
             if (ofs[j + 1] == ofs[j]) return;
             MulJob &J = jobs[j];
             TreeH &out = *J.out;
-            const double *nrm = h + hofs[j];
-            for (int i : J.work) {
-                std::memcpy(&out.cnorm[8 * (size_t)i], &nrm[8 * (size_t)i], 8 * sizeof(double));
-                if (J.first && out.depth[i] == 0) J.sNorm += nrm[8 * i] * nrm[8 * i];
-                for (int c = 1; c < 8; c++) J.wNorm += nrm[8 * i + c] * nrm[8 * i + c];
+            const double *nrm = h + 8 * ofs[j];
+            for (size_t w = 0; w < J.work.size(); w++) {
+                const int i = J.work[w];
+                const double *p = nrm + 8 * w;
+                std::memcpy(&out.cnorm[8 * (size_t)i], p, 8 * sizeof(double));
+                if (J.first && out.depth[i] == 0) J.sNorm += p[0] * p[0];
+                for (int c = 1; c < 8; c++) J.wNorm += p[c] * p[c];
             }
             J.first = false;
             const double tnorm = std::sqrt(J.sNorm + J.wNorm);
@@ -2663,93 +2622,38 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
                 const int d = out.depth[i];
                 if (d >= M.maxDepth) continue;
                 double wn = 0.0;
-                for (int c = 1; c < 8; c++) wn += out.cnorm[8 * i + c] * out.cnorm[8 * i + c];
+                for (int c = 1; c < 8; c++) wn += out.cnorm[8 * (size_t)i + c] * out.cnorm[8 * (size_t)i + c];
                 if (split_check(M.n0 + d, std::sqrt(wn), J.prec, tnorm)) {
-                    out.split(i);
+                    J.split(i);
                     for (int a = 0; a < 8; a++) next.push_back(out.child[i] + a);
                 }
             }
             J.work.swap(next);
         });
     }
-    // bottom-up compression, all jobs' parents of a depth in one launch
-    std::vector<std::vector<std::vector<int>>> L(jobs.size());
-    int maxd = 0;
-    for (size_t j = 0; j < jobs.size(); j++) {
-        L[j] = jobs[j].out->internal_by_depth();
-        maxd = std::max(maxd, (int)L[j].size());
-    }
-    std::vector<TransformItem> titems;
-    std::vector<size_t> lofs(maxd + 1, 0);
-    for (int d = 0; d < maxd; d++) {
-        lofs[d] = titems.size();
-        for (size_t j = 0; j < jobs.size(); j++)
-            if (d < (int)L[j].size())
-                for (int p : L[j][d]) titems.push_back({jobs[j].out->coef.p, nullptr, p, jobs[j].out->child[p]});
-    }
-    lofs[maxd] = titems.size();
-    if (!titems.empty()) {
-        upload_async(C, C.titems, titems.data(), titems.size());
-        for (int d = maxd - 1; d >= 0; d--)
-            HC(launch_transform(s, 0, (int)(lofs[d + 1] - lofs[d]), C.titems.p + lofs[d], M.W.p, M.B.K));
-    }
-    // every node's norms (as refresh_norms), one read-back for all jobs
-    size_t total = 0;
-    for (MulJob &J : jobs) {
-        HC(launch_norms(s, J.out->n(), nullptr, J.out->coef.p, J.out->norm.p, J.out->K3()));
-        total += 8 * (size_t)J.out->n();
-    }
-    C.rb.reserve(total * sizeof(double));
-    double *h = (double *)C.rb.h;
-    size_t off = 0;
-    for (MulJob &J : jobs) {
-        const size_t m = 8 * (size_t)J.out->n();
-        HC(hipMemcpyAsync(h + off, J.out->norm.p, m * sizeof(double), hipMemcpyDeviceToHost, s));
-        off += m;
-    }
-    stream_wait(C);
-    C.stage.off = 0;
-    off = 0;
-    for (MulJob &J : jobs) {
-        const size_t m = 8 * (size_t)J.out->n();
-        J.out->cnorm.assign(h + off, h + off + m);
-        off += m;
-        J.out->sqnorm_from_cnorm();
-        J.out->fit_dev();
-    }
+    std::vector<TreeH *> trees;
+    for (MulJob &J : jobs) trees.push_back(J.out);
+    compress_trees(C, M, trees);
 }
 
 // out = ca * a + cb * b on the union grid (mrcpp::add)
 static void add_trees(TreeH &out, double ca, TreeH &A, double cb, TreeH &B) {
     MraH &M = *A.mra;
     Ctx &C = *M.ctx;
-    hipStream_t s = C.stream;
     if (A.n() == 0 || B.n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
-    out.make_roots();
-    std::vector<int> order(out.roots.begin(), out.roots.end());
-    for (size_t w = 0; w < order.size(); w++) {
-        const int i = order[w];
-        const int d = out.depth[i], x = out.lr[3 * i], y = out.lr[3 * i + 1], z = out.lr[3 * i + 2];
-        const int ia = A.find(d, x, y, z), ib = B.find(d, x, y, z);
-        if ((ia >= 0 && A.child[ia] >= 0) || (ib >= 0 && B.child[ib] >= 0)) {
-            out.split(i);
-            for (int a = 0; a < 8; a++) order.push_back(out.child[i] + a);
-        }
-    }
-    out.ensure_dev(out.n());
-    std::vector<MulItem> items(out.n());
-    for (int i = 0; i < out.n(); i++) {
-        MulItem &it = items[i];
-        it.node = i;
-        it.depth = out.depth[i];
-        for (int q = 0; q < 3; q++) it.l[q] = out.lr[3 * i + q];
-        locate(A, it.depth, it.l, it.asrc, it.asteps);
-        locate(B, it.depth, it.l, it.bsrc, it.bsteps);
-    }
-    DBuf<MulItem> ditems;
-    ditems.upload(items.data(), items.size(), s);
-    HC(launch_add(s, (int)items.size(), ditems.p, M.dev(), ca, A.coef.p, cb, B.coef.p, out.coef.p));
-    out.refresh_norms();
+    std::vector<MulJob> jobs(1);
+    jobs[0].out = &out;
+    jobs[0].a = &A;
+    jobs[0].b = &B;
+    jobs[0].coef = ca;
+    jobs[0].coefb = cb;
+    jobs[0].union_grid(INT_MAX);
+    std::vector<size_t> ofs;
+    const double *h = run_items(C, jobs, ofs, [&](int n, const MulItem *items, const MulJobDev *jd, double *cn) {
+        HC(launch_add(C.stream, n, items, jd, M.dev(), cn));
+    });
+    out.cnorm.assign(h, h + 8 * (size_t)out.n());  // (the work list is every node in order)
+    out.sqnorm_from_cnorm();
 }
 
 }  // namespace mwg
@@ -2900,6 +2804,20 @@ int mwg_mra_create(mwg_ctx ctx, int root_scale, const int *corner, const int *bo
         for (int i = 0; i < N; i++)
             for (int j = 0; j < N; j++) WT[i * N + j] = m->B.W[j * N + i];
         m->WT.upload(WT.data(), WT.size(), s);
+        // row q of E: the value at point q of the children (half q / K of the cell) of every
+        // component function; C = its transpose times the quadrature weights
+        const int K = m->B.K;
+        std::vector<double> E(N * N), Cm(N * N);
+        for (int q = 0; q < N; q++)
+            for (int p = 0; p < N; p++) {
+                long double v = 0.0L;
+                for (int i = 0; i < K; i++)
+                    v += (long double)m->B.phiq[(q % K) * K + i] * m->B.W[p * N + (q / K) * K + i];
+                E[q * N + p] = (double)v;
+                Cm[p * N + q] = (double)(v * m->B.qw[q % K]);
+            }
+        m->E.upload(E.data(), E.size(), s);
+        m->C.upload(Cm.data(), Cm.size(), s);
         m->ccoef.upload(m->B.ccoef.data(), m->B.ccoef.size(), s);
     });
     if (rc) {
@@ -3354,17 +3272,21 @@ int mwg_project_gauss(double prec, mwg_tree out, int n, const double *coef, cons
     Ctx *C = out->mra->ctx;
     return guarded(C, [&] {
         hipStream_t s = C->stream;
-        DBuf<double> dc, da, dce, dp;
-        dc.upload(coef, n, s);
-        da.upload(alpha, n, s);
-        dce.upload(center, 3 * (size_t)n, s);
-        dp.upload(poly, 15 * (size_t)n, s);
+        // coef | alpha | center | poly
+        std::vector<double> par(20 * (size_t)n);
+        std::copy(coef, coef + n, par.begin());
+        std::copy(alpha, alpha + n, par.begin() + n);
+        std::copy(center, center + 3 * (size_t)n, par.begin() + 2 * (size_t)n);
+        std::copy(poly, poly + 15 * (size_t)n, par.begin() + 5 * (size_t)n);
+        upload_async(*C, C->ppar, par.data(), par.size());
+        const double *dp = C->ppar.p;
         std::vector<double> va(alpha, alpha + n), vc(center, center + 3 * (size_t)n);
         MraH &M = *out->mra;
         project_adaptive(
             *out, prec,
-            [&](int nw, const int *work, const int *depth, const int *lr, double *dst) {
-                HC(launch_project_gauss(s, nw, work, depth, lr, M.geom(), M.dev(), n, dc.p, da.p, dce.p, dp.p, dst));
+            [&](int nw, const MulItem *items, double *dst, double *norm, double *compact) {
+                HC(launch_project_gauss(s, nw, items, M.geom(), M.dev(), n, dp, dp + n, dp + 2 * n, dp + 5 * n, dst, norm,
+                                        compact));
             },
             &va, &vc);
     });
@@ -3376,16 +3298,18 @@ int mwg_project_hydrogen(double prec, mwg_tree out, int n, const double *coef, c
     Ctx *C = out->mra->ctx;
     return guarded(C, [&] {
         hipStream_t s = C->stream;
-        DBuf<double> dc, dorig;
-        DBuf<int> dq;
-        dc.upload(coef, n, s);
-        dq.upload(q, 6 * (size_t)n, s);
-        dorig.upload(origin, 3, s);
+        // coef | origin, and the quantum numbers
+        std::vector<double> par(coef, coef + n);
+        par.insert(par.end(), origin, origin + 3);
+        upload_async(*C, C->ppar, par.data(), par.size());
+        upload_async(*C, C->mwork, q, 6 * (size_t)n);
+        const double *dp = C->ppar.p;
+        const int *dq = C->mwork.p;
         MraH &M = *out->mra;
         project_adaptive(
             *out, prec,
-            [&](int nw, const int *work, const int *depth, const int *lr, double *dst) {
-                HC(launch_project_hyd(s, nw, work, depth, lr, M.geom(), M.dev(), n, dc.p, dq.p, Z, dorig.p, dst));
+            [&](int nw, const MulItem *items, double *dst, double *norm, double *compact) {
+                HC(launch_project_hyd(s, nw, items, M.geom(), M.dev(), n, dp, dq, Z, dp + n, dst, norm, compact));
             },
             nullptr, nullptr);
     });
@@ -3462,7 +3386,14 @@ int mwg_multiply(double prec, mwg_tree out, double coef, mwg_tree a, mwg_tree b)
     return guarded(C, [&] {
         if (out == a || out == b) throw Error(MWG_ERR_ARG, "multiply: output must differ from the inputs");
         if (!(prec > 0.0)) throw Error(MWG_ERR_ARG, "multiply: precision must be positive");
-        multiply_trees(*out, prec, coef, *a, *b);
+        std::vector<MulJob> jobs(1);
+        jobs[0].out = out;
+        jobs[0].a = a;
+        jobs[0].b = b;
+        jobs[0].prec = prec;
+        jobs[0].coef = coef;
+        jobs[0].coefb = 0.0;
+        multiply_batch(jobs);
     });
 }
 
@@ -3486,6 +3417,7 @@ int mwg_multiply_batch(int n, const double *prec, mwg_tree *out, const double *c
             jobs[i].b = b[i];
             jobs[i].prec = prec[i];
             jobs[i].coef = coef[i];
+            jobs[i].coefb = 0.0;
         }
         multiply_batch(jobs);
     });

@@ -38,6 +38,32 @@ __device__ inline int dhash_find(const DHash &h, uint64_t key) {
     return -1;
 }
 
+// sums over a block of 256 threads of 8 values per thread in a fixed order (lanes by butterfly,
+// then the waves); thread c < 8 gets the sum of value c
+__device__ inline double block_sum8(double (&ss)[8], double (*wsum)[8]) {
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss[c] += __shfl_xor(ss[c], o, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int c = 0; c < 8; c++) wsum[threadIdx.x >> 6][c] = ss[c];
+    __syncthreads();
+    const int c = threadIdx.x & 7;
+    return (wsum[0][c] + wsum[1][c]) + (wsum[2][c] + wsum[3][c]);
+}
+
+// a node's 8 component norms (from the threads' sums of squares) into the tree's array and, if
+// given, a compact one for the host
+__device__ inline void put_norms(double (&ss)[8], double (*wsum)[8], double *norm, double *compact) {
+    const double v = sqrt(block_sum8(ss, wsum));
+    if (threadIdx.x < 8) {
+        norm[threadIdx.x] = v;
+        if (compact) compact[threadIdx.x] = v;
+    }
+}
+
 // one active Gaussian term at the current depth, as the work-list build sees it
 constexpr int BM = 16;  // translations |d| < BM have precomputed combination masks
 struct TermTab {

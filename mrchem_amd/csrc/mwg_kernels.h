@@ -30,6 +30,9 @@ struct DevBasis {
     const double *qw;    // K
     const double *phiq;  // K x K, [q][i]
     const double *W;     // 2K x 2K
+    // products: components -> values at the quadrature points of the children, and values ->
+    // components with the quadrature weights (2K x 2K, row-major)
+    const double *E, *C;
 };
 
 struct ProjGeom {
@@ -161,12 +164,6 @@ hipError_t launch_dot(hipStream_t s, int n, const int *ia, const int *ib, const 
 hipError_t launch_dot_pairs(hipStream_t s, int n, const unsigned long long *pairs, const double *A,
                             const double *B, int K3, int nblocks, double *part, double *res);
 hipError_t launch_scale(hipStream_t s, size_t n, double *x, double c);
-hipError_t launch_project_gauss(hipStream_t s, int nw, const int *work, const int *depth, const int *lr,
-                                const ProjGeom &geo, const DevBasis &B, int nterm, const double *coef,
-                                const double *alpha, const double *center, const double *poly, double *out);
-hipError_t launch_project_hyd(hipStream_t s, int nw, const int *work, const int *depth, const int *lr,
-                              const ProjGeom &geo, const DevBasis &B, int nterm, const double *coef, const int *q,
-                              double Z, const double *origin, double *out);
 // the device loop's start of an iteration, done by the screening-box kernels (LoopJob etc.
 // are declared below): thresholds from the jobs' running norms instead of the tables'
 // (table jb = job jb), table counts cleared, work counters and contraction stamps reset,
@@ -219,11 +216,13 @@ hipError_t launch_contract_slices64(hipStream_t s, int K, int ntask, const TaskS
 hipError_t launch_stamp(hipStream_t s, unsigned long long *t);
 struct TransformItem {
     double *coef;
-    double *norm;  // component norms of the tree (null: not updated)
+    double *norm;  // component norms of the tree
     int parent;
     int first_child;
 };
-hipError_t launch_transform(hipStream_t s, int mode, int n, const TransformItem *items, const double *M, int K);
+// (compact: the parents' norms in item order, mode 0)
+hipError_t launch_transform(hipStream_t s, int mode, int n, const TransformItem *items, const double *M, int K,
+                            double *compact = nullptr);
 hipError_t launch_enum_mixed(hipStream_t s, int mode, int K, int nw, int nparts, const WorkItem *work,
                              const JobTab *jobs, const TermTab *tabs, const GenState &gs, int *thread_off,
                              int *seg_total, const long long *seg_ofs, Slice *out64, Slice *out16,
@@ -260,17 +259,32 @@ hipError_t launch_contract_mfma(hipStream_t s, int K, int ntask, const TaskSumma
                                 const SliceTask *tasks, const WorkItem *work, const JobTab *jobs,
                                 const TermTab *tabs, const Slice *slices, const double *genPool, double *nodeslots,
                                 long long *tabcnt, const uint4 *genPool16, const int *genExp16);
+// an output node of a product, sum or projection, with the inputs that represent it
 struct MulItem {
-    int node;          // output node
+    int node;
     int depth;
     int l[3];
     int asrc, asteps;  // input a: node (steps = 0) or leaf ancestor and levels to refine
     int bsrc, bsteps;
+    int job;
 };
-hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
-                           double coef, const double *acoef, const double *bcoef, double *out);
-hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const DevBasis &B, double ca, const double *acoef,
-                      double cb, const double *bcoef, double *out);
+// product (ca a b) or sum (ca a + cb b)
+struct MulJobDev {
+    const double *a, *b;
+    double *out, *norm;
+    double ca, cb;
+};
+// each writes the nodes' coefficients, their norms into the tree and into compact[8 item]
+hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const MulJobDev *jobs, const ProjGeom &geo,
+                           const DevBasis &B, double *compact);
+hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const MulJobDev *jobs, const DevBasis &B,
+                      double *compact);
+hipError_t launch_project_gauss(hipStream_t s, int nw, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
+                                int nterm, const double *coef, const double *alpha, const double *center,
+                                const double *poly, double *out, double *norm, double *compact);
+hipError_t launch_project_hyd(hipStream_t s, int nw, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
+                              int nterm, const double *coef, const int *q, double Z, const double *origin, double *out,
+                              double *norm, double *compact);
 // from the per-(node, segment, part) counts (nseg = 1: plain FP64, 2: mixed): part offsets,
 // task sizes, every node's first slices and tasks.  wchunk: slices per MFMA task, or (<= 0)
 // about -wchunk tasks over the iteration's slices.

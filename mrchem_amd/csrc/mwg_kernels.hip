@@ -235,65 +235,17 @@ __global__ void k_nsblocks(int n, const long long *item_delta, const int *item_r
     }
 }
 
-// ----------------------------------------------------------------- tensor line passes
-
-// (2K)^3 node tensor in LDS with the x rows padded to N + 1 doubles: x-lines (stride 1)
-// of neighbouring lanes then start 2(N+1) banks apart instead of 2N (no conflicts)
-template <int K>
-struct PadT {
-    static constexpr int N = 2 * K, P = N + 1, PL = N * P, SIZE = N * PL;
-};
-
-template <int K>
-__device__ inline int padded_index(int c, int e) {
-    constexpr int N = 2 * K, P = N + 1;
-    const int x = e % K, y = (e / K) % K, z = e / (K * K);
-    const int bx = c & 1, by = (c >> 1) & 1, bz = (c >> 2) & 1;
-    return ((bz * K + z) * N + (by * K + y)) * P + bx * K + x;
-}
-
-// in-place N x N filter on every line of the padded tensor along dim (0 = x)
-template <int N>
-__device__ inline void line_pass_padded(double *T, const double *M, int dim) {
-    constexpr int P = N + 1, N2 = N * N;
-    for (int line = threadIdx.x; line < N2; line += blockDim.x) {
-        const int u = line % N, v = line / N;
-        int base, stride;
-        if (dim == 0) {
-            base = line * P;
-            stride = 1;
-        } else if (dim == 1) {
-            base = v * N * P + u;
-            stride = P;
-        } else {
-            base = v * P + u;
-            stride = N * P;
-        }
-        double in[N];
-#pragma unroll
-        for (int q = 0; q < N; q++) in[q] = T[base + q * stride];
-        // (output rows two at a time: a full unroll would keep all N^2 matrix entries live)
-#pragma unroll 2
-        for (int p = 0; p < N; p++) {
-            double acc = 0.0;
-#pragma unroll
-            for (int q = 0; q < N; q++) acc += M[p * N + q] * in[q];
-            T[base + p * stride] = acc;
-        }
-    }
-}
-
-// component norms of listed nodes (one wave per node)
-__global__ void k_norms(int n, const int *nodes, const double *coef, double *norm, int K3) {
+// component norms of listed nodes (a workgroup per node, a wave per two components)
+__global__ void __launch_bounds__(256) k_norms(int n, const int *nodes, const double *coef, double *norm, int K3) {
     const int i = blockIdx.x;
     if (i >= n) return;
-    const int node = nodes ? nodes[i] : i;
+    const int node = nodes ? nodes[i] : i, lane = threadIdx.x & 63;
     const double *p = coef + (size_t)node * 8 * K3;
-    for (int c = 0; c < 8; c++) {
+    for (int c = threadIdx.x >> 6; c < 8; c += 4) {
         double s = 0.0;
-        for (int e = threadIdx.x; e < K3; e += 64) s += p[c * K3 + e] * p[c * K3 + e];
+        for (int e = lane; e < K3; e += 64) s += p[c * K3 + e] * p[c * K3 + e];
         for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        if (threadIdx.x == 0) norm[(size_t)node * 8 + c] = sqrt(s);
+        if (lane == 0) norm[(size_t)node * 8 + c] = sqrt(s);
     }
 }
 
@@ -349,16 +301,16 @@ __global__ void k_scale(size_t n, double *x, double c) {
 // Gaussian sums are separable: the children's scaling tensor is a sum of outer
 // products of 2K-vectors (one per dimension), and so is its compression.
 template <int K>
-__global__ void __launch_bounds__(256) k_project_gauss(int nw, const int *work, const int *depth, const int *lr,
-                                                       ProjGeom geo, DevBasis B, int nterm, const double *coef,
+__global__ void __launch_bounds__(256) k_project_gauss(const MulItem *items, ProjGeom geo, DevBasis B, int nterm, const double *coef,
                                                        const double *alpha, const double *center,
-                                                       const double *poly, double *out) {
+                                                       const double *poly, double *out, double *norm,
+                                                       double *compact) {
     constexpr int N = 2 * K, K3 = K * K * K;
     constexpr int LPER = (N * N + 255) / 256;  // x-lines (y, z) per thread
     constexpr int CH = 8;
     __shared__ double P[CH][3][N], WP[CH][3][N], Ws[N * N], cf[CH];
-    const int node = work[blockIdx.x];
-    const int d = depth[node];
+    const MulItem it = items[blockIdx.x];
+    const int node = it.node, d = it.depth;
     const double hc = geo.sfac * ldexp(1.0, -(geo.n0 + d + 1));
     const double pre = sqrt(hc);
     const int tid = threadIdx.x;
@@ -376,7 +328,7 @@ __global__ void __launch_bounds__(256) k_project_gauss(int nw, const int *work, 
             const int t = t0 + tt;
             double s = 0.0;
             if (t < nterm) {
-                const double x0 = geo.lo[dim] + hc * (double)(2 * lr[3 * node + dim] + bit);
+                const double x0 = geo.lo[dim] + hc * (double)(2 * it.l[dim] + bit);
                 const double c = center[3 * t + dim];
                 for (int q = 0; q < K; q++) {
                     const double u = x0 + hc * B.qx[q] - c;
@@ -415,110 +367,31 @@ __global__ void __launch_bounds__(256) k_project_gauss(int nw, const int *work, 
             }
         }
     }
+    __shared__ double wsum[4][8];
+    double ss[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int r = 0; r < LPER; r++) {
         const int line = tid + 256 * r;
         if (line < N * N) {
-            const int py = line % N, pz = line / N;
+            const int py = line % N, pz = line / N, hi = (py / K) | ((pz / K) << 1);
+            double *dst = out + (size_t)node * 8 * K3 + hi * 2 * K3 + ((pz % K) * K + (py % K)) * K;
+            double s[2] = {0.0, 0.0};
 #pragma unroll
             for (int px = 0; px < N; px++) {
-                const int c = (px / K) | ((py / K) << 1) | ((pz / K) << 2);
-                const int idx = ((pz % K) * K + (py % K)) * K + (px % K);
-                out[(size_t)node * 8 * K3 + c * K3 + idx] = acc[r][px];
+                dst[(px / K) * K3 + px % K] = acc[r][px];
+                s[px / K] += acc[r][px] * acc[r][px];
             }
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (hi == q) {
+                    ss[2 * q] += s[0];
+                    ss[2 * q + 1] += s[1];
+                }
         }
     }
-    (void)nw;
+    put_norms(ss, wsum, norm + (size_t)node * 8, compact + (size_t)blockIdx.x * 8);
 }
 
-__device__ double d_hydrogen_orb(int N, int L, int M, double Z, double x, double y, double z) {
-    const double r = sqrt(x * x + y * y + z * z);
-    double c0;
-    if (N == 1 && L == 0) c0 = 2.0;
-    else if (N == 2 && L == 0) c0 = 1.0 / (2.0 * sqrt(2.0));
-    else if (N == 3 && L == 0) c0 = 1.0 / (9.0 * sqrt(3.0));
-    else if (N == 2 && L == 1) c0 = 1.0 / (2.0 * sqrt(6.0));
-    else if (N == 3 && L == 1) c0 = 1.0 / (9.0 * sqrt(6.0));
-    else if (N == 3 && L == 2) c0 = 1.0 / (9.0 * sqrt(30.0));
-    else return 0.0;
-    c0 *= pow(Z, 1.5);
-    const double rho = 2.0 * Z / N * r;
-    double poly;
-    if (N == 1 && L == 0) poly = 1.0;
-    else if (N == 2 && L == 0) poly = 2.0 - rho;
-    else if (N == 3 && L == 0) poly = 6.0 - 6.0 * rho + rho * rho;
-    else if (N == 2 && L == 1) poly = rho;
-    else if (N == 3 && L == 1) poly = rho * (4.0 - rho);
-    else poly = rho * rho;
-    const double Rr = c0 * poly * exp(-rho / 2.0);
-    double ang, ca;
-    if (L == 0) {
-        ca = 1.0;
-        ang = 1.0;
-    } else if (L == 1) {
-        ca = sqrt(3.0);
-        const double q = (M == 0) ? x : (M == 1) ? y : z;
-        ang = (r > 0.0) ? q / r : 0.0;
-    } else {
-        const double r2 = r * r;
-        ca = (M <= 2) ? sqrt(15.0) : (M == 3 ? sqrt(15.0 / 4.0) : sqrt(5.0 / 4.0));
-        if (r2 == 0.0) ang = 0.0;
-        else if (M == 0) ang = x * y / r2;
-        else if (M == 1) ang = x * z / r2;
-        else if (M == 2) ang = y * z / r2;
-        else if (M == 3) ang = (x * x - y * y) / r2;
-        else ang = (2.0 * z * z - x * x - y * y) / r2;
-    }
-    return Rr * ca / (2.0 * sqrt(M_PI)) * ang;
-}
-
-// hydrogen functions are not separable: values at the K^3 quadrature points of
-// each child, then three 1D quadrature passes, then compression
-template <int K>
-__global__ void __launch_bounds__(256) k_project_hyd(int nw, const int *work, const int *depth, const int *lr,
-                                                     ProjGeom geo, DevBasis B, int nterm, const double *coef,
-                                                     const int *q, double Z, const double *origin, double *out) {
-    using L = PadT<K>;
-    constexpr int N = L::N, P = L::P, N3 = N * N * N, K3 = K * K * K;
-    extern __shared__ double smem[];
-    double *T = smem;
-    double *Ws = smem + L::SIZE;
-    double *Qm = Ws + N * N;  // N x N block-diagonal quadrature matrix: phi_i(x_q) w_q * pre
-    const int node = work[blockIdx.x];
-    const int d = depth[node];
-    const double hc = geo.sfac * ldexp(1.0, -(geo.n0 + d + 1));
-    const double pre = sqrt(hc);
-    for (int e = threadIdx.x; e < N * N; e += blockDim.x) {
-        Ws[e] = B.W[e];
-        const int p = e / N, qq = e % N;
-        Qm[e] = ((p / K) == (qq / K)) ? B.phiq[(qq % K) * K + (p % K)] * B.qw[qq % K] * pre : 0.0;
-    }
-    for (int e = threadIdx.x; e < N3; e += blockDim.x) {
-        const int px = e % N, py = (e / N) % N, pz = e / (N * N);
-        const double x = geo.lo[0] + hc * ((double)(2 * lr[3 * node] + px / K) + B.qx[px % K]) - origin[0];
-        const double y = geo.lo[1] + hc * ((double)(2 * lr[3 * node + 1] + py / K) + B.qx[py % K]) - origin[1];
-        const double z = geo.lo[2] + hc * ((double)(2 * lr[3 * node + 2] + pz / K) + B.qx[pz % K]) - origin[2];
-        double v = 0.0;
-        for (int t = 0; t < nterm; t++) {
-            double a = d_hydrogen_orb(q[6 * t], q[6 * t + 1], q[6 * t + 2], Z, x, y, z);
-            if (q[6 * t + 3] > 0) a *= d_hydrogen_orb(q[6 * t + 3], q[6 * t + 4], q[6 * t + 5], Z, x, y, z);
-            v += coef[t] * a;
-        }
-        T[(pz * N + py) * P + px] = v;
-    }
-    __syncthreads();
-    for (int dim = 0; dim < 3; dim++) {
-        line_pass_padded<N>(T, Qm, dim);
-        __syncthreads();
-    }
-    for (int dim = 0; dim < 3; dim++) {
-        line_pass_padded<N>(T, Ws, dim);
-        __syncthreads();
-    }
-    for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x)
-        out[(size_t)node * 8 * K3 + e] = T[padded_index<K>(e / K3, e % K3)];
-    (void)nw;
-}
 
 // ----------------------------------------------------------------- apply: generated nodes
 
@@ -650,170 +523,6 @@ __global__ void __launch_bounds__(256) k_gen_mark(int nw, const int *nwp, int *q
     const int n = nwp ? *nwp : nw;
     for_items(n, queue, [&](int i) { gen_mark_node(i, work, jobs, tabs, gs); });
 }
-
-// Refines the node tensor in T (padded (2K)^3, all 8 components of an ancestor) down
-// `steps` levels along the path bits of l (bit steps-1 first): the first step uses
-// the scaling and wavelet parts (2K -> K per line), the others the scaling part only.
-// The scaling block of the descendant is left at T[(z N + y) P + x], x, y, z < K.
-template <int K, class IT>
-__device__ void descend_padded(double *T, const double *Ws, const IT *l, int steps) {
-    using L = PadT<K>;
-    constexpr int N = L::N, P = L::P;
-    // first step: child a of the (s, d) parent; line (2K) -> K values, s_j = sum_p W[p][a*K+j] in_p
-    {
-        const int sh = steps - 1;
-        const int ax = (int)((l[0] >> sh) & 1), ay = (int)((l[1] >> sh) & 1), az = (int)((l[2] >> sh) & 1);
-        // x: lines (z, y) over all N x N
-        for (int line = threadIdx.x; line < N * N; line += blockDim.x) {
-            const int base = line * P;
-            double in[N];
-#pragma unroll
-            for (int p = 0; p < N; p++) in[p] = T[base + p];
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                double acc = 0.0;
-#pragma unroll
-                for (int p = 0; p < N; p++) acc += Ws[p * N + ax * K + j] * in[p];
-                T[base + j] = acc;
-            }
-        }
-        __syncthreads();
-        // y: lines (z, x < K)
-        for (int line = threadIdx.x; line < N * K; line += blockDim.x) {
-            const int z = line / K, x = line % K;
-            const int base = z * N * P + x;
-            double in[N];
-#pragma unroll
-            for (int p = 0; p < N; p++) in[p] = T[base + p * P];
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                double acc = 0.0;
-#pragma unroll
-                for (int p = 0; p < N; p++) acc += Ws[p * N + ay * K + j] * in[p];
-                T[base + j * P] = acc;
-            }
-        }
-        __syncthreads();
-        // z: lines (y < K, x < K)
-        for (int line = threadIdx.x; line < K * K; line += blockDim.x) {
-            const int y = line / K, x = line % K;
-            const int base = y * P + x;
-            double in[N];
-#pragma unroll
-            for (int p = 0; p < N; p++) in[p] = T[base + p * N * P];
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                double acc = 0.0;
-#pragma unroll
-                for (int p = 0; p < N; p++) acc += Ws[p * N + az * K + j] * in[p];
-                T[base + j * N * P] = acc;
-            }
-        }
-        __syncthreads();
-    }
-    // further steps: scaling-only descent, K x K filter per dimension
-    for (int sh = steps - 2; sh >= 0; sh--) {
-        const int a3[3] = {(int)((l[0] >> sh) & 1), (int)((l[1] >> sh) & 1), (int)((l[2] >> sh) & 1)};
-        for (int dim = 0; dim < 3; dim++) {
-            for (int line = threadIdx.x; line < K * K; line += blockDim.x) {
-                const int u = line % K, v = line / K;
-                int base, stride;
-                if (dim == 0) {
-                    base = (v * N + u) * P;
-                    stride = 1;
-                } else if (dim == 1) {
-                    base = v * N * P + u;
-                    stride = P;
-                } else {
-                    base = v * P + u;
-                    stride = N * P;
-                }
-                double in[K];
-#pragma unroll
-                for (int p = 0; p < K; p++) in[p] = T[base + p * stride];
-#pragma unroll
-                for (int j = 0; j < K; j++) {
-                    double acc = 0.0;
-#pragma unroll
-                    for (int p = 0; p < K; p++) acc += Ws[p * N + a3[dim] * K + j] * in[p];
-                    T[base + j * stride] = acc;
-                }
-            }
-            __syncthreads();
-        }
-    }
-}
-
-// scaling block of a generated node: reconstruct from the leaf ancestor (using its
-// wavelets for the first step), then refine with the low-pass filters only
-template <int K>
-__device__ void gen_one(int g, const JobTab *jobs, const GenState &gs, double *T, const double *Ws) {
-    using L = PadT<K>;
-    constexpr int N = L::N, P = L::P, K3 = K * K * K;
-    const uint64_t key = gs.keys[g];
-    const JobTab &J = jobs[gs.job[g]];
-    const int d = (int)(key >> 57);
-    const int64_t l[3] = {(int64_t)((key >> 38) & 0x7FFFF), (int64_t)((key >> 19) & 0x7FFFF), (int64_t)(key & 0x7FFFF)};
-    // the deepest ancestor present in the input tree: one thread per level probes it
-    __shared__ int s_anc, s_ad;
-    if (threadIdx.x == 0) {
-        s_anc = -1;
-        s_ad = -1;
-    }
-    __syncthreads();
-    const int my_dd = d - 1 - (int)threadIdx.x;
-    int my_a = -1;
-    if (my_dd >= 0) {
-        const int sh = d - my_dd;
-        my_a = dhash_find(J.inHash, dnode_key(my_dd, l[0] >> sh, l[1] >> sh, l[2] >> sh));
-        if (my_a >= 0) atomicMax(&s_ad, my_dd);
-    }
-    __syncthreads();
-    if (my_a >= 0 && my_dd == s_ad) s_anc = my_a;
-    __syncthreads();
-    const int anc = s_anc, ad = s_ad;
-    double *outp = gs.pool + (size_t)g * K3;
-    if (anc < 0) {
-        for (int e = threadIdx.x; e < K3; e += blockDim.x) outp[e] = 0.0;
-        if (threadIdx.x == 0) gs.norm[g] = 0.0;
-        __syncthreads();
-        return;
-    }
-    const double *src = J.inCoef + (size_t)anc * 8 * K3;
-    for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x) T[padded_index<K>(e / K3, e % K3)] = src[e];
-    __syncthreads();
-    descend_padded<K>(T, Ws, l, d - ad);
-    __shared__ double wsum[4];
-    double s2 = 0.0;
-    for (int e = threadIdx.x; e < K3; e += blockDim.x) {
-        const int x = e % K, y = (e / K) % K, z = e / (K * K);
-        const double v = T[(z * N + y) * P + x];
-        outp[e] = v;
-        s2 += v * v;
-    }
-    s2 = block_sum_256(s2, wsum);
-    if (threadIdx.x == 0) gs.norm[g] = sqrt(s2);
-    __syncthreads();
-}
-
-// Generated nodes first .. min(count, cap) - 1, count read from the device counter
-// that k_gen_mark advanced (no host round trip); grid-stride over the range.
-template <int K>
-__global__ void __launch_bounds__(256) k_gen_compute(int first, const int *firstp, int cap, const JobTab *jobs,
-                                                     GenState gs, const double *W) {
-    using L = PadT<K>;
-    constexpr int N = L::N;
-    extern __shared__ double smem[];
-    double *T = smem;
-    double *Ws = smem + L::SIZE;
-    if (firstp) first = *firstp;
-    const int end = min(*(volatile const int *)gs.count, cap);
-    if (first + (int)blockIdx.x >= end) return;
-    for (int e = threadIdx.x; e < N * N; e += blockDim.x) Ws[e] = W[e];
-    __syncthreads();
-    for (int g = first + blockIdx.x; g < end; g += gridDim.x) gen_one<K>(g, jobs, gs, T, Ws);
-}
-
 
 // Per output node, the input node (>= 0), generated node (-(g+1)) or nothing
 // (INT_MIN) at every translation of the union box over all terms, cached in LDS so
@@ -1885,72 +1594,6 @@ __global__ void __launch_bounds__(256) k_loop_emit(int njobs, LoopJob *lj, const
     }
 }
 
-// batched two-scale transforms over (tree, parent) items:
-// mode 0 compress children -> parent (and the parent's 8 component norms),
-// mode 1 add reconstruct(parent) to the children's scaling parts (and their norms)
-template <int K>
-__global__ void __launch_bounds__(256) k_transform(int mode, int n, const TransformItem *items, const double *M) {
-    using L = PadT<K>;
-    constexpr int N = L::N, K3 = K * K * K;
-    extern __shared__ double smem[];
-    __shared__ double wsum[4][8];
-    double *T = smem;
-    double *Ms = smem + L::SIZE;
-    const TransformItem it = items[blockIdx.x];
-    for (int e = threadIdx.x; e < N * N; e += blockDim.x) Ms[e] = M[e];
-    if (mode == 0) {
-        for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x) {
-            const int a = e / K3, r = e % K3;
-            T[padded_index<K>(a, r)] = it.coef[(size_t)(it.first_child + a) * 8 * K3 + r];
-        }
-    } else {
-        for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x)
-            T[padded_index<K>(e / K3, e % K3)] = it.coef[(size_t)it.parent * 8 * K3 + e];
-    }
-    __syncthreads();
-    for (int dim = 0; dim < 3; dim++) {
-        line_pass_padded<N>(T, Ms, dim);
-        __syncthreads();
-    }
-    double ss[8];
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        ss[c] = 0.0;
-        if (mode == 0) {
-            double *dst = it.coef + (size_t)it.parent * 8 * K3 + c * K3;
-            for (int r = threadIdx.x; r < K3; r += blockDim.x) {
-                const double v = T[padded_index<K>(c, r)];
-                dst[r] = v;
-                ss[c] += v * v;
-            }
-        } else {
-            double *dst = it.coef + (size_t)(it.first_child + c) * 8 * K3;
-            for (int r = threadIdx.x; r < K3; r += blockDim.x) {
-                const double v = dst[r] + T[padded_index<K>(c, r)];
-                dst[r] = v;
-                ss[c] += v * v;
-            }
-        }
-    }
-    // the 8 sums over the block at once (fixed order: lanes by butterfly, then waves 0..3)
-#pragma unroll
-    for (int c = 0; c < 8; c++)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) ss[c] += __shfl_xor(ss[c], o, 64);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int c = 0; c < 8; c++) wsum[threadIdx.x >> 6][c] = ss[c];
-    __syncthreads();
-    if (threadIdx.x < 8 && it.norm) {
-        const int c = threadIdx.x;
-        const double tot = (wsum[0][c] + wsum[1][c]) + (wsum[2][c] + wsum[3][c]);
-        if (mode == 0) it.norm[(size_t)it.parent * 8 + c] = sqrt(tot);
-        else it.norm[(size_t)(it.first_child + c) * 8] = sqrt(tot);
-    }
-    (void)n;
-}
-
-
 // ----------------------------------------------------------------- tree compaction
 
 // node groups (8 siblings) moved inside a tree: pair i copies the group at node
@@ -1971,115 +1614,7 @@ hipError_t launch_move_groups(hipStream_t s, int npairs, const int *from_to, dou
     return hipGetLastError();
 }
 
-// ----------------------------------------------------------------- pointwise multiplication
-
-// Loads the representation of an input tree at an output node into the padded node
-// tensor T: the node's 8 components when it exists (steps = 0), else the scaling block
-// refined from the leaf ancestor `src` over `steps` levels (path bits from l) with zero
-// wavelet components.
-template <int K>
-__device__ void load_rep_padded(double *T, const double *coef, int src, int steps, const int *l, const double *Ws) {
-    using L = PadT<K>;
-    constexpr int N = L::N, P = L::P, K3 = K * K * K;
-    const double *p = coef + (size_t)src * 8 * K3;
-    for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x) T[padded_index<K>(e / K3, e % K3)] = p[e];
-    __syncthreads();
-    if (steps == 0) return;
-    descend_padded<K>(T, Ws, l, steps);
-    for (int e = threadIdx.x; e < N * N * N; e += blockDim.x) {
-        const int x = e % N, y = (e / N) % N, z = e / (N * N);
-        if (x >= K || y >= K || z >= K) T[(z * N + y) * P + x] = 0.0;
-    }
-    __syncthreads();
-}
-
-// out = coef * a * b at the listed output nodes: both inputs to values at the K^3
-// quadrature points of the 8 children, product, quadrature projection, compression
-template <int K>
-__global__ void __launch_bounds__(256) k_multiply(int n, const MulItem *items, ProjGeom geo, DevBasis B, double coef,
-                                                  const double *acoef, const double *bcoef, double *out) {
-    using L = PadT<K>;
-    constexpr int N = L::N, P = L::P, N2 = N * N, K3 = K * K * K;
-    extern __shared__ double smem[];
-    double *Ta = smem;
-    double *Tb = Ta + L::SIZE;
-    double *Ws = Tb + L::SIZE;
-    double *WTs = Ws + N2;
-    double *Vs = WTs + N2;
-    double *Ps = Vs + N2;
-    const MulItem it = items[blockIdx.x];
-    for (int e = threadIdx.x; e < N2; e += blockDim.x) {
-        const int r = e / N, c = e % N;
-        Ws[e] = B.W[e];
-        WTs[e] = B.W[c * N + r];
-        const bool same = (r / K) == (c / K);
-        Vs[e] = same ? B.phiq[(r % K) * K + (c % K)] : 0.0;  // values: row = point q, col = function i
-        Ps[e] = same ? B.phiq[(c % K) * K + (r % K)] : 0.0;  // coefficients: row = function i, col = point q
-    }
-    __syncthreads();
-    load_rep_padded<K>(Ta, acoef, it.asrc, it.asteps, it.l, Ws);
-    load_rep_padded<K>(Tb, bcoef, it.bsrc, it.bsteps, it.l, Ws);
-    for (int dim = 0; dim < 3; dim++) {  // reconstruct to the children's scaling coefficients
-        line_pass_padded<N>(Ta, WTs, dim);
-        line_pass_padded<N>(Tb, WTs, dim);
-        __syncthreads();
-    }
-    for (int dim = 0; dim < 3; dim++) {  // values at the quadrature points
-        line_pass_padded<N>(Ta, Vs, dim);
-        line_pass_padded<N>(Tb, Vs, dim);
-        __syncthreads();
-    }
-    const double h = geo.sfac * ldexp(1.0, -(geo.n0 + it.depth + 1));
-    const double scale = coef / (h * sqrt(h));
-    for (int e = threadIdx.x; e < N * N2; e += blockDim.x) {
-        const int x = e % N, y = (e / N) % N, z = e / N2;
-        const int i = (z * N + y) * P + x;
-        Ta[i] = Ta[i] * Tb[i] * scale * B.qw[x % K] * B.qw[y % K] * B.qw[z % K];
-    }
-    __syncthreads();
-    for (int dim = 0; dim < 3; dim++) {  // projection onto the children's scaling functions
-        line_pass_padded<N>(Ta, Ps, dim);
-        __syncthreads();
-    }
-    for (int dim = 0; dim < 3; dim++) {  // compression to the node's 8 components
-        line_pass_padded<N>(Ta, Ws, dim);
-        __syncthreads();
-    }
-    for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x)
-        out[(size_t)it.node * 8 * K3 + e] = Ta[padded_index<K>(e / K3, e % K3)];
-    (void)n;
-}
-
-// out = ca * a + cb * b at the listed output nodes
-template <int K>
-__global__ void __launch_bounds__(256) k_add(int n, const MulItem *items, DevBasis B, double ca,
-                                             const double *acoef, double cb, const double *bcoef, double *out) {
-    using L = PadT<K>;
-    constexpr int N = L::N, K3 = K * K * K;
-    extern __shared__ double smem[];
-    double *Ta = smem;
-    double *Tb = Ta + L::SIZE;
-    double *Ws = Tb + L::SIZE;
-    for (int e = threadIdx.x; e < N * N; e += blockDim.x) Ws[e] = B.W[e];
-    __syncthreads();
-    const MulItem it = items[blockIdx.x];
-    load_rep_padded<K>(Ta, acoef, it.asrc, it.asteps, it.l, Ws);
-    load_rep_padded<K>(Tb, bcoef, it.bsrc, it.bsteps, it.l, Ws);
-    for (int e = threadIdx.x; e < 8 * K3; e += blockDim.x) {
-        const int idx = padded_index<K>(e / K3, e % K3);
-        out[(size_t)it.node * 8 * K3 + e] = ca * Ta[idx] + cb * Tb[idx];
-    }
-    (void)n;
-}
-
 // ----------------------------------------------------------------- launchers
-
-// kernels with more than 64 KiB of dynamic LDS must say so before their launch
-template <class Kern>
-static hipError_t allow_smem(Kern *k, size_t sm) {
-    if (sm <= 65536) return hipSuccess;
-    return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm);
-}
 
 hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
                          double pre, const DevBasis &B, const double *gx, const double *gw, double *out) {
@@ -2106,11 +1641,9 @@ hipError_t launch_nsblocks(hipStream_t s, int n, const long long *item_delta, co
     return hipGetLastError();
 }
 
-static size_t tensor_smem(int K) { return (size_t)(8 * K * K * K + 4 * K * K) * sizeof(double); }
-
 hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_norms, dim3(n), dim3(64), 0, s, n, nodes, coef, norm, K3);
+    hipLaunchKernelGGL(k_norms, dim3(n), dim3(256), 0, s, n, nodes, coef, norm, K3);
     return hipGetLastError();
 }
 
@@ -2135,27 +1668,12 @@ hipError_t launch_scale(hipStream_t s, size_t n, double *x, double c) {
     return hipGetLastError();
 }
 
-hipError_t launch_project_gauss(hipStream_t s, int nw, const int *work, const int *depth, const int *lr,
-                                const ProjGeom &geo, const DevBasis &B, int nterm, const double *coef,
-                                const double *alpha, const double *center, const double *poly, double *out) {
+hipError_t launch_project_gauss(hipStream_t s, int nw, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
+                                int nterm, const double *coef, const double *alpha, const double *center,
+                                const double *poly, double *out, double *norm, double *compact) {
     if (nw <= 0) return hipSuccess;
-    MWG_DISPATCH_K(B.K, hipLaunchKernelGGL(k_project_gauss<KK>, dim3(nw), dim3(256), 0, s, nw, work, depth, lr, geo,
-                                           B, nterm, coef, alpha, center, poly, out));
-    return hipGetLastError();
-}
-
-hipError_t launch_project_hyd(hipStream_t s, int nw, const int *work, const int *depth, const int *lr,
-                              const ProjGeom &geo, const DevBasis &B, int nterm, const double *coef, const int *q,
-                              double Z, const double *origin, double *out) {
-    if (nw <= 0) return hipSuccess;
-    const int K = B.K, N = 2 * K;
-    const size_t sm = (size_t)(N * N * (N + 1) + 2 * N * N) * sizeof(double);
-    MWG_DISPATCH_K(K, {
-        hipError_t e = allow_smem(k_project_hyd<KK>, sm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_project_hyd<KK>, dim3(nw), dim3(256), sm, s, nw, work, depth, lr, geo, B, nterm, coef,
-                           q, Z, origin, out);
-    });
+    MWG_DISPATCH_K(B.K, hipLaunchKernelGGL(k_project_gauss<KK>, dim3(nw), dim3(256), 0, s, items, geo, B, nterm, coef,
+                                           alpha, center, poly, out, norm, compact));
     return hipGetLastError();
 }
 
@@ -2173,22 +1691,6 @@ hipError_t launch_gen_mark(hipStream_t s, int nw, const WorkItem *work, const Jo
     if (nw <= 0) return hipSuccess;
     const int nb = nwp ? std::min(nw, DEVCOUNT_GRID) : nw;
     hipLaunchKernelGGL(k_gen_mark, dim3(nb), dim3(256), 0, s, nw, nwp, queue, work, jobs, tabs, gs);
-    return hipGetLastError();
-}
-
-// padded node tensor + one (2K)^2 filter matrix
-static size_t padded_smem(int K) { return (size_t)(2 * K * 2 * K * (2 * K + 1) + 4 * K * K) * sizeof(double); }
-
-hipError_t launch_gen_compute(hipStream_t s, int first, int cap, const JobTab *jobs, const GenState &gs,
-                              const double *W, int K, const int *firstp) {
-    if (cap <= first) return hipSuccess;
-    const size_t sm = padded_smem(K);
-    const int nb = std::min(cap - first, 2048);
-    MWG_DISPATCH_K(K, {
-        hipError_t e = allow_smem(k_gen_compute<KK>, sm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_gen_compute<KK>, dim3(nb), dim3(256), sm, s, first, firstp, cap, jobs, gs, W);
-    });
     return hipGetLastError();
 }
 
@@ -2241,17 +1743,6 @@ hipError_t launch_loop_emit(hipStream_t s, int njobs, LoopJob *lj, const WorkIte
     return hipGetLastError();
 }
 
-hipError_t launch_transform(hipStream_t s, int mode, int n, const TransformItem *items, const double *M, int K) {
-    if (n <= 0) return hipSuccess;
-    const size_t sm = padded_smem(K);
-    MWG_DISPATCH_K(K, {
-        hipError_t e = allow_smem(k_transform<KK>, sm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_transform<KK>, dim3(n), dim3(256), sm, s, mode, n, items, M);
-    });
-    return hipGetLastError();
-}
-
 hipError_t launch_build_tasks(hipStream_t s, int nw, int nseg, int nparts, int chunk, int wchunk, const int *tot,
                               TaskCaps caps, const int *gen_count, int gen_pcap, long long *ofs, NodeSched *nodes,
                               TaskSummary *sum, const int *gen_overflow, const int *nwp) {
@@ -2282,32 +1773,6 @@ hipError_t launch_enum_mixed(hipStream_t s, int mode, int K, int nw, int nparts,
     else
         hipLaunchKernelGGL(k_enum_mixed<1>, dim3(nb), dim3(256), 0, s, nw, nwp, queue, nparts, K * K, work, jobs,
                            tabs, gs, thread_off, seg_total, seg_ofs, out64, out16, sum, nodes, tasks, stasks);
-    return hipGetLastError();
-}
-
-hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
-                           double coef, const double *acoef, const double *bcoef, double *out) {
-    if (n <= 0) return hipSuccess;
-    const int K = B.K, N = 2 * K;
-    const size_t sm = (size_t)(2 * N * N * (N + 1) + 4 * N * N) * sizeof(double);
-    MWG_DISPATCH_K(K, {
-        hipError_t e = allow_smem(k_multiply<KK>, sm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_multiply<KK>, dim3(n), dim3(256), sm, s, n, items, geo, B, coef, acoef, bcoef, out);
-    });
-    return hipGetLastError();
-}
-
-hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const DevBasis &B, double ca, const double *acoef,
-                      double cb, const double *bcoef, double *out) {
-    if (n <= 0) return hipSuccess;
-    const int K = B.K, N = 2 * K;
-    const size_t sm = (size_t)(2 * N * N * (N + 1) + N * N) * sizeof(double);
-    MWG_DISPATCH_K(K, {
-        hipError_t e = allow_smem(k_add<KK>, sm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_add<KK>, dim3(n), dim3(256), sm, s, n, items, B, ca, acoef, cb, bcoef, out);
-    });
     return hipGetLastError();
 }
 

@@ -1,0 +1,57 @@
+"""Products, sums, projections and generated nodes at every order and in both bases.
+
+Each is a matrix along every line of a node's tensor, 4 x 4 blocks of rows and steps at a time:
+2K is a multiple of 4 or not, K is one, and the last tile of lines is full or not.  The inputs
+end at different depths, so nodes below a leaf by one, two and more levels are met.  Sums of at
+most 2K = 20 terms along three dimensions, a few passes deep, differ from the oracle's
+by its order of summation: 3 x 20 x 1.1e-16 per pass, 1e-12 of the largest coefficient for all.
+"""
+import numpy as np
+import pytest
+
+from mrchem_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    from mrchem_amd import mrcpp
+    mrcpp.default_context()
+    return mrcpp
+
+
+def _same(t, ref):
+    (d0, l0, c0), (d1, l1, c1) = t.export(), ref.export()
+    assert np.array_equal(d0, d1) and np.array_equal(l0, l1)
+    assert np.abs(c0 - c1).max() <= 1e-12 * np.abs(c1).max()
+
+
+@pytest.mark.parametrize("basis", ["L", "I"])
+@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8, 9])
+def test_inputs_of_different_depths(G, oracle, k, basis):
+    prec = 1e-3
+    orbs, _, _ = configs.orbitals(2, n_orb=2)
+    mra = G.mra_from(configs.BOX20, k, basis)
+    omra = oracle.MRA(**configs.BOX20, k=k, basis=basis, max_depth=16)
+    # a coarse tree, and one several levels deeper under some of its leaves
+    fa, fb = orbs[0], orbs[1]
+    oa = oracle.Tree(omra).project_gauss(0.3, fa)
+    ob = oracle.Tree(omra).project_gauss(1e-5, fb)
+    a, b = G.project(0.3, G.FunctionTree(mra), fa), G.project(1e-5, G.FunctionTree(mra), fb)
+    _same(a, oa)
+    _same(b, ob)
+    da, db = a.export()[0], b.export()[0]
+    assert db.max() >= da.max() + 2
+    for (x, y), (ox, oy) in (((a, b), (oa, ob)), ((b, a), (ob, oa))):
+        _same(G.multiply(prec, G.FunctionTree(mra), 1.5, x, y),
+              oracle.multiply(prec, oracle.Tree(omra), 1.5, ox, oy))
+        s = G.add(G.FunctionTree(mra), 0.7, x, -1.3, y)
+        pts = np.random.default_rng(3).uniform(-6, 6, (500, 3))
+        ex = 0.7 * x.evalf(pts) - 1.3 * y.evalf(pts)
+        assert np.abs(s.evalf(pts) - ex).max() <= 1e-12 * np.abs(ex).max()
+    # an apply finer than its input: scaling blocks generated below the input's leaves
+    out, oout = G.FunctionTree(mra), oracle.Tree(omra)
+    G.apply(prec, out, G.PoissonOperator(mra, prec), a)
+    oracle.apply(prec, oout, oracle.Oper(omra, 0.0, prec), oa)
+    _same(out, oout)
