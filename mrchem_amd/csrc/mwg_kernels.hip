@@ -1255,6 +1255,32 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
+// The sum of n slots, in order, SLOT_FLY reads in flight.  One at a time, the latency of the reads
+// was the kernel's time: 18.6 us per launch of a Poisson apply at k = 5 (6.2 now), 39 of a
+// Coulomb potential at k = 7 (10), 59 of eight Helmholtz applies at k = 9 (43; there the traffic
+// counts too).  Workgroups of 1024 with a quarter of the slots each were no better for few nodes
+// (8 and 14 us) and slower for many (75).
+constexpr int SLOT_FLY = 16;
+
+__device__ inline double sum_slots(const double *p, int n, size_t stride) {
+    double s = 0.0;
+    int q = 0;
+    for (; q + SLOT_FLY <= n; q += SLOT_FLY) {
+        double v[SLOT_FLY];
+#pragma unroll
+        for (int i = 0; i < SLOT_FLY; i++) v[i] = p[(q + i) * stride];
+#pragma unroll
+        for (int i = 0; i < SLOT_FLY; i++) s += v[i];
+    }
+    if (q == n) return s;
+    double v[SLOT_FLY];
+#pragma unroll
+    for (int i = 0; i < SLOT_FLY; i++) v[i] = q + i < n ? p[(q + i) * stride] : 0.0;
+#pragma unroll
+    for (int i = 0; i < SLOT_FLY; i++) s += v[i];
+    return s;
+}
+
 // Sums the task slots of an output component in a fixed order (FP64 tasks, then MFMA tasks)
 // into the node, and its norm into the tree and the compact per-work-node array.  One
 // workgroup per (work node, component).
@@ -1276,9 +1302,7 @@ __global__ void __launch_bounds__(256) k_reduce_slots(int nw, const int *nwp, co
         const double *p16 = slots16 + ((size_t)nd.task16 * 8 + gt) * K3;
         double ss = 0.0;
         for (int e = threadIdx.x; e < K3; e += blockDim.x) {
-            double s = 0.0;
-            for (int q = 0; q < n64; q++) s += p64[(size_t)q * 8 * K3 + e];
-            for (int q = 0; q < n16; q++) s += p16[(size_t)q * 8 * K3 + e];
+            const double s = sum_slots(p64 + e, n64, (size_t)8 * K3) + sum_slots(p16 + e, n16, (size_t)8 * K3);
             dst[e] = s;
             ss += s * s;
         }
