@@ -205,6 +205,10 @@ int mwg_multiply_batch(int n, const double *prec, mwg_tree *out, const double *c
  * QMFunction::add / qmfunction::linear_combination (src/qmfunctions/QMFunction.cpp:157-200):
  * out = ca*a + cb*b on the union grid of a and b (exact in the compressed representation). */
 int mwg_add(mwg_tree out, double ca, mwg_tree a, double cb, mwg_tree b);
+/* n linear combinations out[i] = sum_k coef_k f_k, each on the union grid of its nterms[i] >= 1
+ * terms; coef and inp hold the terms of all, one combination after the other.  As a chain of
+ * mwg_add, with one launch for everything. */
+int mwg_add_batch(int n, mwg_tree *out, const int *nterms, const double *coef, mwg_tree *inp);
 
 /* ---- operators: replace new mrcpp::PoissonOperator(MRA, prec) (SCFDriver.cpp:279) and
  * mrcpp::HelmholtzOperator(MRA, mu, prec) (HelmholtzVector.cpp:171).  Kernels 1/r and

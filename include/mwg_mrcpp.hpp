@@ -289,33 +289,20 @@ inline void add(double prec, FunctionTree<3> &out, double a, FunctionTree<3> &in
 template <int D>
 using FunctionTreeVector = std::vector<std::tuple<double, FunctionTree<D> *>>;
 
-// out = sum_i c_i f_i (QMFunction::add / qmfunction::linear_combination), by pairwise
-// exact union-grid sums
+// out = sum_i c_i f_i (QMFunction::add / qmfunction::linear_combination) on the union grid
 inline void add(double prec, FunctionTree<3> &out, FunctionTreeVector<3> &inp, int maxIter = -1) {
+    (void)prec;
     (void)maxIter;
     if (inp.empty()) throw Error("mrcpp::add: empty FunctionTreeVector");
-    if (inp.size() == 1) {
-        // c * f: f + 0 f on f's grid, then the scale
-        detail::check(mwg_add(out.handle(), std::get<0>(inp[0]), std::get<1>(inp[0])->handle(), 0.0,
-                              std::get<1>(inp[0])->handle()));
-        return;
+    std::vector<double> coef;
+    std::vector<mwg_tree> f;
+    for (auto &t : inp) {
+        coef.push_back(std::get<0>(t));
+        f.push_back(std::get<1>(t)->handle());
     }
-    std::vector<std::unique_ptr<mwg_tree_s, int (*)(mwg_tree)>> tmp;
-    mwg_tree acc = std::get<1>(inp[0])->handle();
-    double cacc = std::get<0>(inp[0]);
-    for (size_t i = 1; i < inp.size(); i++) {
-        mwg_tree t = (i + 1 == inp.size()) ? out.handle() : nullptr;
-        if (!t) {
-            mwg_mra m = nullptr;
-            detail::check(mwg_tree_mra(acc, &m));
-            detail::check(mwg_tree_create(m, &t));
-            tmp.emplace_back(t, mwg_tree_destroy);
-        }
-        detail::check(mwg_add(t, cacc, acc, std::get<0>(inp[i]), std::get<1>(inp[i])->handle()));
-        acc = t;
-        cacc = 1.0;
-    }
-    (void)prec;
+    mwg_tree o = out.handle();
+    const int n = (int)inp.size();
+    detail::check(mwg_add_batch(1, &o, &n, coef.data(), f.data()));
 }
 
 // copy_func: out = inp (grid and coefficients); copy_grid: inp's grid, zero coefficients;

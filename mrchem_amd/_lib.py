@@ -98,6 +98,7 @@ def _sig():
         "mwg_multiply": [d, vp, d, vp, vp],
         "mwg_multiply_batch": [i, fd, pvp, fd, pvp, pvp],
         "mwg_add": [vp, d, vp, d, vp],
+        "mwg_add_batch": [i, pvp, fi, fd, pvp],
         "mwg_apply": [d, vp, vp, vp, i, u, C.POINTER(ApplyStats)],
         "mwg_apply_batch": [i, fd, pvp, pvp, pvp, i, u, C.POINTER(ApplyStats)],
         "mwg_predictor_create": [vp, C.c_uint64, pvp],
@@ -124,7 +125,7 @@ EXPORTED = ["mwg_ctx_create", "mwg_ctx_destroy", "mwg_last_error", "mwg_sync", "
             "mwg_tree_eval", "mwg_meta_write", "mwg_meta_read", "mwg_tree_save", "mwg_tree_load",
             "mwg_tree_file_write", "mwg_tree_file_read",
             "mwg_project_gauss", "mwg_project_hydrogen", "mwg_oper_poisson", "mwg_oper_helmholtz",
-            "mwg_oper_destroy", "mwg_oper_nterms", "mwg_oper_terms", "mwg_oper_blocks", "mwg_multiply", "mwg_multiply_batch", "mwg_add", "mwg_apply",
+            "mwg_oper_destroy", "mwg_oper_nterms", "mwg_oper_terms", "mwg_oper_blocks", "mwg_multiply", "mwg_multiply_batch", "mwg_add", "mwg_add_batch", "mwg_apply",
             "mwg_apply_batch", "mwg_predictor_create", "mwg_predictor_destroy", "mwg_predictor_sizes",
             "mwg_predictor_get", "mwg_predictor_set", "mwg_predictor_train", "mwg_predictor_gradient",
             "mwg_predictor_infer", "mwg_ctx_set_predictor", "mwg_trace_enable", "mwg_trace_size", "mwg_trace_get"]

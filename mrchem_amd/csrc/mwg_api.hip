@@ -284,8 +284,10 @@ struct Ctx {
     DBuf<unsigned long long> genHashKeys;
     DBuf<int> genHashVals;
     DBuf<TransformItem> titems;
-    DBuf<MulItem> mitems;  // products, sums, projections: items of all jobs, and the jobs
+    DBuf<MulItem> mitems;  // products and projections: items of all jobs, and the jobs
     DBuf<MulJobDev> mjobs;
+    DBuf<SumItem> sitems;  // linear combinations: output nodes and their terms
+    DBuf<SumSrc> ssrcs;
     DBuf<double> ppar;  // parameters of a projected function
     DBuf<int> mwork;    // (quantum numbers)
     // FP64 slices, tasks and slots; the same for the MFMA slices
@@ -2500,12 +2502,12 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
 
 // ------------------------------------------------------------------ multiplication
 
-// Products and sums: out on the union grid of a and b (products are refined further).  For every
+// Products: out on the union grid of a and b, refined further.  For every
 // output node the input node that represents it (steps 0) or its leaf ancestor and the levels
 // between, known from the parent's as the nodes are made.
 struct MulJob {
     TreeH *out, *a, *b;
-    double prec, coef, coefb;
+    double prec, coef;
     std::vector<int> work;
     double sNorm = 0.0, wNorm = 0.0;
     bool first = true;
@@ -2572,7 +2574,7 @@ static const double *run_items(Ctx &C, std::vector<MulJob> &jobs, std::vector<si
     for (size_t j = 0; j < jobs.size(); j++) {
         MulJob &J = jobs[j];
         if (!J.work.empty()) J.out->ensure_dev(J.out->n());
-        jd[j] = MulJobDev{J.a->coef.p, J.b->coef.p, J.out->coef.p, J.out->norm.p, J.coef, J.coefb};
+        jd[j] = MulJobDev{J.a->coef.p, J.b->coef.p, J.out->coef.p, J.out->norm.p, J.coef};
         ofs[j + 1] = ofs[j] + J.work.size();
     }
     const size_t n = ofs[jobs.size()];
@@ -2636,24 +2638,90 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
     compress_trees(C, M, trees);
 }
 
-// out = ca * a + cb * b on the union grid (mrcpp::add)
-static void add_trees(TreeH &out, double ca, TreeH &A, double cb, TreeH &B) {
-    MraH &M = *A.mra;
+// A linear combination out = sum of coef_k f_k on the union grid of its terms.
+struct SumJob {
+    TreeH *out;
+    std::vector<double> coef;
+    std::vector<TreeH *> f;
+    struct Src {
+        int node, steps;
+    };
+    std::vector<Src> src;  // per output node and term
+    void union_grid() {
+        const size_t m = f.size();
+        size_t most = 0;
+        for (TreeH *t : f) {
+            if (t->n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
+            most = std::max(most, (size_t)t->n());
+        }
+        out->make_roots();
+        out->reserve_host(most);
+        src.clear();
+        src.reserve(most * m);
+        for (int r : out->roots)
+            for (TreeH *t : f) {
+                const int i = t->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+                if (i < 0) throw Error(MWG_ERR_STATE, "input tree does not cover the box");
+                src.push_back(Src{i, 0});
+            }
+        for (int i = 0; i < out->n(); i++) {  // (breadth first: the nodes' own order)
+            bool sp = false;
+            for (size_t k = 0; k < m; k++) {
+                const Src s = src[i * m + k];
+                sp = sp || (s.steps == 0 && f[k]->child[s.node] >= 0);
+            }
+            if (!sp) continue;
+            out->split(i);
+            for (int c = 0; c < 8; c++)
+                for (size_t k = 0; k < m; k++) {
+                    const Src s = src[i * m + k];
+                    const int ch = s.steps == 0 ? f[k]->child[s.node] : -1;
+                    src.push_back(ch >= 0 ? Src{ch + c, 0} : Src{s.node, s.steps + 1});
+                }
+        }
+    }
+};
+
+// Linear combinations as one launch: every output node of every combination (mrcpp::add)
+static void sum_batch(std::vector<SumJob> &jobs) {
+    MraH &M = *jobs[0].out->mra;
     Ctx &C = *M.ctx;
-    if (A.n() == 0 || B.n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
-    std::vector<MulJob> jobs(1);
-    jobs[0].out = &out;
-    jobs[0].a = &A;
-    jobs[0].b = &B;
-    jobs[0].coef = ca;
-    jobs[0].coefb = cb;
-    jobs[0].union_grid(INT_MAX);
-    std::vector<size_t> ofs;
-    const double *h = run_items(C, jobs, ofs, [&](int n, const MulItem *items, const MulJobDev *jd, double *cn) {
-        HC(launch_add(C.stream, n, items, jd, M.dev(), cn));
+    size_t nodes = 0;
+    for (SumJob &J : jobs)
+        for (TreeH *t : J.f) nodes += t->n();
+    for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(); });
+    std::vector<size_t> iofs(jobs.size() + 1, 0), sofs(jobs.size() + 1, 0);
+    for (size_t j = 0; j < jobs.size(); j++) {
+        jobs[j].out->ensure_dev(jobs[j].out->n());
+        iofs[j + 1] = iofs[j] + jobs[j].out->n();
+        sofs[j + 1] = sofs[j] + jobs[j].src.size();
+    }
+    const size_t n = iofs.back(), ns = sofs.back(), B8 = 8 * (size_t)M.B.K3;
+    if (ns > (size_t)INT_MAX) throw Error(MWG_ERR_RANGE, "add: too many nodes and terms for one call");
+    std::vector<SumItem> items(n);
+    std::vector<SumSrc> srcs(ns);
+    for_jobs_of(jobs.size(), ns, [&](size_t j) {
+        const SumJob &J = jobs[j];
+        const TreeH &T = *J.out;
+        const int m = (int)J.f.size();
+        for (int i = 0; i < T.n(); i++)
+            items[iofs[j] + i] = SumItem{T.coef.p + i * B8, T.norm.p + 8 * (size_t)i,
+                                         T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2],
+                                         (int)(sofs[j] + (size_t)i * m), m};
+        for (size_t q = 0; q < J.src.size(); q++) {
+            const int k = (int)(q % m);
+            srcs[sofs[j] + q] = SumSrc{J.f[k]->coef.p + J.src[q].node * B8, J.coef[k], J.src[q].steps};
+        }
     });
-    out.cnorm.assign(h, h + 8 * (size_t)out.n());  // (the work list is every node in order)
-    out.sqnorm_from_cnorm();
+    upload_async(C, C.sitems, items.data(), n);
+    upload_async(C, C.ssrcs, srcs.data(), ns);
+    C.rbd.alloc(8 * n * sizeof(double));
+    HC(launch_sum(C.stream, (int)n, C.sitems.p, C.ssrcs.p, M.dev(), (double *)C.rbd.p));
+    const double *h = read_compact(C, 8 * n);
+    for (size_t j = 0; j < jobs.size(); j++) {  // (the items are every node in order)
+        jobs[j].out->cnorm.assign(h + 8 * iofs[j], h + 8 * iofs[j + 1]);
+        jobs[j].out->sqnorm_from_cnorm();
+    }
 }
 
 }  // namespace mwg
@@ -3392,7 +3460,6 @@ int mwg_multiply(double prec, mwg_tree out, double coef, mwg_tree a, mwg_tree b)
         jobs[0].b = b;
         jobs[0].prec = prec;
         jobs[0].coef = coef;
-        jobs[0].coefb = 0.0;
         multiply_batch(jobs);
     });
 }
@@ -3417,19 +3484,49 @@ int mwg_multiply_batch(int n, const double *prec, mwg_tree *out, const double *c
             jobs[i].b = b[i];
             jobs[i].prec = prec[i];
             jobs[i].coef = coef[i];
-            jobs[i].coefb = 0.0;
         }
         multiply_batch(jobs);
     });
 }
 
 int mwg_add(mwg_tree out, double ca, mwg_tree a, double cb, mwg_tree b) {
-    if (!out || !a || !b) return MWG_ERR_ARG;
-    if (a->mra != b->mra || out->mra != a->mra) return MWG_ERR_ARG;
-    Ctx *C = a->mra->ctx;
-    return guarded(C, [&] {
-        if (out == a || out == b) throw Error(MWG_ERR_ARG, "add: output must differ from the inputs");
-        add_trees(*out, ca, *a, cb, *b);
+    const int two = 2;
+    const double coef[2] = {ca, cb};
+    mwg_tree inp[2] = {a, b};
+    return mwg_add_batch(1, &out, &two, coef, inp);
+}
+
+int mwg_add_batch(int n, mwg_tree *out, const int *nterms, const double *coef, mwg_tree *inp) {
+    if (n <= 0 || !out || !nterms || !coef || !inp) return MWG_ERR_ARG;
+    size_t total = 0;
+    for (int i = 0; i < n; i++) {
+        if (!out[i] || nterms[i] <= 0) return MWG_ERR_ARG;
+        total += nterms[i];
+    }
+    for (size_t q = 0; q < total; q++)
+        if (!inp[q]) return MWG_ERR_ARG;
+    MraH *M = inp[0]->mra;
+    for (int i = 0; i < n; i++)
+        if (out[i]->mra != M) return MWG_ERR_ARG;
+    for (size_t q = 0; q < total; q++)
+        if (inp[q]->mra != M) return MWG_ERR_ARG;
+    return guarded(M->ctx, [&] {
+        std::vector<const void *> outs(out, out + n);
+        std::sort(outs.begin(), outs.end());
+        bool clash = std::adjacent_find(outs.begin(), outs.end()) != outs.end();
+        for (size_t q = 0; q < total; q++)
+            clash = clash || std::binary_search(outs.begin(), outs.end(), (const void *)inp[q]);
+        if (clash) throw Error(MWG_ERR_ARG, "add: outputs must differ from the inputs and each other");
+        std::vector<SumJob> jobs(n);
+        size_t q = 0;
+        for (int i = 0; i < n; i++) {
+            jobs[i].out = out[i];
+            for (int k = 0; k < nterms[i]; k++, q++) {
+                jobs[i].coef.push_back(coef[q]);
+                jobs[i].f.push_back(inp[q]);
+            }
+        }
+        sum_batch(jobs);
     });
 }
 

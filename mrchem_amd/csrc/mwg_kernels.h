@@ -268,16 +268,28 @@ struct MulItem {
     int bsrc, bsteps;
     int job;
 };
-// product (ca a b) or sum (ca a + cb b)
+// product (coef a b)
 struct MulJobDev {
     const double *a, *b;
     double *out, *norm;
-    double ca, cb;
+    double coef;
+};
+// an output node of a linear combination: its coefficients and norms, its terms
+struct SumItem {
+    double *out, *norm;
+    int lx, ly, lz;
+    int src0, nsrc;
+};
+// a term: the node (steps = 0) or leaf ancestor that represents the input, levels to refine
+struct SumSrc {
+    const double *p;
+    double coef;
+    long long steps;
 };
 // each writes the nodes' coefficients, their norms into the tree and into compact[8 item]
 hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const MulJobDev *jobs, const ProjGeom &geo,
                            const DevBasis &B, double *compact);
-hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const MulJobDev *jobs, const DevBasis &B,
+hipError_t launch_sum(hipStream_t s, int n, const SumItem *items, const SumSrc *srcs, const DevBasis &B,
                       double *compact);
 hipError_t launch_project_gauss(hipStream_t s, int nw, const MulItem *items, const ProjGeom &geo, const DevBasis &B,
                                 int nterm, const double *coef, const double *alpha, const double *center,

@@ -8,7 +8,7 @@
 // instruction, the same for the 4 blocks), 16 lines as the columns of B, 4 products long.  One
 // thread per line with the matrix read from LDS for every product was bound by those reads.
 // Before and after (kernel time, norms launches not counted): the products of an eight-orbital
-// exchange step at k = 7, 34.7 ms -> 6.2; its sums, 113 us per launch -> 43; k_transform
+// exchange step at k = 7, 34.7 ms -> 6.2; k_transform
 // 17.7 -> 8.7 us (k = 7, Coulomb potential of six Gaussians) and 48 -> 19 (k = 9, eight
 // Helmholtz applies); k_gen_compute there 58 -> 33.  What bounds them now is the latency of one node's
 // chain (read, three or nine passes with a barrier each, write), 2 to 3 workgroups per CU.
@@ -357,7 +357,7 @@ k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B
         __syncthreads();
     }
     const double h = geo.sfac * ldexp(1.0, -(geo.n0 + it.depth + 1));
-    const double scale = J.ca / (h * sqrt(h));
+    const double scale = J.coef / (h * sqrt(h));
     double ss[8];
 #pragma unroll
     for (int c = 0; c < 8; c++) {
@@ -373,27 +373,29 @@ k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B
 
 // ----------------------------------------------------------------- sums
 
-// out = ca * a + cb * b at the listed output nodes.  An input that ends above the node
-// contributes its descended scaling block only (the wavelet parts below a leaf are zero).
+// out = sum of coef_k f_k at the listed output nodes, all terms at once.  A term that ends above
+// the node contributes its descended scaling block only (the wavelet parts below a leaf are
+// zero).  Bound by the reads of the terms, so two terms' are in flight.  As a chain of pairwise sums
+// the 56 sums of an eight-orbital exchange step (k = 7) wrote and read every partial sum and
+// cost a union grid and a round trip each: the SCF step of four orbitals 9.2 -> 7.6 ms, the density
+// and Coulomb potential of six 4.1 -> 3.1, a five-orbital exchange step 20.9 -> 18.8.
 template <int K>
-__global__ void __launch_bounds__(256) k_add(const MulItem *items, const MulJobDev *jobs, DevBasis B,
-                                             double *compact) {
+__global__ void __launch_bounds__(256) k_sum(const SumItem *items, const SumSrc *srcs, DevBasis B, double *compact) {
     using L = PadT<K>;
-    constexpr int N = L::N, P = L::P, K3 = K * K * K, KN = K * N;
+    constexpr int N = L::N, P = L::P, K3 = K * K * K, KN = K * N, PER = NodeRegs<K>::PER;
     extern __shared__ double smem[];
     __shared__ double wsum[4][8];
     double *T = smem, *F = T + L::SIZE, *sc = F + 3 * KN;
-    const MulItem it = items[blockIdx.x];
-    const MulJobDev J = jobs[it.job];
-    const double *src[2] = {J.a + (size_t)it.asrc * 8 * K3, J.b + (size_t)it.bsrc * 8 * K3};
-    const int steps[2] = {it.asteps, it.bsteps};
-    const double cf[2] = {J.ca, J.cb};
+    const SumItem it = items[blockIdx.x];
+    const SumSrc *src = srcs + it.src0;
     bool any = false;  // sc holds the descended parts
-    for (int q = 0; q < 2; q++) {
-        if (steps[q] == 0) continue;
+    for (int q = 0; q < it.nsrc; q++) {
+        const SumSrc t = src[q];
+        if (t.steps == 0) continue;
         NodeRegs<K> in;
-        in.load([&](unsigned e) { return src[q] + e; });
-        descent_matrices<K>(F, T, B.W, it.l[0], it.l[1], it.l[2], steps[q]);  // (T as scratch; ends with a barrier)
+        in.load([&](unsigned e) { return t.p + e; });
+        // (T as scratch; ends with a barrier)
+        descent_matrices<K>(F, T, B.W, it.lx, it.ly, it.lz, (int)t.steps);
         in.store(T);
         __syncthreads();
         line_pass<N, K, N>(T, F, N, 0, N, N);
@@ -404,37 +406,48 @@ __global__ void __launch_bounds__(256) k_add(const MulItem *items, const MulJobD
         __syncthreads();
         for (int e = threadIdx.x; e < K3; e += 256) {
             const int x = e % K, y = (e / K) % K, z = e / (K * K);
-            const double v = cf[q] * T[(z * N + y) * P + x];
+            const double v = t.coef * T[(z * N + y) * P + x];
             sc[e] = any ? sc[e] + v : v;
         }
         any = true;
         __syncthreads();
     }
+    NodeRegs<K> acc;
+#pragma unroll
+    for (int w = 0; w < PER; w++) {
+        const int e = threadIdx.x + 256 * w;
+        acc.v[w] = any && e < K3 ? sc[e] : 0.0;
+    }
+    for (int q = 0; q < it.nsrc;) {
+        // the next two terms given at the node itself
+        while (q < it.nsrc && src[q].steps) q++;
+        if (q == it.nsrc) break;
+        const SumSrc ta = src[q++];
+        while (q < it.nsrc && src[q].steps) q++;
+        const bool two = q < it.nsrc;
+        const SumSrc tb = two ? src[q++] : ta;
+        NodeRegs<K> va, vb;
+        va.load([&](unsigned e) { return ta.p + e; });
+        if (two) vb.load([&](unsigned e) { return tb.p + e; });
+#pragma unroll
+        for (int w = 0; w < PER; w++) {
+            acc.v[w] += ta.coef * va.v[w];
+            if (two) acc.v[w] += tb.coef * vb.v[w];
+        }
+    }
     double ss[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double *dst = J.out + (size_t)it.node * 8 * K3;
-    constexpr int PER = NodeRegs<K>::PER;
-    NodeRegs<K> va, vb;
-    if (steps[0] == 0) va.load([&](unsigned e) { return src[0] + e; });
-    if (steps[1] == 0) vb.load([&](unsigned e) { return src[1] + e; });
 #pragma unroll
     for (int w = 0; w < PER; w++) {
         const int e = threadIdx.x + 256 * w;
         if (8 * K3 % 256 != 0 && e >= 8 * K3) break;
         const int c = e / K3;
-        double v;
-        if (!any) {
-            v = cf[0] * va.v[w] + cf[1] * vb.v[w];
-        } else {
-            v = e < K3 ? sc[e] : 0.0;
-            if (steps[0] == 0) v += cf[0] * va.v[w];
-            if (steps[1] == 0) v += cf[1] * vb.v[w];
-        }
-        dst[e] = v;
+        const double v = acc.v[w];
+        it.out[e] = v;
 #pragma unroll
         for (int q = 0; q < 8; q++)
             if (256 * w / K3 <= q && q <= (256 * w + 255) / K3) ss[q] += c == q ? v * v : 0.0;
     }
-    put_norms(ss, wsum, J.norm + (size_t)it.node * 8, compact + (size_t)blockIdx.x * 8);
+    put_norms(ss, wsum, it.norm, compact + (size_t)blockIdx.x * 8);
 }
 
 // ----------------------------------------------------------------- hydrogen functions
@@ -586,14 +599,14 @@ hipError_t launch_multiply(hipStream_t s, int n, const MulItem *items, const Mul
     return hipGetLastError();
 }
 
-hipError_t launch_add(hipStream_t s, int n, const MulItem *items, const MulJobDev *jobs, const DevBasis &B,
+hipError_t launch_sum(hipStream_t s, int n, const SumItem *items, const SumSrc *srcs, const DevBasis &B,
                       double *compact) {
     if (n <= 0) return hipSuccess;
     MWG_DISPATCH_K(B.K, {
         const size_t sm = tensor_bytes<KK>(6 * KK * KK + KK * KK * KK);
-        hipError_t e = allow_smem(k_add<KK>, sm);
+        hipError_t e = allow_smem(k_sum<KK>, sm);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_add<KK>, dim3(n), dim3(256), sm, s, items, jobs, B, compact);
+        hipLaunchKernelGGL(k_sum<KK>, dim3(n), dim3(256), sm, s, items, srcs, B, compact);
     });
     return hipGetLastError();
 }

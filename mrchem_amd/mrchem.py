@@ -83,23 +83,31 @@ class HelmholtzVector:
         else:
             if Psi is not None and len(Psi) != len(Phi):
                 raise M.MwgError("OrbitalVector size mismatch")
-            rhs = []
-            for i, p in enumerate(Phi):
-                vphi = M.multiply(self.prec, M.FunctionTree(self.mra), 1.0, V, p.tree)
-                if Psi is not None:
-                    vphi = M.add(M.FunctionTree(self.mra), 1.0, vphi, 1.0, Psi[i].tree)
-                vphi.rescale(-1.0 / (2.0 * math.pi))
-                rhs.append(vphi)
-            outs = self.apply(rhs)
+            vphi = M.multiply_batch(self.prec, [M.FunctionTree(self.mra) for _ in Phi], 1.0, [V] * len(Phi),
+                                    [p.tree for p in Phi])
+            c = -1.0 / (2.0 * math.pi)
+            if Psi is None:
+                for v in vphi:
+                    v.rescale(c)
+            else:
+                vphi = M.add_batch([M.FunctionTree(self.mra) for _ in Phi],
+                                   [[(c, v), (c, q.tree)] for v, q in zip(vphi, Psi)])
+            outs = self.apply(vphi)
         return [Orbital(o, p.occ, p.spin) for o, p in zip(outs, Phi)]
+
+
+DENSITY_BATCH = 32  # squares held at once
 
 
 def density(prec: float, Phi, mra) -> M.FunctionTree:
     """rho = sum_i occ_i phi_i^2 (src/qmfunctions/density_utils.cpp:65-133)."""
     rho = None
-    for p in Phi:
-        sq = M.multiply(prec, M.FunctionTree(mra), p.occ, p.tree, p.tree)
-        rho = sq if rho is None else M.add(M.FunctionTree(mra), 1.0, rho, 1.0, sq)
+    for i in range(0, len(Phi), DENSITY_BATCH):
+        part = Phi[i:i + DENSITY_BATCH]
+        sq = M.multiply_batch(prec, [M.FunctionTree(mra) for _ in part], [p.occ for p in part],
+                              [p.tree for p in part], [p.tree for p in part])
+        terms = sq if rho is None else [rho] + sq
+        rho = terms[0] if len(terms) == 1 else M.add_batch([M.FunctionTree(mra)], [[(1.0, t) for t in terms]])[0]
     return rho
 
 
@@ -199,15 +207,7 @@ class ExchangePotential:
         rho = pair_densities if pair_densities is not None else self.pair_densities(pairs)
         outs = [M.FunctionTree(self.mra) for _ in pairs]
         self.stats = M.apply_batch([p for _, _, p in pairs], outs, [self.poisson] * len(pairs), rho, flags=flags)
-        ex = [None] * len(Phi)
-
-        def acc(k, f, t):
-            if ex[k] is None:
-                if f != 1.0:
-                    t.rescale(f)
-                ex[k] = t
-            else:
-                ex[k] = M.add(M.FunctionTree(self.mra), 1.0, ex[k], f, t)
+        terms = [[] for _ in Phi]
 
         # the products V_ij phi_j (and V_ij phi_i) of all pairs in one batched multiply, then
         # summed into the exchange functions in pair order
@@ -225,7 +225,7 @@ class ExchangePotential:
                 t = prods[n]
                 n += 1
                 self.part_norms[i, i] = math.sqrt(t.getSquareNorm())
-                acc(i, 1.0, t)
+                terms[i].append((1.0, t))
             else:
                 fi = spin_factor(Phi[i], Phi[j])
                 fj = spin_factor(Phi[j], Phi[i])
@@ -233,8 +233,17 @@ class ExchangePotential:
                 n += 2
                 self.part_norms[j, i] = math.sqrt(tj.getSquareNorm())
                 self.part_norms[i, j] = math.sqrt(ti.getSquareNorm())
-                acc(i, fi, tj)
-                acc(j, fj, ti)
+                terms[i].append((fi, tj))
+                terms[j].append((fj, ti))
+        ex = [None] * len(Phi)
+        for k, t in enumerate(terms):
+            if len(t) == 1:
+                ex[k] = t[0][1]
+                if t[0][0] != 1.0:
+                    ex[k].rescale(t[0][0])
+        many = [k for k, t in enumerate(terms) if len(t) > 1]
+        for k, o in zip(many, M.add_batch([M.FunctionTree(self.mra) for _ in many], [terms[k] for k in many])):
+            ex[k] = o
         self.exchange = ex
         for i in range(len(Phi)):
             self.tot_norms[i] = math.sqrt(ex[i].getSquareNorm()) if ex[i] is not None else 0.0
@@ -249,31 +258,25 @@ class ExchangePotential:
 MACHINE_ZERO = 1e-14  # mrcpp::MachineZero
 
 
-def _lincomb(mra, terms, grid=None):
-    """sum_k c_k f_k for (c_k, tree_k) terms, exact on the union grid (pairwise adds in
-    term order); coefficients below MachineZero are skipped (qmfunction_utils.cpp:152-165)
-    and no remaining term gives the zero function on the grid of `grid`."""
-    kept = [(c, t) for c, t in terms if abs(c) > MACHINE_ZERO]
-    if not kept:
-        g = grid if grid is not None else terms[0][1]
-        return M.add(M.FunctionTree(mra), 0.0, g, 0.0, g)
-    terms = kept
-    c0, t0 = terms[0]
-    acc = M.add(M.FunctionTree(mra), c0, t0, 0.0, t0)
-    for c, t in terms[1:]:
-        acc = M.add(M.FunctionTree(mra), 1.0, acc, c, t)
-    return acc
+def _lincomb(sums, grids):
+    """sum_k c_k f_k for each list of (c_k, tree_k) terms, exact on the union grid, all in one
+    launch; coefficients below MachineZero are skipped (qmfunction_utils.cpp:152-165)
+    and no remaining term gives the zero function on the grid of the list's entry of `grids`."""
+    kept = [[(c, t) for c, t in terms if abs(c) > MACHINE_ZERO] or [(0.0, g)] for terms, g in zip(sums, grids)]
+    outs = [M.FunctionTree(g.mra) for g in grids]
+    if any(g.mra is not grids[0].mra for g in grids):
+        for o, k in zip(outs, kept):
+            M.add_batch([o], [k])
+        return outs
+    return M.add_batch(outs, kept)
 
 
 def add(a: float, Phi_a, b: float, Phi_b):
     """orbital::add: out_i = a (Phi_a)_i + b (Phi_b)_i."""
     if len(Phi_a) != len(Phi_b):
         raise M.MwgError("Size mismatch")
-    out = []
-    for pa, pb in zip(Phi_a, Phi_b):
-        mra = pa.tree.mra
-        out.append(Orbital(_lincomb(mra, [(a, pa.tree), (b, pb.tree)]), pa.occ, pa.spin))
-    return out
+    sums = [[(a, pa.tree), (b, pb.tree)] for pa, pb in zip(Phi_a, Phi_b)]
+    return [Orbital(t, pa.occ, pa.spin) for t, pa in zip(_lincomb(sums, [pa.tree for pa in Phi_a]), Phi_a)]
 
 
 def rotate(U, Phi):
@@ -281,11 +284,9 @@ def rotate(U, Phi):
     U = np.asarray(U, float)
     if U.shape != (len(Phi), len(Phi)):
         raise M.MwgError("rotation matrix size mismatch")
-    out = []
-    for i, p in enumerate(Phi):
-        out.append(Orbital(_lincomb(p.tree.mra, [(U[i, j], Phi[j].tree) for j in range(len(Phi))], p.tree),
-                           p.occ, p.spin))
-    return out
+    sums = [[(U[i, j], Phi[j].tree) for j in range(len(Phi))] for i in range(len(Phi))]
+    trees = _lincomb(sums, [p.tree for p in Phi])
+    return [Orbital(t, p.occ, p.spin) for t, p in zip(trees, Phi)]
 
 
 def get_norms(Phi) -> np.ndarray:

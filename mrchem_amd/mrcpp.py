@@ -298,6 +298,21 @@ def add(out: FunctionTree, ca: float, a: FunctionTree, cb: float, b: FunctionTre
     return out
 
 
+def add_batch(outs, sums) -> list:
+    """outs[i] = sum of c f over sums[i] = [(c, f), ...], each on the union grid of its terms:
+    the linear combinations of a whole orbital vector in one launch."""
+    if len(sums) != len(outs) or any(len(t) == 0 for t in sums):
+        raise MwgError("add_batch: length mismatch")
+    if not outs:
+        return outs
+    terms = [t for s in sums for t in s]
+    arr, n = C.c_void_p, len(outs)
+    check(lib().mwg_add_batch(n, (arr * n)(*[o.h for o in outs]), np.array([len(s) for s in sums], np.int32),
+                              np.array([c for c, _ in terms], np.float64), (arr * len(terms))(*[f.h for _, f in terms])),
+          outs[0].mra.ctx.h)
+    return outs
+
+
 def dot(a: FunctionTree, b: FunctionTree) -> float:
     v = C.c_double()
     check(lib().mwg_tree_dot(a.h, b.h, C.byref(v)), a.mra.ctx.h)

@@ -55,3 +55,31 @@ def test_inputs_of_different_depths(G, oracle, k, basis):
     G.apply(prec, out, G.PoissonOperator(mra, prec), a)
     oracle.apply(prec, oout, oracle.Oper(omra, 0.0, prec), oa)
     _same(out, oout)
+
+
+@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8, 9])
+def test_linear_combinations_equal_chains_of_sums(G, k):
+    """One launch for several combinations of one to five terms, some above the node and some at
+    it, against pairwise sums: the same grid, and coefficients that differ by the order of at most
+    five additions and by where a term is refined (1e-13 of the largest)."""
+    mra = G.mra_from(configs.BOX20, k)
+    orbs, _, _ = configs.orbitals(4, n_orb=5)
+    f = [G.project(p, G.FunctionTree(mra), o) for p, o in zip((0.3, 1e-4, 1e-2, 1e-5, 1e-1), orbs)]
+    c = [0.7, -1.3, 2.0, 1e-3, -0.5]
+    sums = [list(zip(c[:m], f[s:s + m])) for m, s in ((1, 1), (2, 0), (3, 2), (5, 0), (2, 3))]
+    outs = G.add_batch([G.FunctionTree(mra) for _ in sums], sums)
+    for o, terms in zip(outs, sums):
+        ref = G.add(G.FunctionTree(mra), terms[0][0], terms[0][1], 0.0, terms[0][1])
+        for cc, t in terms[1:]:
+            ref = G.add(G.FunctionTree(mra), 1.0, ref, cc, t)
+        (d0, l0, c0), (d1, l1, c1) = o.export(), ref.export()
+        key0, key1 = np.lexsort((*l0.reshape(-1, 3).T, d0)), np.lexsort((*l1.reshape(-1, 3).T, d1))
+        assert np.array_equal(d0[key0], d1[key1])
+        assert np.array_equal(l0.reshape(-1, 3)[key0], l1.reshape(-1, 3)[key1])
+        a, b = c0.reshape(len(d0), -1)[key0], c1.reshape(len(d1), -1)[key1]
+        assert np.abs(a - b).max() <= 1e-13 * np.abs(b).max()
+        assert abs(o.getSquareNorm() - ref.getSquareNorm()) <= 1e-12 * ref.getSquareNorm()
+    with pytest.raises(G.MwgError):
+        G.add_batch([f[0]], [[(1.0, f[0]), (1.0, f[1])]])
+    with pytest.raises(G.MwgError):
+        G.add_batch([outs[0], outs[0]], [[(1.0, f[0])], [(1.0, f[1])]])
