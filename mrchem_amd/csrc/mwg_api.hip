@@ -251,6 +251,7 @@ struct Ctx {
     int gen_shift = 0;
     int hw_chunk[LOOP_MAX_DEPTH] = {}, hw_schunk[LOOP_MAX_DEPTH] = {};  // per refinement iteration
     double hw_ratio = 0.0;
+    double mul_growth = 1.0;  // nodes of the last products over those of their union grids, and a tenth
     std::vector<int> last_in, last_out;  // input and output node counts of the last batch, per job
     DBuf<WorkItem> lwork[2];
     DBuf<int> lcidx, ltopo, lroots;
@@ -284,6 +285,10 @@ struct Ctx {
     DBuf<unsigned long long> genHashKeys;
     DBuf<int> genHashVals;
     DBuf<TransformItem> titems;
+    DBuf<HashItem> hitems;  // node tables to build, and their nodes' keys
+    DBuf<unsigned long long> hkeys;
+    DBuf<GatherItem> gitems;
+    DBuf<unsigned long long> dotpairs;
     DBuf<MulItem> mitems;  // products and projections: items of all jobs, and the jobs
     DBuf<MulJobDev> mjobs;
     DBuf<SumItem> sitems;  // linear combinations: output nodes and their terms
@@ -362,8 +367,7 @@ struct MraH {
     ProjGeom geom() const { return ProjGeom{{lo(0), lo(1), lo(2)}, sfac, n0}; }
 };
 
-// open-addressing node index (slot key = node key + 1, 0 = empty; load at most 1/2):
-// the layout of the device tables, so that build_hash uploads it as it is
+// open-addressing node index (slot key = node key + 1, 0 = empty; load at most 1/2)
 struct NodeIndex {
     std::vector<unsigned long long> keys;
     std::vector<int> vals;
@@ -412,13 +416,13 @@ struct NodeIndex {
 struct TreeH {
     MraH *mra = nullptr;
     std::vector<int> depth, parent, child, lr;  // lr: 3 per node
-    NodeIndex index;
     std::vector<int> roots;
     std::vector<double> cnorm;  // 8 per node (host copy)
     double sqnorm = 0.0;
     DBuf<double> coef, norm;
-    DBuf<unsigned long long> hkeys;
-    DBuf<int> hvals;
+    // device table of the nodes (DHash), one block of the context's cache: the slots' keys, then
+    // their values; made when the tree is an apply's input
+    DBuf<char> hash;
     uint32_t hmask = 0;
     bool hvalid = false;
     // split-FP16 copy of the coefficients for the mixed-precision apply, made when the tree
@@ -435,7 +439,6 @@ struct TreeH {
         parent.clear();
         child.clear();
         lr.clear();
-        index.clear();
         roots.clear();
         cnorm.clear();
         sqnorm = 0.0;
@@ -450,7 +453,6 @@ struct TreeH {
         lr.push_back(y);
         lr.push_back(z);
         cnorm.resize(8 * (size_t)(id + 1), 0.0);
-        index.put(node_key(d, x, y, z), id);
         hvalid = false;
         return id;
     }
@@ -461,9 +463,6 @@ struct TreeH {
         child.reserve(m);
         lr.reserve(3 * m);
         cnorm.reserve(8 * m);
-        size_t cap = 1024;
-        while (cap < 2 * m + 2) cap <<= 1;
-        if (index.keys.size() < cap) index.rehash(cap);
     }
     void make_roots() {
         clear();
@@ -477,8 +476,9 @@ struct TreeH {
         for (int a = 0; a < 8; a++) add(d + 1, 2 * x + (a & 1), 2 * y + ((a >> 1) & 1), 2 * z + ((a >> 2) & 1), i);
         child[i] = first;
     }
-    int find(int d, int x, int y, int z) const {
-        return index.get(node_key(d, x, y, z));
+    // the root at (x, y, z) (the roots come first, x fastest), -1 in an empty tree
+    int root_at(int x, int y, int z) const {
+        return roots.empty() ? -1 : (z * mra->boxes[1] + y) * mra->boxes[0] + x;
     }
     // the topology of m nodes built elsewhere (the device refinement loop), the roots first
     void set_topology(int m, const int *dep, const int *par, const int *chi, const int *l3) {
@@ -491,7 +491,6 @@ struct TreeH {
         child.assign(chi, chi + m);
         lr.assign(l3, l3 + 3 * (size_t)m);
         cnorm.assign(8 * (size_t)m, 0.0);
-        for (int i = 0; i < m; i++) index.put(node_key(depth[i], lr[3 * i], lr[3 * i + 1], lr[3 * i + 2]), i);
     }
     // grow the coefficient and norm arrays through the context's block cache (the old
     // contents are copied on the stream; no synchronisation).  Growth is by half again, and
@@ -533,15 +532,23 @@ struct TreeH {
         const size_t cb = coef.n * sizeof(double), nb = norm.n * sizeof(double);
         C.cache.put(coef.release(), cb);
         C.cache.put(norm.release(), nb);
+        drop_hash();
     }
-    void build_hash() {
-        if (hvalid) return;
-        if (index.keys.empty()) index.rehash(1024);
-        hipStream_t s = mra->ctx->stream;
-        hkeys.upload(index.keys.data(), index.keys.size(), s);
-        hvals.upload(index.vals.data(), index.vals.size(), s);
-        hmask = index.mask();
-        hvalid = true;
+    void drop_hash() {
+        const size_t hb = hash.n;
+        if (hash.p) mra->ctx->cache.put(hash.release(), hb);
+    }
+    // the device table's block: load at most 1/2, as dhash_find needs an empty slot
+    void alloc_hash() {
+        size_t cap = 1024, got = 0;
+        while (cap < 2 * (size_t)n() + 2) cap <<= 1;
+        const size_t need = cap * (sizeof(unsigned long long) + sizeof(int));
+        if (hash.n < need) {
+            drop_hash();
+            char *q = (char *)mra->ctx->cache.get(need, got);
+            hash.adopt(q, got);
+        }
+        hmask = (uint32_t)(cap - 1);
     }
     // the split-FP16 arrays, sized for the tree (through the block cache, where drop16
     // returns them)
@@ -575,7 +582,10 @@ struct TreeH {
         if (exp16.p) C.cache.put(exp16.release(), eb);
         ver16 = 0;
     }
-    DHash dhash() const { return DHash{hkeys.p, hvals.p, hmask}; }
+    DHash dhash() const {
+        return DHash{(unsigned long long *)hash.p, (int *)(hash.p + ((size_t)hmask + 1) * sizeof(unsigned long long)),
+                     hmask};
+    }
     void refresh_norms() {  // device norms -> host, square norm
         hipStream_t s = mra->ctx->stream;
         HC(launch_norms(s, n(), nullptr, coef.p, norm.p, K3()));
@@ -1355,7 +1365,6 @@ static void compact_tree(TreeH &T, const std::vector<char> &alive) {
     const size_t nb = (size_t)8 * T.K3();  // doubles per node
     const int nroots = (int)T.roots.size();
     int n = T.n();
-    auto key_of = [&](int i) { return node_key(T.depth[i], T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2]); };
     std::vector<int> holes;
     for (int i = nroots; i < n; i += 8)
         if (!alive[i]) holes.push_back(i);
@@ -1397,8 +1406,6 @@ static void compact_tree(TreeH &T, const std::vector<char> &alive) {
     T.child.resize(n);
     T.lr.resize(3 * (size_t)n);
     T.cnorm.resize(8 * (size_t)n);
-    T.index.clear();
-    for (int i = 0; i < n; i++) T.index.put(key_of(i), i);
     T.hvalid = false;
 }
 
@@ -1450,6 +1457,36 @@ static void for_each_job(size_t n, F f) {
         if (e) std::rethrow_exception(e);
 }
 
+// device tables of the trees that lack one, built there from the nodes' keys: one upload and two
+// launches for all of them
+static void build_hashes(Ctx &C, const std::vector<TreeH *> &trees) {
+    std::vector<TreeH *> todo;
+    for (TreeH *T : trees)
+        if (!T->hvalid && std::find(todo.begin(), todo.end(), T) == todo.end()) todo.push_back(T);
+    if (todo.empty()) return;
+    std::vector<size_t> ofs(todo.size() + 1, 0);
+    for (size_t j = 0; j < todo.size(); j++) {
+        todo[j]->alloc_hash();
+        ofs[j + 1] = ofs[j] + (size_t)todo[j]->n();
+    }
+    std::vector<unsigned long long> keys(ofs.back());
+    std::vector<HashItem> items(todo.size());
+    auto fill = [&](size_t j) {
+        const TreeH &T = *todo[j];
+        unsigned long long *k = keys.data() + ofs[j];
+        for (int i = 0; i < T.n(); i++) k[i] = node_key(T.depth[i], T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2]);
+        items[j] = HashItem{T.dhash(), (long long)ofs[j], T.n()};
+    };
+    if (ofs.back() < 65536)
+        for (size_t j = 0; j < todo.size(); j++) fill(j);
+    else
+        for_each_job(todo.size(), fill);
+    upload_async(C, C.hkeys, keys.data(), keys.size());
+    upload_async(C, C.hitems, items.data(), items.size());
+    HC(launch_hash_build(C.stream, (int)items.size(), C.hitems.p, C.hkeys.p));
+    for (TreeH *T : todo) T->hvalid = true;
+}
+
 // milliseconds between two device-clock stamps of a contraction (0 when they are missing)
 static float clock_ms(const Ctx &C, unsigned long long start, unsigned long long end) {
     if (start == 0ull || end == 0ull || end < start) return 0.0f;
@@ -1499,8 +1536,12 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         if (J.in->mra != &M || J.out->mra != &M || J.op->mra != &M)
             throw Error(MWG_ERR_ARG, "all trees and operators of an apply must share one MRA");
         if (J.in->n() == 0) throw Error(MWG_ERR_STATE, "input tree is empty");
-        J.in->build_hash();
         in_nodes += J.in->n();
+    }
+    {
+        std::vector<TreeH *> ins;
+        for (JobH &J : jobs) ins.push_back(J.in);
+        build_hashes(C, ins);
     }
     std::vector<int> dmax_in(jobs.size(), 0);
     auto scan_input = [&](size_t j) {
@@ -2451,10 +2492,18 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         C.rb.reserve(total * sizeof(double));
         double *h = (double *)C.rb.h;
         size_t off = 0;
-        for (JobH &J : jobs) {
-            const size_t m = 8 * (size_t)J.out->n();
-            if (m) HC(hipMemcpyAsync(h + off, J.out->norm.p, m * sizeof(double), hipMemcpyDeviceToHost, s));
-            off += m;
+        if (jobs.size() == 1) {
+            HC(hipMemcpyAsync(h, jobs[0].out->norm.p, total * sizeof(double), hipMemcpyDeviceToHost, s));
+        } else {  // (a copy per tree costs more than the gather)
+            std::vector<GatherItem> items;
+            for (JobH &J : jobs) {
+                items.push_back(GatherItem{J.out->norm.p, (long long)off, 8 * J.out->n()});
+                off += 8 * (size_t)J.out->n();
+            }
+            upload_async(C, C.gitems, items.data(), items.size());
+            C.rbd.alloc(total * sizeof(double));
+            HC(launch_gather(s, (int)items.size(), C.gitems.p, (double *)C.rbd.p));
+            HC(hipMemcpyAsync(h, C.rbd.p, total * sizeof(double), hipMemcpyDeviceToHost, s));
         }
         stream_wait(C);
         C.stage.off = 0;
@@ -2534,8 +2583,8 @@ struct MulJob {
         out->make_roots();
         src.clear();
         for (int r : out->roots) {
-            const int ia = a->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
-            const int ib = b->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+            const int ia = a->root_at(out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+            const int ib = b->root_at(out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
             if (ia < 0 || ib < 0) throw Error(MWG_ERR_STATE, "input tree does not cover the box");
             src.push_back(Src{ia, 0, ib, 0});
         }
@@ -2600,6 +2649,13 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
         nodes += J.a->n() + J.b->n();
     }
     for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(M.maxDepth); });
+    // room for the refinement that the last batch needed beyond the union grids (a tree that
+    // grows level by level is allocated and copied at each)
+    double n_union = 0.0, n_out = 0.0;
+    for (MulJob &J : jobs) {
+        n_union += J.out->n();
+        J.out->ensure_dev((size_t)(J.out->n() * std::min(2.0, C.mul_growth)));
+    }
     std::vector<size_t> ofs;
     while (const double *h = run_items(C, jobs, ofs, [&](int n, const MulItem *items, const MulJobDev *jd, double *cn) {
                HC(launch_multiply(C.stream, n, items, jd, M.geom(), M.dev(), cn));
@@ -2634,7 +2690,11 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
         });
     }
     std::vector<TreeH *> trees;
-    for (MulJob &J : jobs) trees.push_back(J.out);
+    for (MulJob &J : jobs) {
+        trees.push_back(J.out);
+        n_out += J.out->n();
+    }
+    C.mul_growth = 1.1 * n_out / n_union;
     compress_trees(C, M, trees);
 }
 
@@ -2660,7 +2720,7 @@ struct SumJob {
         src.reserve(most * m);
         for (int r : out->roots)
             for (TreeH *t : f) {
-                const int i = t->find(0, out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
+                const int i = t->root_at(out->lr[3 * r], out->lr[3 * r + 1], out->lr[3 * r + 2]);
                 if (i < 0) throw Error(MWG_ERR_STATE, "input tree does not cover the box");
                 src.push_back(Src{i, 0});
             }
@@ -2771,6 +2831,27 @@ static int guarded(Ctx *ctx, F f) {
         (ctx ? ctx->err : g_err) = e.what();
         return MWG_ERR_STATE;
     }
+}
+
+// f(node of A, node of B, 1 but for roots) for the nodes that both trees hold
+template <class F>
+static void common_below(const TreeH &A, const TreeH &B, int ia, int ib, F &f) {
+    const int ca = A.child[ia], cb = B.child[ib];
+    if (ca < 0 || cb < 0) return;
+    for (int c = 0; c < 8; c++) {
+        f(ca + c, cb + c, 1);
+        common_below(A, B, ca + c, cb + c, f);
+    }
+}
+template <class F>
+static void common_nodes(const TreeH &A, const TreeH &B, F f) {
+    for (size_t r = 0; r < A.roots.size(); r++) {
+        f(A.roots[r], B.roots[r], 0);
+        common_below(A, B, A.roots[r], B.roots[r], f);
+    }
+}
+static unsigned long long dot_pair(int ia, int ib, int skip0) {
+    return (unsigned long long)(unsigned)ia | ((unsigned long long)skip0 << 31) | ((unsigned long long)(unsigned)ib << 32);
 }
 
 extern "C" {
@@ -2955,10 +3036,13 @@ int mwg_tree_import(mwg_tree tree, int64_t n, const int *depth, const int64_t *l
         const MraH &M = *T.mra;
         const std::string bad = check_tree_layout(M.boxes, M.maxDepth, n, depth, lr);
         if (!bad.empty()) throw Error(MWG_ERR_ARG, "tree import: " + bad);
+        T.reserve_host((size_t)n);
+        NodeIndex index;
         for (int64_t i = 0; i < n; i++) {
             const int d = depth[i], x = (int)lr[3 * i], y = (int)lr[3 * i + 1], z = (int)lr[3 * i + 2];
-            const int par = d > 0 ? T.find(d - 1, x >> 1, y >> 1, z >> 1) : -1;
+            const int par = d > 0 ? index.get(node_key(d - 1, x >> 1, y >> 1, z >> 1)) : -1;
             const int id = T.add(d, x, y, z, par);
+            index.put(node_key(d, x, y, z), id);
             if (par < 0) T.roots.push_back(id);
             else if (((x & 1) | (y & 1) | (z & 1)) == 0) T.child[par] = id;
         }
@@ -3162,32 +3246,14 @@ int mwg_tree_dot(mwg_tree a, mwg_tree b, double *out) {
             *out = 0.0;
             return;
         }
-        std::vector<int> ia, ib, c0;
-        for (size_t r = 0; r < a->roots.size(); r++) {
-            ia.push_back(a->roots[r]);
-            ib.push_back(b->roots[r]);
-            c0.push_back(0);
-        }
-        for (int i = 0; i < a->n(); i++) {
-            if (a->depth[i] == 0) continue;
-            const int j = b->find(a->depth[i], a->lr[3 * i], a->lr[3 * i + 1], a->lr[3 * i + 2]);
-            if (j < 0) continue;
-            ia.push_back(i);
-            ib.push_back(j);
-            c0.push_back(1);
-        }
-        hipStream_t s = C->stream;
-        DBuf<int> dia, dib, dc0;
-        DBuf<double> part;
-        dia.upload(ia.data(), ia.size(), s);
-        dib.upload(ib.data(), ib.size(), s);
-        dc0.upload(c0.data(), c0.size(), s);
-        part.alloc(ia.size());
-        HC(launch_dot(s, (int)ia.size(), dia.p, dib.p, dc0.p, a->coef.p, b->coef.p, a->K3(), part.p));
-        std::vector<double> hp(ia.size());
-        part.download(hp.data(), hp.size(), s);
+        std::vector<unsigned long long> pairs;
+        common_nodes(*a, *b, [&](int ia, int ib, int skip0) { pairs.push_back(dot_pair(ia, ib, skip0)); });
+        upload_async(*C, C->dotpairs, pairs.data(), pairs.size());
+        C->rbd.alloc(pairs.size() * sizeof(double));
+        HC(launch_dot(C->stream, (int)pairs.size(), C->dotpairs.p, a->coef.p, b->coef.p, a->K3(), (double *)C->rbd.p));
+        const double *hp = read_compact(*C, pairs.size());
         double sum = 0.0;
-        for (double v : hp) sum += v;
+        for (size_t i = 0; i < pairs.size(); i++) sum += hp[i];
         *out = sum;
     });
 }
@@ -3209,12 +3275,8 @@ int mwg_tree_dot_noalloc(mwg_tree a, mwg_tree b, double *out) {
             *out = 0.0;
             return;
         }
-        auto match = [&](int i) {
-            return B.find(A.depth[i], A.lr[3 * i], A.lr[3 * i + 1], A.lr[3 * i + 2]);
-        };
-        int64_t np = (int64_t)A.roots.size();
-        for (int i = 0; i < A.n(); i++)
-            if (A.depth[i] > 0 && match(i) >= 0) np++;
+        int64_t np = 0;
+        common_nodes(A, B, [&](int, int, int) { np++; });
         if (np > DOT_NOALLOC_MAX_PAIRS)
             throw Error(MWG_ERR_RANGE, "mwg_tree_dot_noalloc: " + std::to_string(np) +
                                            " node pairs exceed the scratch limit of " +
@@ -3232,17 +3294,10 @@ int mwg_tree_dot_noalloc(mwg_tree a, mwg_tree b, double *out) {
             off += nb;
             nb = 0;
         };
-        auto put = [&](int ia, int ib, int skip0) {
-            buf[nb++] = (unsigned long long)(unsigned)ia | ((unsigned long long)skip0 << 31) |
-                        ((unsigned long long)(unsigned)ib << 32);
+        common_nodes(A, B, [&](int ia, int ib, int skip0) {
+            buf[nb++] = dot_pair(ia, ib, skip0);
             if (nb == STAGE) flush();
-        };
-        for (size_t r = 0; r < A.roots.size(); r++) put(A.roots[r], B.roots[r], 0);
-        for (int i = 0; i < A.n(); i++) {
-            if (A.depth[i] == 0) continue;
-            const int j = match(i);
-            if (j >= 0) put(i, j, 1);
-        }
+        });
         flush();
         HC(launch_dot_pairs(s, (int)np, pairs, A.coef.p, B.coef.p, A.K3(), DOT_NOALLOC_BLOCKS, part, res));
         double h = 0.0;
@@ -3277,7 +3332,7 @@ int mwg_tree_eval(mwg_tree tree, int64_t n, const double *xyz, double *out) {
                 out[pi] = 0.0;
                 continue;
             }
-            int node = T.find(0, (int)u0[0], (int)u0[1], (int)u0[2]);
+            int node = T.root_at((int)u0[0], (int)u0[1], (int)u0[2]);
             int depth = 0;
             while (node >= 0 && T.child[node] >= 0) {
                 depth++;

@@ -158,8 +158,8 @@ hipError_t launch_nsblocks(hipStream_t s, int n, const long long *item_delta, co
                            const int *item_tlo, const int *item_thi, const double *t1, const double *W, int K,
                            double *blocks, double *norms, double *norms2 = nullptr);
 hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3);
-hipError_t launch_dot(hipStream_t s, int n, const int *ia, const int *ib, const int *c0, const double *A,
-                      const double *B, int K3, double *part);
+hipError_t launch_dot(hipStream_t s, int n, const unsigned long long *pairs, const double *A, const double *B, int K3,
+                      double *part);
 // sum over node pairs of a . b (part: nblocks doubles of block sums, res: the total)
 hipError_t launch_dot_pairs(hipStream_t s, int n, const unsigned long long *pairs, const double *A,
                             const double *B, int K3, int nblocks, double *part, double *res);
@@ -259,6 +259,20 @@ hipError_t launch_contract_mfma(hipStream_t s, int K, int ntask, const TaskSumma
                                 const SliceTask *tasks, const WorkItem *work, const JobTab *jobs,
                                 const TermTab *tabs, const Slice *slices, const double *genPool, double *nodeslots,
                                 long long *tabcnt, const uint4 *genPool16, const int *genExp16);
+// a tree's node table and where its nodes' keys lie
+struct HashItem {
+    DHash h;
+    long long first;
+    int n;
+};
+hipError_t launch_hash_build(hipStream_t s, int n, const HashItem *items, const unsigned long long *keys);
+// n doubles from p to dst + first
+struct GatherItem {
+    const double *p;
+    long long first;
+    int n;
+};
+hipError_t launch_gather(hipStream_t s, int n, const GatherItem *items, double *dst);
 // an output node of a product, sum or projection, with the inputs that represent it
 struct MulItem {
     int node;

@@ -249,17 +249,52 @@ __global__ void __launch_bounds__(256) k_norms(int n, const int *nodes, const do
     }
 }
 
-// per-pair partial dot products: sum over components [c0, 8)
-__global__ void k_dot(int n, const int *ia, const int *ib, const int *c0, const double *A, const double *B, int K3,
-                      double *part) {
-    const int i = blockIdx.x;
-    if (i >= n) return;
-    const double *a = A + (size_t)ia[i] * 8 * K3;
-    const double *b = B + (size_t)ib[i] * 8 * K3;
+// Node tables of trees that become an apply's inputs, HASH_BLOCKS workgroups a tree: cleared, then
+// every node takes the first free slot from its hash on (the load is at most 1/2).  Built on
+// the host and uploaded, a table was 24 to 48 bytes a node and two blocking copies a tree: the
+// inputs of a batch of 36 pair potentials took 1.5 ms before the first launch, 0.35 now.
+constexpr int HASH_BLOCKS = 8;
+
+__global__ void __launch_bounds__(256) k_hash_clear(const HashItem *items) {
+    const DHash h = items[blockIdx.x / HASH_BLOCKS].h;
+    for (uint32_t i = (blockIdx.x % HASH_BLOCKS) * 256 + threadIdx.x; i <= h.mask; i += 256 * HASH_BLOCKS) h.keys[i] = 0ull;
+}
+
+__global__ void __launch_bounds__(256) k_hash_insert(const HashItem *items, const unsigned long long *keys) {
+    const HashItem it = items[blockIdx.x / HASH_BLOCKS];
+    for (int i = (blockIdx.x % HASH_BLOCKS) * 256 + threadIdx.x; i < it.n; i += 256 * HASH_BLOCKS) {
+        const unsigned long long key = keys[it.first + i], kk = key + 1ull;
+        uint32_t q = dkey_hash(key) & it.h.mask;
+        for (uint32_t probe = 0; probe <= it.h.mask; probe++) {
+            if (atomicCAS(&it.h.keys[q], 0ull, kk) == 0ull) {
+                it.h.vals[q] = i;
+                break;
+            }
+            q = (q + 1) & it.h.mask;
+        }
+    }
+}
+
+// several trees' norms into one array (one transfer to the host)
+__global__ void __launch_bounds__(256) k_gather(const GatherItem *items, double *dst) {
+    const GatherItem it = items[blockIdx.x / HASH_BLOCKS];
+    for (int i = (blockIdx.x % HASH_BLOCKS) * 256 + threadIdx.x; i < it.n; i += 256 * HASH_BLOCKS)
+        dst[it.first + i] = it.p[i];
+}
+
+// per-pair partial dot products (pair words as for k_dot_pairs), one workgroup per pair
+__global__ void __launch_bounds__(256) k_dot(const unsigned long long *pairs, const double *A, const double *B, int K3,
+                                             double *part) {
+    __shared__ double wsum[4];
+    const unsigned long long p = pairs[blockIdx.x];
+    const int c0 = (int)((p >> 31) & 1u);
+    const double *a = A + (size_t)(p & 0x7fffffffu) * 8 * K3;
+    const double *b = B + (size_t)(p >> 32) * 8 * K3;
     double s = 0.0;
-    for (int e = c0[i] * K3 + threadIdx.x; e < 8 * K3; e += 64) s += a[e] * b[e];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if (threadIdx.x == 0) part[i] = s;
+#pragma unroll 8
+    for (int e = c0 * K3 + threadIdx.x; e < 8 * K3; e += 256) s += a[e] * b[e];
+    s = block_sum_256(s, wsum);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // node-pair dot products over a fixed grid, one wave per pair (a pair word holds the a node
@@ -1679,10 +1714,23 @@ hipError_t launch_dot_pairs(hipStream_t s, int n, const unsigned long long *pair
     return hipGetLastError();
 }
 
-hipError_t launch_dot(hipStream_t s, int n, const int *ia, const int *ib, const int *c0, const double *A,
-                      const double *B, int K3, double *part) {
+hipError_t launch_dot(hipStream_t s, int n, const unsigned long long *pairs, const double *A, const double *B, int K3,
+                      double *part) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dot, dim3(n), dim3(64), 0, s, n, ia, ib, c0, A, B, K3, part);
+    hipLaunchKernelGGL(k_dot, dim3(n), dim3(256), 0, s, pairs, A, B, K3, part);
+    return hipGetLastError();
+}
+
+hipError_t launch_hash_build(hipStream_t s, int n, const HashItem *items, const unsigned long long *keys) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_hash_clear, dim3(n * HASH_BLOCKS), dim3(256), 0, s, items);
+    hipLaunchKernelGGL(k_hash_insert, dim3(n * HASH_BLOCKS), dim3(256), 0, s, items, keys);
+    return hipGetLastError();
+}
+
+hipError_t launch_gather(hipStream_t s, int n, const GatherItem *items, double *dst) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_gather, dim3(n * HASH_BLOCKS), dim3(256), 0, s, items, dst);
     return hipGetLastError();
 }
 
