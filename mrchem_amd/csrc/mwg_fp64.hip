@@ -377,17 +377,22 @@ k_contract_slices64(int ntask_arg, const TaskSummary *sum, const SliceTask *task
 // 16; the four blocks of an instruction get the same A rows), a workgroup one gt_x.  Passes x
 // and y exchange through the wave's own LDS rows, pass z over the workgroup.  Eight k = 9
 // Helmholtz applies at prec 1e-6 (6.6 M combinations in 1.2 M slices): contractions 14.7 ms one
-// combination at a time, 10.2 ms here (FP64 pipe busy 49 %, LDS 39 %; two waves per SIMD), 11.2 with the
-// split over rows a' above (one wave per SIMD).
+// combination at a time, 11.2 with the split over rows a' above (one wave per SIMD), 10.1 here with a
+// select per entry of A and a branch per exchanged value, 9.6 with neither: the staged rows end in
+// zeros, and what has no place goes to a row's padding.  Now the FP64 pipe is busy 46 % of the
+// time and LDS 51 %, with the two waves per SIMD that the accumulators leave room for.
 template <int K>
 struct Wide {
     static constexpr int RG = (K + 3) / 4, KS = RG;  // row groups; products per lane group
     static constexpr int WV = K == 9 ? 3 : 4, S = (K + WV - 1) / WV, T = (S * K + 15) / 16, NT = WV * 64;
-    static constexpr int K2 = K * K, K3 = K2 * K, ROW = K | 1;  // ROW: values per LDS row, odd
+    static constexpr int K2 = K * K, K3 = K2 * K, ROW = (K + 1) | 1;  // ROW: an LDS row, odd
+    // rows of the staged operator blocks: a lane group's KS entries are there for all four, zeros
+    // beyond K (a select per entry of A otherwise)
+    static constexpr int AR = 4 * KS, A2 = K * AR;
     static constexpr int U_WAVE = 4 * S * K * ROW, V_ALL = 4 * K2 * ROW;
     static constexpr int XCH = WV * U_WAVE > V_ALL ? WV * U_WAVE : V_ALL;
     // staged values of a slice: f | X | Y, Z block pairs
-    static constexpr int P = K % 2 == 0 ? 2 : 1, SLOT = K3 + 5 * K2;
+    static constexpr int P = K % 2 == 0 ? 2 : 1, SLOT = K3 + AR - K + 5 * A2, A0 = K3 + AR - K;
     static constexpr int FC = (K3 / P + NT - 1) / NT, PC = (5 * K2 / P + NT - 1) / NT;
 };
 
@@ -400,7 +405,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
     constexpr int RG = D::RG, KS = D::KS, T = D::T, S = D::S, K2 = D::K2, K3 = D::K3, NT = D::NT, ROW = D::ROW;
     constexpr int RB = 64;  // records in LDS
     __shared__ __align__(16) double stage[2][(D::SLOT + 1) & ~1];
-    __shared__ __align__(16) double xch[D::XCH];  // rows of U per wave; rows of V of the workgroup
+    __shared__ __align__(16) double xch[D::XCH + D::AR];  // rows of U per wave; rows of V of the workgroup
     __shared__ __align__(16) Slice recs[RB + 2];
     if (ts && blockIdx.x == 0) {
         if (threadIdx.x == 0) *ts = (unsigned long long)wall_clock64();
@@ -415,21 +420,25 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
     const JobTab &J = jobs[work[task.g].job];
     const gdbl *oper = (const gdbl *)J.operBlocks, *in = (const gdbl *)J.inCoef, *gen = (const gdbl *)genPool;
     double *Ul = xch + wave * D::U_WAVE, *Vl = xch;
-    const int ib = min(KS * kq, K - KS);  // entries ib + s of a row; those the group before holds are zeroed in A
-    bool ok[KS];
+    const int ib = KS * kq;  // entries ib + s of a row (beyond K: the next row's, times a zero of A)
+    int ar[RG];
 #pragma unroll
-    for (int s = 0; s < KS; s++) ok[s] = ib + s >= KS * kq;
-    bool xok[T], yok[T], zok[T];  // this lane's column of pass x (l, j), pass y (a, l), pass z (b, a) exists
-    int xb[T], xu[T], yv[T], yr[T], zc[T];
+    for (int r = 0; r < RG; r++) ar[r] = min(4 * r + r4, K - 1) * D::AR + ib;
+    bool zok[T];  // this lane's column of pass x (l, j), pass y (a, l), pass z (b, a) exists
+    // (positions: rows and columns that do not exist go to entry K of some row, which counts for nothing)
+    int xb[T], xu[RG][T], yv[RG][T], yr[T], zc[T];
 #pragma unroll
     for (int t = 0; t < T; t++) {
         const int n = t * 16 + col, nc = min(n, S * K - 1), l = nc / K, j = nc % K, a = nc / S, m = nc % S;
-        xok[t] = n < S * K && wave * S + l < K;
+        const bool xok = n < S * K && wave * S + l < K, yok = n < S * K && wave * S + m < K;
         xb[t] = (min(wave * S + l, K - 1) * K + j) * K + ib;  // f
-        xu[t] = l * ROW + j;                                 // row (a, l), entry j of U, but for a
-        yok[t] = n < S * K && wave * S + m < K;
-        yr[t] = nc * ROW + ib;                 // row nc of U
-        yv[t] = a * ROW + wave * S + m;        // row (b, a), entry l of V, but for b
+        yr[t] = nc * ROW + ib;                                // row nc of U
+#pragma unroll
+        for (int r = 0; r < RG; r++) {
+            const int q = 4 * r + kq;
+            xu[r][t] = xok && q < K ? (q * S + l) * ROW + j : col * ROW + K;            // row (a, l), entry j of U
+            yv[r][t] = yok && q < K ? (q * K + a) * ROW + wave * S + m : lane * ROW + K;  // row (b, a), entry l of V
+        }
         const int z = (wave * T + t) * 16 + col;
         zok[t] = z < K2;
         zc[t] = min(z, K2 - 1);
@@ -470,17 +479,20 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
             if (tid + c * NT < K3 / D::P) *(piece *)(st + D::P * (tid + c * NT)) = lf[c];
 #pragma unroll
         for (int c = 0; c < D::PC; c++)
-            if (tid + c * NT < 5 * K2 / D::P) *(piece *)(st + K3 + D::P * (tid + c * NT)) = lp[c];
+            if (tid + c * NT < 5 * K2 / D::P) {
+                const int e = D::P * (tid + c * NT), row = e / K;
+                *(piece *)(st + D::A0 + row * D::AR + (e - row * K)) = lp[c];
+            }
     };
-    auto load_a = [&](const double *blk, double (&a)[RG][KS], double w) {
+    auto load_a = [&](const double *blk, double (&a)[RG][KS]) {
 #pragma unroll
         for (int r = 0; r < RG; r++)
 #pragma unroll
-            for (int s = 0; s < KS; s++) {
-                const double v = blk[min(4 * r + r4, K - 1) * K + ib + s];
-                a[r][s] = ok[s] ? w * v : 0.0;
-            }
+            for (int s = 0; s < KS; s++) a[r][s] = blk[ar[r] + s];
     };
+    // zeros behind the rows of f and of the blocks; finite values wherever a row's end is read
+    for (int q = tid; q < 2 * ((D::SLOT + 1) & ~1); q += NT) (&stage[0][0])[q] = 0.0;
+    for (int q = tid; q < D::XCH + D::AR; q += NT) xch[q] = 0.0;
     load_recs(0);
     __syncthreads();
     load(0, 0);
@@ -501,7 +513,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
         const bool endz = end || u(cur.zo) != u(nxt.zo), endy = endz || u(cur.yo) != u(nxt.yo);
         if (mask) {  // pass x
             double X[RG][KS], f[T][KS], t1[RG][T];
-            load_a(st + K3, X, 1.0);
+            load_a(st + D::A0, X);
 #pragma unroll
             for (int t = 0; t < T; t++)
 #pragma unroll
@@ -536,8 +548,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
                     for (int r = 0; r < RG; r++)
 #pragma unroll
                         for (int t = 0; t < T; t++) {
-                            const int a = 4 * r + kq;
-                            if (xok[t] && a < K) Ul[(p * S * K + a * S) * ROW + xu[t]] = U[p][r][t];
+                            Ul[p * S * K * ROW + xu[r][t]] = U[p][r][t];
                             U[p][r][t] = 0.0;
                         }
                 }
@@ -545,7 +556,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
 #pragma unroll
             for (int gy = 0; gy < 2; gy++) {
                 double Y[RG][KS];
-                load_a(st + K3 + (1 + gy) * K2, Y, 1.0);
+                load_a(st + D::A0 + (1 + gy) * D::A2, Y);
 #pragma unroll
                 for (int p = gy; p < 4; p += 2)
                     if ((umask >> (2 * p)) & 1) {
@@ -575,8 +586,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
                     for (int r = 0; r < RG; r++)
 #pragma unroll
                         for (int t = 0; t < T; t++) {
-                            const int bb = 4 * r + kq;
-                            if (yok[t] && bb < K) Vl[(p * K2 + bb * K) * ROW + yv[t]] = V[p][r][t];
+                            Vl[p * K2 * ROW + yv[r][t]] = V[p][r][t];
                             V[p][r][t] = 0.0;
                         }
                 }
@@ -585,7 +595,11 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
 #pragma unroll
             for (int gz = 0; gz < 2; gz++) {
                 double Z[RG][KS];
-                load_a(st + K3 + (3 + gz) * K2, Z, w);
+                load_a(st + D::A0 + (3 + gz) * D::A2, Z);
+#pragma unroll
+                for (int r = 0; r < RG; r++)
+#pragma unroll
+                    for (int s = 0; s < KS; s++) Z[r][s] *= w;
 #pragma unroll
                 for (int p = 2 * gz; p < 2 * gz + 2; p++)
                     if ((vmask >> (2 * p)) & 1) {
