@@ -249,7 +249,7 @@ __device__ inline floatx4 mfmah(uint4 a, uint4 b) {
 struct OpsH8 {
     uint4 bx, ay, az;  // X' (B role), Y', Z' (A role) fragments of this lane
     uint4 f[4];        // f (A role) per tile (yh, zq)
-    int exz;           // exponents of this lane's X' block (gt_x) + Z' block (gt_z) + f
+    int ex0, ex1, ez0, ez1, ef;  // exponents of the X' and Z' blocks and of f
     int ey0, ey1;      // the two Y' blocks
     double w;
     int mask;
@@ -282,6 +282,10 @@ __device__ inline uint2 ld8(const uint2 *p) {
 // a wave-uniform exponent (scalar load; written by an earlier kernel, read-only here)
 __device__ inline int ld_exp(const int *p) { return *(cint *)p; }
 
+// the same per lane
+typedef const int __attribute__((address_space(1))) gint;
+__device__ inline int ld_exp1(const int *p) { return *(gint *)p; }
+
 // a lane's fragment offsets (uint4 units) inside an operator block pair and an f block: the
 // same for every slice, so that a load is a uniform base (scalar registers) plus a lane offset
 struct LaneOffs8 {
@@ -304,7 +308,6 @@ __device__ inline OpsH8 load_opsh8(const Slice &sl, const Arr16 &J, const uint4 
                                    int m, int q, const LaneOffs8 &L) {
     OpsH8 o;
     const int bxb = sl.xo / 64, byb = sl.yo / 64, bzb = sl.zo / 64;  // block indices (gt_d = 0)
-    const int rx = (m >> 3) * 2;
     o.bx = ld16(J.oper + (size_t)bxb * 16 + L.bx);
     o.ay = ld16(J.oper + (size_t)byb * 16 + L.ayz);
     o.az = ld16(J.oper + (size_t)bzb * 16 + L.ayz);
@@ -319,10 +322,10 @@ __device__ inline OpsH8 load_opsh8(const Slice &sl, const Arr16 &J, const uint4 
     }
 #pragma unroll
     for (int tl = 0; tl < 4; tl++) o.f[tl] = ld16(fb + L.f[tl]);
-    // block exponents: uniform loads, then this lane's gt_x (rx) and gt_z (q >> 1)
+    // block exponents: uniform loads (added up when the slice is contracted: not waited for here)
     const int ex0 = ld_exp(J.operExp + bxb), ex1 = ld_exp(J.operExp + bxb + 2);
     const int ez0 = ld_exp(J.operExp + bzb), ez1 = ld_exp(J.operExp + bzb + 2);
-    o.exz = (rx ? ex1 : ex0) + ((q >> 1) ? ez1 : ez0) + ef;
+    o.ex0 = ex0, o.ex1 = ex1, o.ez0 = ez0, o.ez1 = ez1, o.ef = ef;
     o.ey0 = ld_exp(J.operExp + byb);
     o.ey1 = ld_exp(J.operExp + byb + 2);
     o.w = sl.w;
@@ -412,9 +415,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
             }
             wave_sync();
             // pass z: a half (gt_y) without a surviving component is skipped (uniform mask)
-            const int mk = cur.mask;
-            const float wlo = ((mk >> (gx | (gz << 2))) & 1) ? (float)ldexp(cur.w, -(cur.exz + cur.ey0 + s1 + s2)) : 0.f;
-            const float whi = ((mk >> (gx | 2 | (gz << 2))) & 1) ? (float)ldexp(cur.w, -(cur.exz + cur.ey1 + s1 + s2)) : 0.f;
+            const int mk = cur.mask, exz = (gx ? cur.ex1 : cur.ex0) + (gz ? cur.ez1 : cur.ez0) + cur.ef;
+            const float wlo = ((mk >> (gx | (gz << 2))) & 1) ? (float)ldexp(cur.w, -(exz + cur.ey0 + s1 + s2)) : 0.f;
+            const float whi = ((mk >> (gx | 2 | (gz << 2))) & 1) ? (float)ldexp(cur.w, -(exz + cur.ey1 + s1 + s2)) : 0.f;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 if (h == 0 ? !(mk & 0x33) : !(mk & 0xCC)) continue;
@@ -571,7 +574,7 @@ __device__ inline unsigned pack_hl(float v, float sc) {
 __device__ inline void put_h10(unsigned *P, int col, int pos, float v, float sc) {
     const unsigned d = pack_hl(v, sc);
     P[col * H10_COL + pos] = d;
-    if (pos < 6) P[col * H10_COL + 10 + pos] = d;
+    P[col * H10_COL + min(10 + pos, 16)] = d;  // (16 is unused)
 }
 // the B fragment of column col for lane group kg (sel: the lane's v_perm selectors)
 __device__ inline uint4 get_h10(const unsigned *P, int col, int start, const unsigned (&sel)[4]) {
@@ -594,7 +597,7 @@ k_contract_mfma10h(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks
     constexpr int K3 = 1000;
     __shared__ __align__(16) unsigned P1[H10_P1];
     __shared__ __align__(16) unsigned P2[H10_P2];
-    __shared__ double Wl[8];
+    __shared__ double Wl[2][8];  // the weights of the 8 output components, of this slice and the next
     const int ntask = sum ? (sum->overflow ? 0 : sum->nstasks) : ntask_arg;
     if ((int)blockIdx.x >= ntask) return;
     const SliceTask task = tasks[blockIdx.x];
@@ -620,7 +623,7 @@ k_contract_mfma10h(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks
     const Slice *srec = slices + task.start;
     const int last = task.count - 1;
     int ntup = 0;
-    auto contract = [&](const OpsH10 &cur, const Slice &cs) {
+    auto contract = [&](const OpsH10 &cur, const Slice &cs, const double *W) {
         ntup += __popc((unsigned)cs.mask);
         // pass x
 #pragma unroll
@@ -637,13 +640,6 @@ k_contract_mfma10h(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks
             }
         }
         __syncthreads();
-        if (wave == 0 && lane < 8) {  // the weights of the 8 output components of this slice
-            const int gt = lane, gx = gt & 1, gy = (gt >> 1) & 1, gz = gt >> 2;
-            const int e = ld_exp(J.operExp + cs.xo / 100 + 2 * gx) + ld_exp(J.operExp + cs.yo / 100 + 2 * gy) +
-                          ld_exp(J.operExp + cs.zo / 100 + 2 * gz) +
-                          (cs.f >= 0 ? ld_exp(J.inExp + (size_t)cs.f * 8 + cs.ft) : ld_exp(genExp + (-cs.f - 1)));
-            Wl[gt] = ((cs.mask >> gt) & 1) ? ldexp(cs.w, -(e + 9)) : 0.0;
-        }
         // pass y
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -669,29 +665,57 @@ k_contract_mfma10h(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks
             const uint4 b = get_h10(P2, n, start, sel);
             const floatx4 d0 = mfmah(cur.z0, b), d1 = mfmah(cur.z1, b);
             const int gxy = (n % 20 >= 10 ? 1 : 0) | (n / 20 >= 10 ? 2 : 0);
-            const double wlo = Wl[gxy], whi = Wl[gxy + 4];
+            const double wlo = W[gxy], whi = W[gxy + 4];
+            const double w01 = kg >= 3 ? whi : wlo, w23 = kg >= 2 ? whi : wlo;  // c' = 4 kg + i >= 10
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc0[t][i] = fma((double)d0[i], 4 * kg + i >= 10 ? whi : wlo, acc0[t][i]);
+            for (int i = 0; i < 4; i++) acc0[t][i] = fma((double)d0[i], i < 2 ? w01 : w23, acc0[t][i]);
             acc1[t] = fma((double)d1[0], whi, acc1[t]);
         }
     };
     // two operand sets in turn; the next slice's operands and the record after it are
     // loaded while a slice is contracted
+    // Wave 3, which has one N-tile of pass x where the others have two, makes the weights: it reads a
+    // slice's exponents with the operands, a slice ahead, and has them in LDS before the slice
+    // before it ends.  (Read between the passes, their latency held up every wave: contractions of
+    // eight k = 9 Helmholtz applies 7.6 ms, 7.3 now.)
+    struct Exps {
+        int x, y, z, f;
+    };
+    const int gt = lane & 7;
+    auto load_exps = [&](const Slice &sl) {
+        Exps e{0, 0, 0, 0};
+        if (wave == 3) {
+            e.x = ld_exp1(J.operExp + sl.xo / 100 + 2 * (gt & 1));
+            e.y = ld_exp1(J.operExp + sl.yo / 100 + 2 * ((gt >> 1) & 1));
+            e.z = ld_exp1(J.operExp + sl.zo / 100 + 2 * (gt >> 2));
+            e.f = ld_exp1(sl.f >= 0 ? J.inExp + (size_t)sl.f * 8 + sl.ft : genExp + (-sl.f - 1));
+        }
+        return e;
+    };
+    auto put_weights = [&](const Slice &sl, const Exps &e, double *W) {
+        if (wave == 3 && lane < 8)
+            W[gt] = ((sl.mask >> gt) & 1) ? ldexp(sl.w, -(e.x + e.y + e.z + e.f + 9)) : 0.0;
+    };
     const LaneOffs10 LO = lane_offs10(wave, m, kg);
     Slice cA = slice_at(srec, 0), cB;
     OpsH10 opA = load_opsh10(cA, J, gen16, m, kg, LO), opB;
+    put_weights(cA, load_exps(cA), Wl[0]);
     Slice rnext = slice_at(srec, min(1, last));
     for (int it = 0; it < task.count;) {
         cB = rnext;
         opB = load_opsh10(cB, J, gen16, m, kg, LO);
+        const Exps eB = load_exps(cB);
         rnext = slice_at(srec, min(it + 2, last));
-        contract(opA, cA);
+        contract(opA, cA, Wl[0]);
         if (++it >= task.count) break;
+        put_weights(cB, eB, Wl[1]);
         cA = rnext;
         opA = load_opsh10(cA, J, gen16, m, kg, LO);
+        const Exps eA = load_exps(cA);
         rnext = slice_at(srec, min(it + 2, last));
-        contract(opB, cB);
+        contract(opB, cB, Wl[1]);
         ++it;
+        put_weights(cA, eA, Wl[0]);
     }
     if (threadIdx.x == 0) atomicAdd((unsigned long long *)&tabcnt[4 * wi.job + 2], (unsigned long long)ntup);
     double *dst = nodeslots + (size_t)task.slot * 8 * K3;
