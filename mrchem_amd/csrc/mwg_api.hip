@@ -266,7 +266,7 @@ struct Ctx {
     // apply scratch
     DBuf<TermTab> tabs;
     DBuf<double> tbmax;
-    DBuf<int> tpre, tpre0;
+    DBuf<int> tpre;
     // per-iteration read-back block, written by the kernels and copied to the host in
     // one transfer: schedule summary | per-table counts | work norms | child
     // probabilities | child features
@@ -1846,7 +1846,6 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
             max_terms = std::max(max_terms, J.op->nterms());
         }
         C.tpre.alloc((size_t)ntabs + njobs + 1);
-        C.tpre0.alloc((size_t)ntabs + njobs + 1);
         C.tabs.alloc((size_t)std::max(ntabs, 1));
         C.tbmax.alloc((size_t)std::max(njobs * max_terms, 1));
         const size_t o_bj = ((size_t)njobs * sizeof(JobTab) + 255) & ~(size_t)255;
@@ -1861,7 +1860,6 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
             for (int j = 0; j < njobs; j++) add_table(jobs[j], d, jt, bj, nt, mt);
             for (int q = 0; q < njobs; q++) {
                 jt[q].pre = C.tpre.p + jt[q].tab0 + q;
-                jt[q].pre0 = C.tpre0.p + jt[q].tab0 + q;
             }
             std::memcpy(dst, jt.data(), (size_t)njobs * sizeof(JobTab));
             std::memcpy(dst + o_bj, bj.data(), (size_t)njobs * sizeof(BoxJob));
@@ -1896,7 +1894,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
             const WorkItem *dw = C.lwork[cur].p;
             unsigned long long *dts = (unsigned long long *)(ctlb + offsetof(LoopCtl, ts)) + 2 * d;
             const LoopInit li{C.ljobs.p, dtab, C.lctl.p, dts, C.genCount.p};
-            HC(launch_job_boxes(s, njobs, max_terms, dbj, C.tabs.p, C.tbmax.p, djt, C.tpre.p, C.tpre0.p,
+            HC(launch_job_boxes(s, njobs, max_terms, dbj, C.tabs.p, C.tbmax.p, djt, C.tpre.p,
                                 C.genOverflow.p, li));
             GenState gs{C.genKeys.p, C.genJob.p, C.genCount.p, genCap, C.genOverflow.p, C.genPool.p, C.genNorm.p,
                         genPoolCap, dtab};
@@ -2092,10 +2090,8 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         PT.lap("opers+boxes");
         // per-table prefix arrays (ntab + 1 entries each), filled on the device
         C.tpre.alloc((size_t)ntabs + jt.size() + 1);
-        C.tpre0.alloc((size_t)ntabs + jt.size() + 1);
         for (size_t q = 0; q < jt.size(); q++) {
             jt[q].pre = C.tpre.p + jt[q].tab0 + q;
-            jt[q].pre0 = C.tpre0.p + jt[q].tab0 + q;
         }
         // the iteration's tables in one upload: work items | job tables | box requests
         const size_t o_jobs = (work.size() * sizeof(WorkItem) + 255) & ~(size_t)255;
@@ -2135,7 +2131,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         C.tabs.alloc((size_t)std::max(ntabs, 1));
         C.tbmax.alloc((size_t)std::max<size_t>(bjobs.size() * max_terms, 1));
         HC(launch_job_boxes(s, (int)bjobs.size(), max_terms, dbjobs, C.tabs.p, C.tbmax.p, djobs, C.tpre.p,
-                            C.tpre0.p, C.genOverflow.p));
+                            C.genOverflow.p));
         PT.lap("launch boxes");
         // generated input nodes: marked, then computed for the range the device counter
         // reached (read back with the work-list counts below, not before)

@@ -67,7 +67,6 @@ struct JobTab {
     double thr;
     double route;  // mixed mode: slices with a bound above this run in FP64
     const int *pre;   // [ntab + 1] candidate prefix over terms (union boxes ub), device-built
-    const int *pre0;  // [ntab + 1] same over the ft = 0 union boxes ub0
     int tab0, ntab;
     int lmax[3];
     int depth;
@@ -180,7 +179,7 @@ struct LoopInit {
 // TermTab[tab0 + t] for every (table, term): per-combination screening boxes from the
 // monotone norm envelopes, union boxes, and the table's FP64 routing bound
 hipError_t launch_job_boxes(hipStream_t s, int nbj, int max_terms, const BoxJob *bj, TermTab *tabs, double *tbmax,
-                            JobTab *jobs, int *pre, int *pre0, int *gen_overflow, const LoopInit &li = LoopInit{});
+                            JobTab *jobs, int *pre, int *gen_overflow, const LoopInit &li = LoopInit{});
 // Device work counts: the work-list kernels below take an optional nwp, the work list's
 // node count on the device (written by an earlier kernel of the stream); nw is then only
 // an upper bound for the launch, and the kernels loop over the nodes on a grid of at most

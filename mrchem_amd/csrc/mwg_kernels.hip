@@ -473,20 +473,61 @@ __device__ inline void gen_insert(const JobTab &J, const GenState &gs, int job, 
     }
 }
 
-// Walks the (term, delta) candidates of the ft = 0 boxes; the translations that some
-// term needs are first collected in an LDS bitmap over the job's union box, so that
-// each input position is probed once (candidates of different terms share them).
+__device__ inline int wave_incl_scan(int v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
+// marks one translation of an output node, if the box holds it and the input does not
+__device__ __forceinline__ void gen_mark_one(const WorkItem &wi, const JobTab &J, const GenState &gs, int dx, int dy,
+                                             int dz) {
+    const int fx = wi.l[0] - dx, fy = wi.l[1] - dy, fz = wi.l[2] - dz;
+    if (fx < 0 || fy < 0 || fz < 0 || fx >= J.lmax[0] || fy >= J.lmax[1] || fz >= J.lmax[2]) return;
+    const uint64_t key = dnode_key(J.depth, fx, fy, fz);
+    if (dhash_find(J.inHash, key) < 0) gen_insert(J, gs, wi.job, key);
+}
+
+// Walks the (term, |delta|) candidates of the ft = 0 boxes (a box is symmetric in every
+// dimension): the |delta| that some term needs are first collected in an LDS bitmap over the job's
+// union box, so that each input position is probed once.  A union box beyond the bitmap is
+// walked candidate by candidate.  One workgroup per node; its time is a chain of reads, so the fewer
+// rounds the better: over every signed delta of every term it was 9.7 us a launch for a Poisson
+// apply at k = 5 and 61 for the 36 pair potentials of an exchange step, 7.4 and 53 over |delta|.
 __device__ __forceinline__ void gen_mark_node(int item, const WorkItem *work, const JobTab *jobs,
                                               const TermTab *tabs, const GenState &gs) {
     const WorkItem wi = work[item];
     const JobTab &J = jobs[wi.job];
     __shared__ int start[257];
+    __shared__ short4 ub0[256];
     __shared__ unsigned need[FCACHE / 32];
-    for (int t = threadIdx.x; t <= J.ntab; t += blockDim.x) start[t] = J.pre0[t];
     const int ux = J.ubox[0], uy = J.ubox[1], uz = J.ubox[2];
-    const int nx = 2 * ux + 1, ny = 2 * uy + 1, nz = 2 * uz + 1;
-    const bool cached = ux >= 0 && nx * ny * nz <= FCACHE;
-    for (int q = threadIdx.x; q < FCACHE / 32; q += blockDim.x) need[q] = 0u;
+    if (ux < 0) return;  // (no term has a box)
+    const int nx = 2 * ux + 1, ny = 2 * uy + 1, nz = 2 * uz + 1, ax = ux + 1, ay = uy + 1;
+    const bool cached = nx * ny * nz <= FCACHE;
+    if (threadIdx.x < 64) {  // the terms' boxes and the prefix of their candidates
+        int carry = 0;
+        for (int base = 0; base < J.ntab; base += 64) {
+            const int t = base + (int)threadIdx.x;
+            int v = 0;
+            if (t < J.ntab) {
+                const TermTab &tb = tabs[J.tab0 + t];
+                const short4 u = make_short4(tb.ub0[0], tb.ub0[1], tb.ub0[2], 0);
+                ub0[t] = u;
+                v = u.x < 0 ? 0 : (u.x + 1) * (u.y + 1) * (u.z + 1);
+            }
+            const int incl = wave_incl_scan(v);
+            if (t < J.ntab) start[t] = carry + incl - v;
+            carry += __shfl(incl, 63, 64);
+        }
+        if (threadIdx.x == 0) start[J.ntab] = carry;
+    } else {
+        for (int q = threadIdx.x - 64; q < FCACHE / 32; q += blockDim.x - 64) need[q] = 0u;
+    }
     __syncthreads();
     const int total = start[J.ntab];
     for (int k = threadIdx.x; k < total; k += blockDim.x) {
@@ -496,30 +537,26 @@ __device__ __forceinline__ void gen_mark_node(int item, const WorkItem *work, co
             if (start[mid] <= k) lo = mid;
             else hi = mid - 1;
         }
-        const TermTab &tb = tabs[J.tab0 + lo];
-        const int c = k - start[lo];
-        const int vx = tb.ub0[0], vy = tb.ub0[1], vz = tb.ub0[2];
-        const int dx = c % (2 * vx + 1) - vx;
-        const int dy = (c / (2 * vx + 1)) % (2 * vy + 1) - vy;
-        const int dz = c / ((2 * vx + 1) * (2 * vy + 1)) - vz;
-        const int fx = wi.l[0] - dx, fy = wi.l[1] - dy, fz = wi.l[2] - dz;
-        if (fx < 0 || fy < 0 || fz < 0 || fx >= J.lmax[0] || fy >= J.lmax[1] || fz >= J.lmax[2]) continue;
-        if (!(combo_mask(tb, dx, dy, dz) & FT0_COMBOS)) continue;
+        const short4 u = ub0[lo];
+        const int c = k - start[lo], wx = u.x + 1, wy = u.y + 1;
+        const int dx = c % wx, dy = (c / wx) % wy, dz = c / (wx * wy);
+        if (!(combo_mask(tabs[J.tab0 + lo], dx, dy, dz) & FT0_COMBOS)) continue;
         if (cached) {
-            const int cell = ((dz + uz) * ny + (dy + uy)) * nx + (dx + ux);
+            const int cell = (dz * ay + dy) * ax + dx;
             atomicOr(&need[cell >> 5], 1u << (cell & 31));
             continue;
         }
-        const uint64_t key = dnode_key(J.depth, fx, fy, fz);
-        if (dhash_find(J.inHash, key) < 0) gen_insert(J, gs, wi.job, key);
+        for (int sgn = 0; sgn < 8; sgn++) {
+            if (((sgn & 1) && !dx) || ((sgn & 2) && !dy) || ((sgn & 4) && !dz)) continue;
+            gen_mark_one(wi, J, gs, (sgn & 1) ? -dx : dx, (sgn & 2) ? -dy : dy, (sgn & 4) ? -dz : dz);
+        }
     }
     if (!cached) return;
     __syncthreads();
     for (int cell = threadIdx.x; cell < nx * ny * nz; cell += blockDim.x) {
-        if (!((need[cell >> 5] >> (cell & 31)) & 1u)) continue;
         const int dx = cell % nx - ux, dy = (cell / nx) % ny - uy, dz = cell / (nx * ny) - uz;
-        const uint64_t key = dnode_key(J.depth, wi.l[0] - dx, wi.l[1] - dy, wi.l[2] - dz);
-        if (dhash_find(J.inHash, key) < 0) gen_insert(J, gs, wi.job, key);
+        const int c = (abs(dz) * ay + abs(dy)) * ax + abs(dx);
+        if ((need[c >> 5] >> (c & 31)) & 1u) gen_mark_one(wi, J, gs, dx, dy, dz);
     }
 }
 
@@ -809,20 +846,11 @@ __global__ void __launch_bounds__(64) k_job_boxes(int nbj, const BoxJob *bjs, Te
 // it run in FP64; above the roots a fixed multiple of the screening threshold, on the
 // roots (no screening) a fraction of the largest bound of the table), the union box of
 // the terms, and the prefix sums over terms of the candidate counts of the union boxes
-// ub and ub0 (the work-list and generated-node kernels split their walks by these).
-__device__ inline int wave_incl_scan(int v) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, 64);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
+// ub (the work-list kernels split their walks by these).
 
 __global__ void __launch_bounds__(64) k_job_route(int nbj, const BoxJob *bjs, const TermTab *tabs,
                                                   const double *tbmax, int max_terms, JobTab *jobs, int *pre,
-                                                  int *pre0, int *gen_overflow, LoopInit li) {
+                                                  int *gen_overflow, LoopInit li) {
     const int jb = blockIdx.x;
     if (jb >= nbj) return;
     if (jb == 0 && threadIdx.x == 0) *gen_overflow = 0;  // the iteration's generated-table flag
@@ -839,10 +867,10 @@ __global__ void __launch_bounds__(64) k_job_route(int nbj, const BoxJob *bjs, co
         }
     }
     double m = 0.0;
-    int ux = -1, uy = -1, uz = -1, carry = 0, carry0 = 0;
+    int ux = -1, uy = -1, uz = -1, carry = 0;
     for (int base = 0; base < B.nterms; base += 64) {
         const int t = base + lane;
-        int v = 0, v0 = 0;
+        int v = 0;
         if (t < B.nterms) {
             m = fmax(m, tbmax[(size_t)jb * max_terms + t]);
             const TermTab &tb = tabs[B.tab0 + t];
@@ -852,15 +880,10 @@ __global__ void __launch_bounds__(64) k_job_route(int nbj, const BoxJob *bjs, co
                 uy = max(uy, (int)tb.ub[1]);
                 uz = max(uz, (int)tb.ub[2]);
             }
-            if (tb.ub0[0] >= 0) v0 = (2 * tb.ub0[0] + 1) * (2 * tb.ub0[1] + 1) * (2 * tb.ub0[2] + 1);
         }
-        const int incl = wave_incl_scan(v), incl0 = wave_incl_scan(v0);
-        if (t < B.nterms) {
-            pre[B.pre_off + t] = carry + incl - v;
-            pre0[B.pre_off + t] = carry0 + incl0 - v0;
-        }
+        const int incl = wave_incl_scan(v);
+        if (t < B.nterms) pre[B.pre_off + t] = carry + incl - v;
         carry += __shfl(incl, 63, 64);
-        carry0 += __shfl(incl0, 63, 64);
     }
     m = wave_max_double(m);
     ux = wave_max_int(ux);
@@ -868,7 +891,6 @@ __global__ void __launch_bounds__(64) k_job_route(int nbj, const BoxJob *bjs, co
     uz = wave_max_int(uz);
     if (lane == 0) {
         pre[B.pre_off + B.nterms] = carry;
-        pre0[B.pre_off + B.nterms] = carry0;
         JobTab &J = jobs[B.jt];
         J.route = thr > 0.0 ? ROUTE_FP64 * thr : ROUTE_ROOT * m;
         J.ubox[0] = ux;
@@ -1202,8 +1224,11 @@ __device__ inline void block_excl_scan_1024_n(long long (&v)[NV], long long (*ws
 // One workgroup.  Per node the slices of its (one or two) segments over all parts, and the parts'
 // offsets inside them; from the totals the task sizes; one block scan of slices and tasks gives
 // every node its first slices and tasks.  The fill kernels write the tasks themselves.
-constexpr long long FP64_TASKS = 2048;  // FP64 tasks an iteration aims at (task size permitting)
-constexpr int FP64_TASK_MIN = 8;        // ... of at least this many slices
+// FP64 tasks an iteration aims at (task size permitting): a k = 9 Poisson apply contracts in 1.70 ms
+// with 2048, 1.94 with 4096, 1.61 with 1024 and 1.66 with 512; smaller orders within 2 % of each
+// other.  Of at least FP64_TASK_MIN slices: 2 to 8 are equal (the slots cost what the waves gain).
+constexpr long long FP64_TASKS = 1024;
+constexpr int FP64_TASK_MIN = 8;
 
 __global__ void __launch_bounds__(1024)
     k_build_tasks(int nw, const int *nwp, int nseg, int nparts, int chunk, int wchunk, const int *__restrict__ tot,
@@ -1750,10 +1775,10 @@ hipError_t launch_project_gauss(hipStream_t s, int nw, const MulItem *items, con
 }
 
 hipError_t launch_job_boxes(hipStream_t s, int nbj, int max_terms, const BoxJob *bj, TermTab *tabs, double *tbmax,
-                            JobTab *jobs, int *pre, int *pre0, int *gen_overflow, const LoopInit &li) {
+                            JobTab *jobs, int *pre, int *gen_overflow, const LoopInit &li) {
     if (nbj <= 0 || max_terms <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_job_boxes, dim3(nbj, max_terms), dim3(64), 0, s, nbj, bj, tabs, tbmax, max_terms, li);
-    hipLaunchKernelGGL(k_job_route, dim3(nbj), dim3(64), 0, s, nbj, bj, tabs, tbmax, max_terms, jobs, pre, pre0,
+    hipLaunchKernelGGL(k_job_route, dim3(nbj), dim3(64), 0, s, nbj, bj, tabs, tbmax, max_terms, jobs, pre,
                        gen_overflow, li);
     return hipGetLastError();
 }
