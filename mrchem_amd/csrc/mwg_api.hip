@@ -2605,7 +2605,7 @@ struct MulJob {
 // f(j) for the jobs, on host threads where the work (nodes) is worth their start
 template <class F>
 static void for_jobs_of(size_t njobs, size_t nodes, F f) {
-    if (nodes < 4096)
+    if (nodes < 65536)  // (starting threads takes up to 5 ms where their stacks and heaps are new)
         for (size_t j = 0; j < njobs; j++) f(j);
     else
         for_each_job(njobs, f);
