@@ -2,11 +2,11 @@
 //
 // mrcpp::apply(prec, out, oper, inp) is restated as an adaptive build whose
 // every numerical step runs on the GPU; the host keeps only the tree topology
-// (node keys, parent/child links) and 8 norms per node, and decides refinement:
-//   per level: screened boxes (host, from operator norm envelopes)
+// (node positions, parent/child links) and 8 norms per node:
+//   per level: screened boxes (device, from operator norm envelopes)
 //            -> generated input nodes (device mark + compute)
-//            -> work list of (g, f, ft, gt, term) tuples (device count + fill)
-//            -> contraction (device) -> norms (device) -> split test (host)
+//            -> work list of slices (g, f, ft, term) (device count + fill)
+//            -> contraction and norms (device) -> split test (device, or host)
 //   after the last level: additive top-down push of the coarse scaling parts,
 //   bottom-up compression and norms (device).
 // Operators (Gaussian-sum fit on the host, NS blocks on the device) are built
@@ -2706,10 +2706,7 @@ struct SumJob {
     void union_grid() {
         const size_t m = f.size();
         size_t most = 0;
-        for (TreeH *t : f) {
-            if (t->n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
-            most = std::max(most, (size_t)t->n());
-        }
+        for (TreeH *t : f) most = std::max(most, (size_t)t->n());
         out->make_roots();
         out->reserve_host(most);
         src.clear();
@@ -2744,7 +2741,10 @@ static void sum_batch(std::vector<SumJob> &jobs) {
     Ctx &C = *M.ctx;
     size_t nodes = 0;
     for (SumJob &J : jobs)
-        for (TreeH *t : J.f) nodes += t->n();
+        for (TreeH *t : J.f) {
+            if (t->n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
+            nodes += t->n();
+        }
     for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(); });
     std::vector<size_t> iofs(jobs.size() + 1, 0), sofs(jobs.size() + 1, 0);
     for (size_t j = 0; j < jobs.size(); j++) {
