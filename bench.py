@@ -539,7 +539,7 @@ def main():
     alg = F * 6.0 * K ** 4
     tc = best["t_contract_per_step"]
     achieved = alg / tc if tc > 0 else 0.0
-    kern = f"k_contract_mfma{K}" if dtype != "f64" else "k_contract_fp64"
+    kern = f"k_contract_mfma{K}" if dtype != "f64" else "k_contract_slices64"
     per_launch = measured_traffic(kern, f"helmholtz{args.orbitals}_k{args.k}_prec{prec_tag(args.prec)}")
     # algorithmic bytes of a step: every input and output node block read or written once (FP64)
     in_nodes = sum(t.getNNodes() for t in trees)
@@ -547,8 +547,8 @@ def main():
     roofline = dict(bound="mfma", achieved=achieved / 1e12, peak=PEAK[dtype] / 1e12, unit="TFLOP/s",
                     frac=achieved / PEAK[dtype],
                     traffic=per_launch,
-                    kernel=(kern + " + k_contract_fp64 + k_reduce_partials") if dtype != "f64"
-                    else "k_contract_fp64 + k_reduce_partials",
+                    kernel=(kern + " + k_contract_slices64 + k_reduce_slots") if dtype != "f64"
+                    else "k_contract_slices64 + k_reduce_slots",
                     plain_tuples_per_step=F, alg_flops_per_tuple=6.0 * K ** 4,
                     issued_tflops=(best["flops_per_step"] / tc / 1e12) if tc > 0 else None,
                     contraction_ms_per_step=1e3 * tc,

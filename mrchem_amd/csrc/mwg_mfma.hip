@@ -10,7 +10,7 @@
 // slice result, scaled by the term weight and masked to the components whose tuples
 // survive the screening, is summed over the task's slices (k = 7: FP32 over at most 64
 // slices per wave, then FP64 over the waves; k = 9: FP64 per slice), and a task's sum goes
-// to one node slot (8 K^3 FP64) that k_reduce_partials adds, in slot order, to the
+// to one node slot (8 K^3 FP64) that k_reduce_slots adds, in slot order, to the
 // node's FP64 tuple partials.  A task is a run of slices of one output node, one task
 // per 256-thread workgroup.
 //
