@@ -228,7 +228,7 @@ struct Readback {
 
 // scratch of the operator level builder: item lists, child-scale blocks, norms
 struct NSScratch {
-    DBuf<double> t1, blk, nrm;
+    DBuf<double> t1, nrm;
     DBuf<char> lists;
 };
 
@@ -673,9 +673,11 @@ struct OperH {
 // of the batch's depth.  Rows (one per translation, 4 K^2 doubles: types by (gt, ft) bit)
 // are numbered in request order (rows, plus the total at the end); the requests from
 // groups[i].r0 up to the next group's r0 write their rows to groups[i].blocks (row 0 = the
-// group's first row), and their norms to groups[i].norms when given; the 4 norms of every
-// row also go to nrm.  The item lists of all batches travel in one upload; the child-scale
-// blocks are computed in chunks of whole groups that fit a bounded scratch.  Asynchronous on
+// group's first row) and their norms to groups[i].norms, each when given; the 4 norms of every
+// row also go to nrm.  The item lists of all batches travel in one upload, and two launches
+// compute the blocks of all of them (a pair per chunk of whole groups whose child-scale rows fit
+// a bounded scratch).  With launches per operator and depth, the new Helmholtz operators of an
+// SCF step (four orbitals, k = 7) took 63 of them and 0.65 ms, now 4 and 0.2.  Asynchronous on
 // the context's stream: the caller synchronises (by downloading the norms).
 struct NSRequest {
     int term;
@@ -704,12 +706,15 @@ static void compute_ns(MraH &M, const std::vector<NSBatch *> &bs) {
     const long long cap = std::max<long long>(1, ((long long)256 << 20) / (8 * K2));
     struct Plan {
         std::vector<long long> lo1, hi1, trow;
-        std::vector<size_t> chunk0;
         size_t b1off = 0, toff = 0, noff = 0;
     };
+    struct Group {  // one group's requests, child-scale items and rows, numbered over all batches
+        size_t b, g, r0, r1;
+        long long t0, t1, f0, f1;
+    };
     std::vector<Plan> pl(bs.size());
+    std::vector<Group> gs;
     size_t nb1 = 0, nt = 0, nn = 0;
-    long long tmax = 0;
     for (size_t b = 0; b < bs.size(); b++) {
         NSBatch &X = *bs[b];
         Plan &P = pl[b];
@@ -729,35 +734,45 @@ static void compute_ns(MraH &M, const std::vector<NSBatch *> &bs) {
         }
         if (X.rows[nr] >= ((long long)1 << 31) || P.trow[nr] >= ((long long)1 << 31))
             throw Error(MWG_ERR_RANGE, "operator level too large");
-        // chunks of groups whose child-scale rows fit the scratch (at least one group each)
-        auto gend = [&](size_t g) { return g + 1 < ng ? X.groups[g + 1].r0 : nr; };
-        P.chunk0 = {0};
-        for (size_t g = 0; g < ng;) {
-            const size_t c0 = g;
-            while (g < ng && (g == c0 || P.trow[gend(g)] - P.trow[X.groups[c0].r0] <= cap)) g++;
-            P.chunk0.push_back(g);
-            tmax = std::max(tmax, P.trow[gend(g - 1)] - P.trow[X.groups[c0].r0]);
-        }
         P.b1off = nb1;
         P.toff = nt;
         P.noff = nn;
+        for (size_t g = 0; g < ng; g++) {
+            const size_t r0 = X.groups[g].r0, r1 = g + 1 < ng ? X.groups[g + 1].r0 : nr;
+            gs.push_back(Group{b, g, r0, r1, (long long)nt + P.trow[r0], (long long)nt + P.trow[r1],
+                               (long long)nn + X.rows[r0], (long long)nn + X.rows[r1]});
+        }
         nb1 += X.b1.size();
         nt += (size_t)P.trow[nr];
         nn += (size_t)X.rows[nr];
     }
+    if (gs.empty()) return;
+    // chunks of groups whose child-scale rows fit the scratch (at least one group each)
+    std::vector<size_t> chunk0 = {0};
+    long long tmax = 0;
+    for (size_t g = 0; g < gs.size();) {
+        const size_t c0 = g;
+        while (g < gs.size() && (g == c0 || gs[g].t1 - gs[c0].t0 <= cap)) g++;
+        chunk0.push_back(g);
+        tmax = std::max(tmax, gs[g - 1].t1 - gs[c0].t0);
+    }
+    if (tmax >= ((long long)1 << 31)) throw Error(MWG_ERR_RANGE, "operator level too large");
     // item lists of all batches; child-scale rows count from their chunk's first row
-    std::vector<double> b1(nb1);
-    std::vector<int> tterm(nt), row0(nn), tlo(nn), thi(nn);
+    std::vector<double> b1(nb1), pre(nb1);
+    std::vector<int> tterm(nt), row0(nn), tlo(nn), thi(nn), grp(nn);
     std::vector<long long> tdelta(nt), ndelta(nn);
+    std::vector<NSOut> outs(gs.size());
     for (size_t b = 0; b < bs.size(); b++) {
-        const NSBatch &X = *bs[b];
-        const Plan &P = pl[b];
-        const size_t nr = X.req.size(), ng = X.groups.size();
-        auto gend = [&](size_t g) { return g + 1 < ng ? X.groups[g + 1].r0 : nr; };
-        std::copy(X.b1.begin(), X.b1.end(), b1.begin() + P.b1off);
-        for (size_t c = 0; c + 1 < P.chunk0.size(); c++) {
-            const long long base = P.trow[X.groups[P.chunk0[c]].r0];
-            for (size_t r = X.groups[P.chunk0[c]].r0; r < gend(P.chunk0[c + 1] - 1); r++) {
+        std::copy(bs[b]->b1.begin(), bs[b]->b1.end(), b1.begin() + pl[b].b1off);
+        std::fill_n(pre.begin() + pl[b].b1off, bs[b]->b1.size(), std::ldexp(1.0, -(M.n0 + bs[b]->d + 1)));
+    }
+    for (size_t c = 0; c + 1 < chunk0.size(); c++)
+        for (size_t g = chunk0[c]; g < chunk0[c + 1]; g++) {
+            const NSBatch &X = *bs[gs[g].b];
+            const Plan &P = pl[gs[g].b];
+            const NSGroup &G = X.groups[gs[g].g];
+            outs[g] = NSOut{G.blocks, G.norms, X.nrm + 4 * X.rows[gs[g].r0], gs[g].f0};
+            for (size_t r = gs[g].r0; r < gs[g].r1; r++) {
                 for (long long q = P.lo1[r]; q <= P.hi1[r]; q++) {
                     const size_t i = P.toff + (size_t)(P.trow[r] + q - P.lo1[r]);
                     tterm[i] = (int)P.b1off + X.req[r].term;
@@ -766,13 +781,13 @@ static void compute_ns(MraH &M, const std::vector<NSBatch *> &bs) {
                 for (long long q = X.req[r].dlo; q <= X.req[r].dhi; q++) {
                     const size_t i = P.noff + (size_t)(X.rows[r] + q - X.req[r].dlo);
                     ndelta[i] = q;
-                    row0[i] = (int)(P.trow[r] - base);
+                    row0[i] = (int)((long long)P.toff + P.trow[r] - gs[chunk0[c]].t0);
                     tlo[i] = (int)P.lo1[r];
                     thi[i] = (int)P.hi1[r];
+                    grp[i] = (int)g;
                 }
             }
         }
-    }
     size_t off = 0;
     auto sec = [&](size_t bytes) {
         const size_t o = off;
@@ -781,7 +796,8 @@ static void compute_ns(MraH &M, const std::vector<NSBatch *> &bs) {
     };
     const size_t o_b1 = sec(nb1 * sizeof(double)), o_tt = sec(nt * sizeof(int)), o_td = sec(nt * sizeof(long long)),
                  o_nd = sec(nn * sizeof(long long)), o_r0 = sec(nn * sizeof(int)), o_lo = sec(nn * sizeof(int)),
-                 o_hi = sec(nn * sizeof(int));
+                 o_hi = sec(nn * sizeof(int)), o_pre = sec(nb1 * sizeof(double)), o_gr = sec(nn * sizeof(int)),
+                 o_out = sec(outs.size() * sizeof(NSOut));
     std::vector<char> pk(std::max<size_t>(off, 1));
     std::memcpy(pk.data() + o_b1, b1.data(), nb1 * sizeof(double));
     std::memcpy(pk.data() + o_tt, tterm.data(), nt * sizeof(int));
@@ -790,33 +806,24 @@ static void compute_ns(MraH &M, const std::vector<NSBatch *> &bs) {
     std::memcpy(pk.data() + o_r0, row0.data(), nn * sizeof(int));
     std::memcpy(pk.data() + o_lo, tlo.data(), nn * sizeof(int));
     std::memcpy(pk.data() + o_hi, thi.data(), nn * sizeof(int));
+    std::memcpy(pk.data() + o_pre, pre.data(), nb1 * sizeof(double));
+    std::memcpy(pk.data() + o_gr, grp.data(), nn * sizeof(int));
+    std::memcpy(pk.data() + o_out, outs.data(), outs.size() * sizeof(NSOut));
     S.lists.alloc(pk.size());
     stage_copy(C, S.lists.p, pk.data(), off);
     const char *L = S.lists.p;
-    const double *db1 = (const double *)(L + o_b1);
-    const int *dtt = (const int *)(L + o_tt), *dr0 = (const int *)(L + o_r0), *dlo = (const int *)(L + o_lo),
-              *dhi = (const int *)(L + o_hi);
-    const long long *dtd = (const long long *)(L + o_td), *dnd = (const long long *)(L + o_nd);
+    const double *db1 = (const double *)(L + o_b1), *dpre = (const double *)(L + o_pre);
+    const int *dtt = (const int *)(L + o_tt);
+    const long long *dtd = (const long long *)(L + o_td);
+    NSItems it{(const long long *)(L + o_nd), (const int *)(L + o_r0), (const int *)(L + o_lo), (const int *)(L + o_hi),
+               (const int *)(L + o_gr), (const NSOut *)(L + o_out)};
     S.t1.alloc((size_t)std::max<long long>(tmax, 1) * K2);
     hipStream_t s = C.stream;
-    for (size_t b = 0; b < bs.size(); b++) {
-        const NSBatch &X = *bs[b];
-        const Plan &P = pl[b];
-        const size_t nr = X.req.size(), ng = X.groups.size();
-        auto gend = [&](size_t g) { return g + 1 < ng ? X.groups[g + 1].r0 : nr; };
-        const double pre1 = std::ldexp(1.0, -(M.n0 + X.d + 1));
-        for (size_t c = 0; c + 1 < P.chunk0.size(); c++) {
-            const long long t0 = P.trow[X.groups[P.chunk0[c]].r0], nt1 = P.trow[gend(P.chunk0[c + 1] - 1)] - t0;
-            HC(launch_tblock_mom(s, (int)nt1, dtt + P.toff + t0, dtd + P.toff + t0, db1, pre1, B.K, M.ccoef.p, C.gx.p,
-                                 C.gw.p, S.t1.p));
-            for (size_t g = P.chunk0[c]; g < P.chunk0[c + 1]; g++) {
-                const long long f0 = X.rows[X.groups[g].r0], n = X.rows[gend(g)] - f0;
-                const size_t i0 = P.noff + (size_t)f0;
-                if (n > 0)
-                    HC(launch_nsblocks(s, (int)n, dnd + i0, dr0 + i0, dlo + i0, dhi + i0, S.t1.p, M.W.p, B.K,
-                                       X.groups[g].blocks, X.nrm + 4 * f0, X.groups[g].norms));
-            }
-        }
+    for (size_t c = 0; c + 1 < chunk0.size(); c++) {
+        const Group &A = gs[chunk0[c]], &Z = gs[chunk0[c + 1] - 1];
+        HC(launch_tblock_mom(s, (int)(Z.t1 - A.t0), dtt + A.t0, dtd + A.t0, db1, dpre, B.K, M.ccoef.p, C.gx.p, C.gw.p,
+                             S.t1.p));
+        HC(launch_nsblocks(s, A.f0, Z.f1 - A.f0, it, S.t1.p, M.W.p, B.K));
     }
 }
 
@@ -849,7 +856,7 @@ static void build_levels(MraH &M, std::vector<LevelJob> &lj, bool with16) {
     const int K2 = M.B.K2;
     const long long boxmax = std::max({M.boxes[0], M.boxes[1], M.boxes[2]});
     // phase 1: near-diagonal blocks decide which terms are active
-    long long n1tot = 0, n1max = 0;
+    long long n1tot = 0;
     std::vector<long long> nrm0(lj.size());
     for (size_t j = 0; j < lj.size(); j++) {
         LevelJob &J = lj[j];
@@ -876,13 +883,11 @@ static void build_levels(MraH &M, std::vector<LevelJob> &lj, bool with16) {
         const long long n1 = ns_rows(J.near.req);
         nrm0[j] = n1tot;
         n1tot += n1;
-        n1max = std::max(n1max, n1);
     }
-    C.ns.blk.alloc((size_t)std::max<long long>(n1max, 1) * 4 * K2);
     C.ns.nrm.alloc((size_t)std::max<long long>(n1tot, 1) * 4);
     std::vector<NSBatch *> batches;
     for (size_t j = 0; j < lj.size(); j++) {
-        lj[j].near.groups = {NSGroup{0, C.ns.blk.p, nullptr}};
+        lj[j].near.groups = {NSGroup{0, nullptr, nullptr}};  // (only their norms are wanted)
         lj[j].near.nrm = C.ns.nrm.p + 4 * nrm0[j];
         batches.push_back(&lj[j].near);
     }

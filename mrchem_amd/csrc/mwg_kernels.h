@@ -150,12 +150,22 @@ struct GenState {
 
 hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
                          double pre, const DevBasis &B, const double *gx, const double *gw, double *out);
-hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta,
-                             const double *b, double pre, int K, const double *ccoef, const double *gx,
-                             const double *gw, double *out);
-hipError_t launch_nsblocks(hipStream_t s, int n, const long long *item_delta, const int *item_row0,
-                           const int *item_tlo, const int *item_thi, const double *t1, const double *W, int K,
-                           double *blocks, double *norms, double *norms2 = nullptr);
+hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
+                             const double *pre, int K, const double *ccoef, const double *gx, const double *gw,
+                             double *out);
+// where a group of NS block rows goes (blocks and norms may be null) and its first row
+struct NSOut {
+    double *blocks, *norms, *nrm;
+    long long first;
+};
+// per row: translation, child-scale rows (the first one's index, their range), group
+struct NSItems {
+    const long long *delta;
+    const int *row0, *tlo, *thi, *grp;
+    const NSOut *outs;
+};
+hipError_t launch_nsblocks(hipStream_t s, long long first, long long n, const NSItems &items, const double *t1,
+                           const double *W, int K);
 hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3);
 hipError_t launch_dot(hipStream_t s, int n, const unsigned long long *pairs, const double *A, const double *B, int K3,
                       double *part);

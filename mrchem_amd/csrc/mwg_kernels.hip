@@ -121,13 +121,13 @@ __global__ void k_tblock(int n, const int *item_term, const long long *item_delt
 // moments in registers; one wave reduction, then the K^2 entries.
 template <int K>
 __global__ void __launch_bounds__(64) k_tblock_mom(int n, const int *item_term, const long long *item_delta,
-                                                   const double *bvals, double pre, const double *ccoef,
+                                                   const double *bvals, const double *pres, const double *ccoef,
                                                    const double *gx, const double *gw, double *out) {
     const int it = blockIdx.x;
     if (it >= n) return;
     constexpr int P = 2 * K, K2 = K * K;
     __shared__ double Ms[2 * P];
-    const double b = bvals[item_term[it]];
+    const double b = bvals[item_term[it]], pre = pres[item_term[it]];
     const double delta = (double)item_delta[it];
     const double zc = -delta;
     const double R = sqrt(GAUSS_CUT_D / b);
@@ -183,17 +183,16 @@ __global__ void __launch_bounds__(64) k_tblock_mom(int n, const int *item_term, 
 
 // NS blocks from the child-scale scaling blocks: R = W M W^T with
 // M = [[t(2d), t(2d-1)], [t(2d+1), t(2d)]]; type = 2*gt_bit + ft_bit.  The 4 block norms of
-// each translation go to norms and, when given, to norms2.
-__global__ void k_nsblocks(int n, const long long *item_delta, const int *item_row0, const int *item_tlo,
-                           const int *item_thi, const double *t1, const double *W, int K, double *blocks,
-                           double *norms, double *norms2) {
-    const int it = blockIdx.x;
-    if (it >= n) return;
+// each translation, and the blocks themselves, go to their group's arrays.
+__global__ void k_nsblocks(long long first, NSItems items, const double *t1, const double *W, int K) {
+    const long long it = first + blockIdx.x;
+    const NSOut o = items.outs[items.grp[it]];
+    const size_t row = (size_t)(it - o.first);
     const int N = 2 * K, K2 = K * K, tid = threadIdx.x, nt = blockDim.x;
     __shared__ double Ms[4 * MAXK * MAXK], R1[4 * MAXK * MAXK], Ws[4 * MAXK * MAXK];
     __shared__ double red[4][256];
-    const long long d = item_delta[it];
-    const int row0 = item_row0[it], tlo = item_tlo[it], thi = item_thi[it];
+    const long long d = items.delta[it];
+    const int row0 = items.row0[it], tlo = items.tlo[it], thi = items.thi[it];
     for (int e = tid; e < N * N; e += nt) Ws[e] = W[e];
     for (int e = tid; e < N * N; e += nt) {
         const int r = e / N, c = e % N;
@@ -218,7 +217,7 @@ __global__ void k_nsblocks(int n, const long long *item_delta, const int *item_r
         for (int l = 0; l < N; l++) s += R1[i * N + l] * Ws[j * N + l];
         const int gb = i / K, a = i % K, fb = j / K, i2 = j % K;
         const int type = 2 * gb + fb;
-        blocks[((size_t)it * 4 + type) * K2 + a * K + i2] = s;
+        if (o.blocks) o.blocks[(row * 4 + type) * K2 + a * K + i2] = s;
         part[type] += s * s;
     }
     for (int q = 0; q < 4; q++) red[q][tid] = part[q];
@@ -230,8 +229,8 @@ __global__ void k_nsblocks(int n, const long long *item_delta, const int *item_r
     }
     if (tid < 4) {
         const double v = sqrt(red[tid][0]);
-        norms[(size_t)it * 4 + tid] = v;
-        if (norms2) norms2[(size_t)it * 4 + tid] = v;
+        o.nrm[row * 4 + tid] = v;
+        if (o.norms) o.norms[row * 4 + tid] = v;
     }
 }
 
@@ -1715,21 +1714,19 @@ hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long 
     return hipGetLastError();
 }
 
-hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta,
-                             const double *b, double pre, int K, const double *ccoef, const double *gx,
-                             const double *gw, double *out) {
+hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
+                             const double *pre, int K, const double *ccoef, const double *gx, const double *gw,
+                             double *out) {
     if (n <= 0) return hipSuccess;
     MWG_DISPATCH_K(K, hipLaunchKernelGGL(k_tblock_mom<KK>, dim3(n), dim3(64), 0, s, n, item_term, item_delta, b, pre,
                                          ccoef, gx, gw, out));
     return hipGetLastError();
 }
 
-hipError_t launch_nsblocks(hipStream_t s, int n, const long long *item_delta, const int *item_row0,
-                           const int *item_tlo, const int *item_thi, const double *t1, const double *W, int K,
-                           double *blocks, double *norms, double *norms2) {
+hipError_t launch_nsblocks(hipStream_t s, long long first, long long n, const NSItems &items, const double *t1,
+                           const double *W, int K) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_nsblocks, dim3(n), dim3(256), 0, s, n, item_delta, item_row0, item_tlo, item_thi, t1, W, K,
-                       blocks, norms, norms2);
+    hipLaunchKernelGGL(k_nsblocks, dim3((unsigned)n), dim3(256), 0, s, first, items, t1, W, K);
     return hipGetLastError();
 }
 
