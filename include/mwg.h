@@ -135,6 +135,8 @@ int mwg_tree_layout_check(const int *boxes, int max_depth, int64_t n, const int 
 int mwg_tree_export(mwg_tree tree, int *depth, int64_t *lr, double *coefs);
 int mwg_tree_rescale(mwg_tree tree, double c);               /* FunctionTree::rescale (HelmholtzVector.cpp:81) */
 int mwg_tree_dot(mwg_tree a, mwg_tree b, double *out);       /* mrcpp::dot */
+/* out[i] = <a[i], b[i]> for n pairs of trees of one MRA, in one launch */
+int mwg_tree_dot_batch(int n, mwg_tree *a, mwg_tree *b, double *out);
 /* mwg_tree_dot without device allocation.  No counterpart in the reference: for callers
  * that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Node pairs and partial sums live in a static 8 MiB

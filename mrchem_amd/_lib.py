@@ -79,6 +79,7 @@ def _sig():
         "mwg_tree_export": [vp, fi, fl, fd],
         "mwg_tree_rescale": [vp, d],
         "mwg_tree_dot": [vp, vp, C.POINTER(C.c_double)],
+        "mwg_tree_dot_batch": [i, pvp, pvp, fd],
         "mwg_tree_dot_noalloc": [vp, vp, C.POINTER(C.c_double)],
         "mwg_meta_write": [C.c_char_p, C.POINTER(OrbitalMeta), i],
         "mwg_meta_read": [C.c_char_p, C.POINTER(OrbitalMeta), C.POINTER(C.c_int)],
@@ -121,7 +122,7 @@ EXPORTED = ["mwg_ctx_create", "mwg_ctx_destroy", "mwg_last_error", "mwg_sync", "
             "mwg_ctx_get_tuning", "mwg_ctx_trim", "mwg_mra_create", "mwg_mra_destroy",
             "mwg_tree_create", "mwg_tree_destroy", "mwg_tree_nnodes", "mwg_tree_sqnorm", "mwg_tree_maxdepth",
             "mwg_tree_mra", "mwg_mra_order",
-            "mwg_tree_import", "mwg_tree_layout_check", "mwg_tree_export", "mwg_tree_rescale", "mwg_tree_dot", "mwg_tree_dot_noalloc",
+            "mwg_tree_import", "mwg_tree_layout_check", "mwg_tree_export", "mwg_tree_rescale", "mwg_tree_dot", "mwg_tree_dot_batch", "mwg_tree_dot_noalloc",
             "mwg_tree_eval", "mwg_meta_write", "mwg_meta_read", "mwg_tree_save", "mwg_tree_load",
             "mwg_tree_file_write", "mwg_tree_file_read",
             "mwg_project_gauss", "mwg_project_hydrogen", "mwg_oper_poisson", "mwg_oper_helmholtz",

@@ -288,7 +288,7 @@ struct Ctx {
     DBuf<HashItem> hitems;  // node tables to build, and their nodes' keys
     DBuf<unsigned long long> hkeys;
     DBuf<GatherItem> gitems;
-    DBuf<unsigned long long> dotpairs;
+    DBuf<DotPair> dotpairs;
     DBuf<MulItem> mitems;  // products and projections: items of all jobs, and the jobs
     DBuf<MulJobDev> mjobs;
     DBuf<SumItem> sitems;  // linear combinations: output nodes and their terms
@@ -3238,24 +3238,34 @@ int mwg_tree_rescale(mwg_tree tree, double c) {
     });
 }
 
-int mwg_tree_dot(mwg_tree a, mwg_tree b, double *out) {
-    if (!a || !b || !out) return MWG_ERR_ARG;
-    if (a->mra != b->mra) return MWG_ERR_ARG;
-    Ctx *C = a->mra->ctx;
+int mwg_tree_dot(mwg_tree a, mwg_tree b, double *out) { return mwg_tree_dot_batch(1, &a, &b, out); }
+
+int mwg_tree_dot_batch(int n, mwg_tree *a, mwg_tree *b, double *out) {
+    if (n <= 0 || !a || !b || !out) return MWG_ERR_ARG;
+    for (int i = 0; i < n; i++)
+        if (!a[i] || !b[i] || a[i]->mra != b[i]->mra || a[i]->mra != a[0]->mra) return MWG_ERR_ARG;
+    Ctx *C = a[0]->mra->ctx;
     return guarded(C, [&] {
-        if (a->roots.empty() || b->roots.empty()) {  // an empty tree is the zero function
-            *out = 0.0;
-            return;
+        const size_t B8 = 8 * (size_t)a[0]->K3();
+        std::vector<DotPair> pairs;
+        std::vector<size_t> ofs(n + 1, 0);
+        for (int i = 0; i < n; i++) {
+            const double *ca = a[i]->coef.p, *cb = b[i]->coef.p;
+            if (!a[i]->roots.empty() && !b[i]->roots.empty())  // (an empty tree is the zero function)
+                common_nodes(*a[i], *b[i], [&](int ia, int ib, int skip0) {
+                    pairs.push_back(DotPair{ca + ia * B8, cb + ib * B8, skip0});
+                });
+            ofs[i + 1] = pairs.size();
         }
-        std::vector<unsigned long long> pairs;
-        common_nodes(*a, *b, [&](int ia, int ib, int skip0) { pairs.push_back(dot_pair(ia, ib, skip0)); });
         upload_async(*C, C->dotpairs, pairs.data(), pairs.size());
-        C->rbd.alloc(pairs.size() * sizeof(double));
-        HC(launch_dot(C->stream, (int)pairs.size(), C->dotpairs.p, a->coef.p, b->coef.p, a->K3(), (double *)C->rbd.p));
+        C->rbd.alloc(std::max<size_t>(pairs.size(), 1) * sizeof(double));
+        HC(launch_dot(C->stream, (int)pairs.size(), C->dotpairs.p, a[0]->K3(), (double *)C->rbd.p));
         const double *hp = read_compact(*C, pairs.size());
-        double sum = 0.0;
-        for (size_t i = 0; i < pairs.size(); i++) sum += hp[i];
-        *out = sum;
+        for (int i = 0; i < n; i++) {
+            double sum = 0.0;
+            for (size_t q = ofs[i]; q < ofs[i + 1]; q++) sum += hp[q];
+            out[i] = sum;
+        }
     });
 }
 

@@ -167,8 +167,12 @@ struct NSItems {
 hipError_t launch_nsblocks(hipStream_t s, long long first, long long n, const NSItems &items, const double *t1,
                            const double *W, int K);
 hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3);
-hipError_t launch_dot(hipStream_t s, int n, const unsigned long long *pairs, const double *A, const double *B, int K3,
-                      double *part);
+// two nodes' coefficients (skip0: without their scaling parts)
+struct DotPair {
+    const double *a, *b;
+    long long skip0;
+};
+hipError_t launch_dot(hipStream_t s, int n, const DotPair *pairs, int K3, double *part);
 // sum over node pairs of a . b (part: nblocks doubles of block sums, res: the total)
 hipError_t launch_dot_pairs(hipStream_t s, int n, const unsigned long long *pairs, const double *A,
                             const double *B, int K3, int nblocks, double *part, double *res);

@@ -281,17 +281,15 @@ __global__ void __launch_bounds__(256) k_gather(const GatherItem *items, double 
         dst[it.first + i] = it.p[i];
 }
 
-// per-pair partial dot products (pair words as for k_dot_pairs), one workgroup per pair
-__global__ void __launch_bounds__(256) k_dot(const unsigned long long *pairs, const double *A, const double *B, int K3,
-                                             double *part) {
+// Per-pair partial dot products, one workgroup per node pair, the pairs of several tree pairs in one
+// launch: the overlaps of four orbitals took ten of them, each with an upload and a wait (an SCF
+// step at k = 7 without its export 4.6 ms, 4.3 now).
+__global__ void __launch_bounds__(256) k_dot(const DotPair *pairs, int K3, double *part) {
     __shared__ double wsum[4];
-    const unsigned long long p = pairs[blockIdx.x];
-    const int c0 = (int)((p >> 31) & 1u);
-    const double *a = A + (size_t)(p & 0x7fffffffu) * 8 * K3;
-    const double *b = B + (size_t)(p >> 32) * 8 * K3;
+    const DotPair p = pairs[blockIdx.x];
     double s = 0.0;
 #pragma unroll 8
-    for (int e = c0 * K3 + threadIdx.x; e < 8 * K3; e += 256) s += a[e] * b[e];
+    for (int e = (int)p.skip0 * K3 + threadIdx.x; e < 8 * K3; e += 256) s += p.a[e] * p.b[e];
     s = block_sum_256(s, wsum);
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -1744,10 +1742,9 @@ hipError_t launch_dot_pairs(hipStream_t s, int n, const unsigned long long *pair
     return hipGetLastError();
 }
 
-hipError_t launch_dot(hipStream_t s, int n, const unsigned long long *pairs, const double *A, const double *B, int K3,
-                      double *part) {
+hipError_t launch_dot(hipStream_t s, int n, const DotPair *pairs, int K3, double *part) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dot, dim3(n), dim3(256), 0, s, pairs, A, B, K3, part);
+    hipLaunchKernelGGL(k_dot, dim3(n), dim3(256), 0, s, pairs, K3, part);
     return hipGetLastError();
 }
 

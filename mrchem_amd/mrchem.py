@@ -97,6 +97,7 @@ class HelmholtzVector:
 
 
 DENSITY_BATCH = 32  # squares held at once
+DOT_BATCH = 32  # overlaps whose node pairs are listed at once
 
 
 def density(prec: float, Phi, mra) -> M.FunctionTree:
@@ -296,9 +297,12 @@ def get_norms(Phi) -> np.ndarray:
 def calc_overlap_matrix(Phi) -> np.ndarray:
     n = len(Phi)
     S = np.zeros((n, n))
-    for i in range(n):
-        for j in range(i, n):
-            S[i, j] = S[j, i] = M.dot(Phi[i].tree, Phi[j].tree)
+    pairs = [(i, j) for i in range(n) for j in range(i, n)]
+    for q in range(0, len(pairs), DOT_BATCH):
+        part = pairs[q:q + DOT_BATCH]
+        v = M.dot_batch([Phi[i].tree for i, _ in part], [Phi[j].tree for _, j in part])
+        for (i, j), s in zip(part, v):
+            S[i, j] = S[j, i] = s
     return S
 
 

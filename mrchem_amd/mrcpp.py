@@ -319,6 +319,18 @@ def dot(a: FunctionTree, b: FunctionTree) -> float:
     return float(v.value)
 
 
+def dot_batch(as_, bs) -> np.ndarray:
+    """<a_i, b_i> for all i, in one launch."""
+    n = len(as_)
+    if len(bs) != n:
+        raise MwgError("dot_batch: length mismatch")
+    out = np.zeros(n)
+    if n:
+        arr = C.c_void_p * n
+        check(lib().mwg_tree_dot_batch(n, arr(*[a.h for a in as_]), arr(*[b.h for b in bs]), out), as_[0].mra.ctx.h)
+    return out
+
+
 class Predictor:
     """Learned refinement predictor (2 x 64 tanh MLP, FP32) trained and run by HIP kernels."""
 

@@ -79,6 +79,8 @@ def test_linear_combinations_equal_chains_of_sums(G, k):
         a, b = c0.reshape(len(d0), -1)[key0], c1.reshape(len(d1), -1)[key1]
         assert np.abs(a - b).max() <= 1e-13 * np.abs(b).max()
         assert abs(o.getSquareNorm() - ref.getSquareNorm()) <= 1e-12 * ref.getSquareNorm()
+    # products of a batch: the single ones, to the bit
+    assert np.array_equal(G.dot_batch(f + outs, f[::-1] + outs), [G.dot(x, y) for x, y in zip(f + outs, f[::-1] + outs)])
     with pytest.raises(G.MwgError):
         G.add_batch([f[0]], [[(1.0, f[0]), (1.0, f[1])]])
     with pytest.raises(G.MwgError):
