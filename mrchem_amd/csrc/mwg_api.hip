@@ -249,7 +249,8 @@ struct Ctx {
     // generated-node table size of the applies (4 << gen_shift entries per input node, at
     // least 2^(14 + gen_shift) per job): raised when a batch overflowed the tables
     int gen_shift = 0;
-    int hw_chunk[LOOP_MAX_DEPTH] = {}, hw_schunk[LOOP_MAX_DEPTH] = {};  // per refinement iteration
+    // per refinement iteration: task sizes that the slot budget raised above the set ones (0: none)
+    int hw_chunk[LOOP_MAX_DEPTH] = {}, hw_schunk[LOOP_MAX_DEPTH] = {};
     double hw_ratio = 0.0;
     double mul_growth = 1.0;  // nodes of the last products over those of their union grids, and a tenth
     std::vector<int> last_in, last_out;  // input and output node counts of the last batch, per job
@@ -2298,10 +2299,10 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         }
         genLastNew = hsum.gen_count - genDone;
         genDone = hsum.gen_count;
-        if (iter < LOOP_MAX_DEPTH) {
-            C.hw_chunk[iter] = std::max(C.hw_chunk[iter], chunk_it);
-            // (a set slice_chunk is raised the same way when the node slots would not fit)
-            if (K != 8 && schunk_it > 0) C.hw_schunk[iter] = std::max(C.hw_schunk[iter], schunk_it);
+        if (iter < LOOP_MAX_DEPTH) {  // (only a raised size: the device loop takes it over the set one)
+            if (chunk_it > C.chunk) C.hw_chunk[iter] = std::max(C.hw_chunk[iter], chunk_it);
+            if (K != 8 && schunk_it > 0 && schunk_it != C.slice_chunk)
+                C.hw_schunk[iter] = std::max(C.hw_schunk[iter], schunk_it);
         }
         if (PT.on) {
             // candidates walked by the work-list kernels: per work node, its table's prefix total
@@ -3780,6 +3781,7 @@ int mwg_ctx_set_tuning(mwg_ctx ctx, int fp64_chunk, int slice_chunk) {
     }
     ctx->chunk = fp64_chunk;
     ctx->slice_chunk = slice_chunk;
+    for (int q = 0; q < LOOP_MAX_DEPTH; q++) ctx->hw_chunk[q] = ctx->hw_schunk[q] = 0;  // (raised from other settings)
     return MWG_OK;
 }
 
