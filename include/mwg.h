@@ -209,7 +209,8 @@ int mwg_multiply_batch(int n, const double *prec, mwg_tree *out, const double *c
 int mwg_add(mwg_tree out, double ca, mwg_tree a, double cb, mwg_tree b);
 /* n linear combinations out[i] = sum_k coef_k f_k, each on the union grid of its nterms[i] >= 1
  * terms; coef and inp hold the terms of all, one combination after the other.  As a chain of
- * mwg_add, with one launch for everything. */
+ * mwg_add, with one launch for everything.  The outputs differ from the inputs and each other
+ * (MWG_ERR_ARG). */
 int mwg_add_batch(int n, mwg_tree *out, const int *nterms, const double *coef, mwg_tree *inp);
 
 /* ---- operators: replace new mrcpp::PoissonOperator(MRA, prec) (SCFDriver.cpp:279) and

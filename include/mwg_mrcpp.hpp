@@ -289,7 +289,8 @@ inline void add(double prec, FunctionTree<3> &out, double a, FunctionTree<3> &in
 template <int D>
 using FunctionTreeVector = std::vector<std::tuple<double, FunctionTree<D> *>>;
 
-// out = sum_i c_i f_i (QMFunction::add / qmfunction::linear_combination) on the union grid
+// out = sum_i c_i f_i (QMFunction::add / qmfunction::linear_combination) on the union grid.  Of three
+// or more terms out may be any but the last (out += ...); else it differs from the terms.
 inline void add(double prec, FunctionTree<3> &out, FunctionTreeVector<3> &inp, int maxIter = -1) {
     (void)prec;
     (void)maxIter;
@@ -301,8 +302,21 @@ inline void add(double prec, FunctionTree<3> &out, FunctionTreeVector<3> &inp, i
         f.push_back(std::get<1>(t)->handle());
     }
     mwg_tree o = out.handle();
-    const int n = (int)inp.size();
-    detail::check(mwg_add_batch(1, &o, &n, coef.data(), f.data()));
+    const int n = (int)inp.size(), one = 1;
+    bool own = false;  // out is a term: summed into another tree, then copied
+    for (int i = 0; n >= 3 && f.back() != o && i < n; i++) own = own || f[i] == o;
+    if (!own) {
+        detail::check(mwg_add_batch(1, &o, &n, coef.data(), f.data()));
+        return;
+    }
+    mwg_mra m = nullptr;
+    mwg_tree t = nullptr;
+    detail::check(mwg_tree_mra(o, &m));
+    detail::check(mwg_tree_create(m, &t));
+    const std::unique_ptr<mwg_tree_s, int (*)(mwg_tree)> hold(t, mwg_tree_destroy);
+    detail::check(mwg_add_batch(1, &t, &n, coef.data(), f.data()));
+    const double c = 1.0;
+    detail::check(mwg_add_batch(1, &o, &one, &c, &t));
 }
 
 // copy_func: out = inp (grid and coefficients); copy_grid: inp's grid, zero coefficients;
