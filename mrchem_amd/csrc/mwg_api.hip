@@ -2741,48 +2741,93 @@ struct SumJob {
     }
 };
 
-// Linear combinations as one launch: every output node of every combination (mrcpp::add)
-static void sum_batch(std::vector<SumJob> &jobs) {
+// Records (output node, term) of one launch: 24 bytes each on the device, in the staging ring and on
+// the host, with 8 more and the nodes' items there.  An orbital vector's linear combinations have a
+// number that grows with its square (32 orbitals at k = 9: 3 million), so the records of all at
+// once are not bounded by the trees themselves.
+constexpr size_t SUM_RECORDS = (size_t)1 << 20;
+
+// every output node of the combinations, SUM_RECORDS records (at least one node) at a time
+static void sum_group(SumJob *jobs, size_t njobs) {
     MraH &M = *jobs[0].out->mra;
     Ctx &C = *M.ctx;
+    const size_t B8 = 8 * (size_t)M.B.K3;
     size_t nodes = 0;
-    for (SumJob &J : jobs)
-        for (TreeH *t : J.f) {
-            if (t->n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
-            nodes += t->n();
+    for (size_t j = 0; j < njobs; j++)
+        for (TreeH *t : jobs[j].f) nodes += t->n();
+    for_jobs_of(njobs, nodes, [&](size_t j) { jobs[j].union_grid(); });
+    for (size_t j = 0; j < njobs; j++) jobs[j].out->ensure_dev(jobs[j].out->n());
+    struct Part {  // nodes i0 .. i1 - 1 of a combination
+        size_t job;
+        int i0, i1;
+        size_t item0, src0;
+    };
+    std::vector<Part> parts;
+    std::vector<SumItem> items;
+    std::vector<SumSrc> srcs;
+    size_t j0 = 0;
+    for (int i0 = 0; j0 < njobs;) {
+        parts.clear();
+        size_t n = 0, ns = 0;
+        while (j0 < njobs) {
+            const int all = jobs[j0].out->n();
+            const size_t m = jobs[j0].f.size(), room = (SUM_RECORDS - std::min(ns, SUM_RECORDS)) / m;
+            if (room == 0 && n > 0) break;
+            const int i1 = (int)std::min<size_t>(all, i0 + std::max<size_t>(room, 1));
+            parts.push_back(Part{j0, i0, i1, n, ns});
+            n += i1 - i0;
+            ns += (i1 - i0) * m;
+            i0 = i1 < all ? i1 : 0;
+            if (i1 < all) break;
+            j0++;
         }
-    for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(); });
-    std::vector<size_t> iofs(jobs.size() + 1, 0), sofs(jobs.size() + 1, 0);
-    for (size_t j = 0; j < jobs.size(); j++) {
-        jobs[j].out->ensure_dev(jobs[j].out->n());
-        iofs[j + 1] = iofs[j] + jobs[j].out->n();
-        sofs[j + 1] = sofs[j] + jobs[j].src.size();
+        items.resize(n);
+        srcs.resize(ns);
+        for_jobs_of(parts.size(), ns, [&](size_t q) {
+            const Part &P = parts[q];
+            const SumJob &J = jobs[P.job];
+            const TreeH &T = *J.out;
+            const int m = (int)J.f.size();
+            const SumJob::Src *from = J.src.data() + (size_t)P.i0 * m;
+            SumSrc *to = srcs.data() + P.src0;
+            for (int i = P.i0; i < P.i1; i++) {
+                items[P.item0 + (i - P.i0)] = SumItem{T.coef.p + i * B8, T.norm.p + 8 * (size_t)i,
+                                                      T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2],
+                                                      (int)(P.src0 + (size_t)(i - P.i0) * m), m};
+                for (int k = 0; k < m; k++, from++)
+                    *to++ = SumSrc{J.f[k]->coef.p + from->node * B8, J.coef[k], from->steps};
+            }
+        });
+        upload_async(C, C.sitems, items.data(), n);
+        upload_async(C, C.ssrcs, srcs.data(), ns);
+        C.rbd.alloc(8 * n * sizeof(double));
+        HC(launch_sum(C.stream, (int)n, C.sitems.p, C.ssrcs.p, M.dev(), (double *)C.rbd.p));
+        const double *h = read_compact(C, 8 * n);
+        for (const Part &P : parts)
+            std::copy(h + 8 * P.item0, h + 8 * (P.item0 + (P.i1 - P.i0)),
+                      jobs[P.job].out->cnorm.begin() + 8 * (size_t)P.i0);
     }
-    const size_t n = iofs.back(), ns = sofs.back(), B8 = 8 * (size_t)M.B.K3;
-    if (ns > (size_t)INT_MAX) throw Error(MWG_ERR_RANGE, "add: too many nodes and terms for one call");
-    std::vector<SumItem> items(n);
-    std::vector<SumSrc> srcs(ns);
-    for_jobs_of(jobs.size(), ns, [&](size_t j) {
-        const SumJob &J = jobs[j];
-        const TreeH &T = *J.out;
-        const int m = (int)J.f.size();
-        for (int i = 0; i < T.n(); i++)
-            items[iofs[j] + i] = SumItem{T.coef.p + i * B8, T.norm.p + 8 * (size_t)i,
-                                         T.lr[3 * i], T.lr[3 * i + 1], T.lr[3 * i + 2],
-                                         (int)(sofs[j] + (size_t)i * m), m};
-        for (size_t q = 0; q < J.src.size(); q++) {
-            const int k = (int)(q % m);
-            srcs[sofs[j] + q] = SumSrc{J.f[k]->coef.p + J.src[q].node * B8, J.coef[k], J.src[q].steps};
-        }
-    });
-    upload_async(C, C.sitems, items.data(), n);
-    upload_async(C, C.ssrcs, srcs.data(), ns);
-    C.rbd.alloc(8 * n * sizeof(double));
-    HC(launch_sum(C.stream, (int)n, C.sitems.p, C.ssrcs.p, M.dev(), (double *)C.rbd.p));
-    const double *h = read_compact(C, 8 * n);
-    for (size_t j = 0; j < jobs.size(); j++) {  // (the items are every node in order)
-        jobs[j].out->cnorm.assign(h + 8 * iofs[j], h + 8 * iofs[j + 1]);
+    for (size_t j = 0; j < njobs; j++) {
         jobs[j].out->sqnorm_from_cnorm();
+        std::vector<SumJob::Src>().swap(jobs[j].src);
+    }
+}
+
+// Linear combinations (mrcpp::add): all inputs are checked first, then the combinations are taken in
+// groups of about SUM_RECORDS records, one launch each where the estimate holds
+static void sum_batch(std::vector<SumJob> &jobs) {
+    std::vector<size_t> est(jobs.size(), 0);
+    for (size_t j = 0; j < jobs.size(); j++) {
+        for (TreeH *t : jobs[j].f) {
+            if (t->n() == 0) throw Error(MWG_ERR_STATE, "add: empty input tree");
+            est[j] = std::max(est[j], (size_t)t->n());
+        }
+        est[j] *= jobs[j].f.size();
+    }
+    for (size_t a = 0, b; a < jobs.size(); a = b) {
+        size_t sum = est[a];
+        for (b = a + 1; b < jobs.size() && sum + est[b] <= SUM_RECORDS; b++) sum += est[b];
+        sum_group(jobs.data() + a, b - a);
     }
 }
 
