@@ -1510,6 +1510,16 @@ static double slice_flops(int K) {
 // device memory for the task slots of one refinement iteration (per kind of task)
 constexpr double SLOT_BUDGET = 8.0 * (1ull << 30);
 
+// a reservation that may prove larger than its use leaves two fifths of the free memory
+static bool fits_comfortably(Ctx &C, double bytes) {
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return bytes <= 0.6 * ((double)fr + (double)C.cache.bytes);
+}
+
 // gen_shift: the generated-node tables hold 4 << gen_shift entries per input node, and at
 // least 2^(14 + gen_shift)
 static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, std::vector<mwg_apply_stats> &stats,
@@ -1745,15 +1755,8 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
             caps_j[j] = (int)std::min<double>((nr + std::ceil(est) + 64 + 7), (double)(INT_MAX / 16)) & ~7;
             need_bytes += std::max(0.0, ((double)caps_j[j] * 8 * K3 - (double)jobs[j].out->coef.n) * sizeof(double));
         }
-        {
-            // the reservation must fit comfortably (else the host loop, which grows as it goes)
-            size_t fr = 0, tot = 0;
-            if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
-            if (need_bytes > 0.6 * ((double)fr + (double)C.cache.bytes)) return false;
-        }
+        // the reservation must fit comfortably (else the host loop, which grows as it goes)
+        if (!fits_comfortably(C, need_bytes)) return false;
         std::vector<LoopJob> lj(njobs);
         size_t topo = 0;
         for (int j = 0; j < njobs; j++) {
@@ -2652,12 +2655,12 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
     }
     for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(M.maxDepth); });
     // room for the refinement that the last batch needed beyond the union grids (a tree that
-    // grows level by level is allocated and copied at each)
-    double n_union = 0.0, n_out = 0.0;
-    for (MulJob &J : jobs) {
-        n_union += J.out->n();
-        J.out->ensure_dev((size_t)(J.out->n() * std::min(2.0, C.mul_growth)));
-    }
+    // grows level by level is allocated and copied at each), where memory is not short: that batch
+    // may have been of quite other functions
+    double n_union = 0.0, n_out = 0.0, room = std::min(2.0, C.mul_growth);
+    for (MulJob &J : jobs) n_union += J.out->n();
+    if (!fits_comfortably(C, room * n_union * 8 * M.B.K3 * sizeof(double))) room = 1.0;
+    for (MulJob &J : jobs) J.out->ensure_dev((size_t)(J.out->n() * room));
     std::vector<size_t> ofs;
     while (const double *h = run_items(C, jobs, ofs, [&](int n, const MulItem *items, const MulJobDev *jd, double *cn) {
                HC(launch_multiply(C.stream, n, items, jd, M.geom(), M.dev(), cn));
