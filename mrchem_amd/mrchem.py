@@ -96,19 +96,35 @@ class HelmholtzVector:
         return [Orbital(o, p.occ, p.spin) for o, p in zip(outs, Phi)]
 
 
-DENSITY_BATCH = 32  # squares held at once
+DENSITY_BATCH = 32  # squares held at once, memory permitting
 DOT_BATCH = 32  # overlaps whose node pairs are listed at once
+
+
+def _add_squares(prec: float, rho, Phi, mra):
+    """rho (None: nothing) + sum_i occ_i phi_i^2, the squares as one batch; None where several fail
+    together (memory: the caller takes them one by one)."""
+    try:
+        sq = M.multiply_batch(prec, [M.FunctionTree(mra) for _ in Phi], [p.occ for p in Phi],
+                              [p.tree for p in Phi], [p.tree for p in Phi])
+        terms = sq if rho is None else [rho] + sq
+        return terms[0] if len(terms) == 1 else M.add_batch([M.FunctionTree(mra)], [[(1.0, t) for t in terms]])[0]
+    except M.MwgError:
+        if len(Phi) == 1:
+            raise
+        return None
 
 
 def density(prec: float, Phi, mra) -> M.FunctionTree:
     """rho = sum_i occ_i phi_i^2 (src/qmfunctions/density_utils.cpp:65-133)."""
-    rho = None
-    for i in range(0, len(Phi), DENSITY_BATCH):
-        part = Phi[i:i + DENSITY_BATCH]
-        sq = M.multiply_batch(prec, [M.FunctionTree(mra) for _ in part], [p.occ for p in part],
-                              [p.tree for p in part], [p.tree for p in part])
-        terms = sq if rho is None else [rho] + sq
-        rho = terms[0] if len(terms) == 1 else M.add_batch([M.FunctionTree(mra)], [[(1.0, t) for t in terms]])[0]
+    rho, i, step = None, 0, DENSITY_BATCH
+    while i < len(Phi):
+        part = Phi[i:i + step]
+        new = _add_squares(prec, rho, part, mra)
+        if new is None:
+            step = 1
+            continue
+        rho, new = new, None
+        i += len(part)
     return rho
 
 
