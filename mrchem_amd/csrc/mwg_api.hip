@@ -1512,6 +1512,7 @@ constexpr double SLOT_BUDGET = 8.0 * (1ull << 30);
 
 // a reservation that may prove larger than its use leaves two fifths of the free memory
 static bool fits_comfortably(Ctx &C, double bytes) {
+    if (bytes <= 0.6 * (double)C.cache.bytes) return true;  // (the query takes longer than small calls' launches)
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
         (void)hipGetLastError();

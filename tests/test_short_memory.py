@@ -4,6 +4,7 @@ A batch of products that fits at its own size runs, whatever ran on the context 
 the card is held by an allocation that no kernel touches; the calls that run out of memory fail
 on the host, in the allocator.
 """
+import ctypes as C
 import gc
 
 import numpy as np
@@ -16,13 +17,20 @@ pytestmark = pytest.mark.gpu
 GIB = 1 << 30
 
 
-def _hold_all_but(ctx, left):
-    import torch
-    gc.collect()
-    ctx.trim()
-    torch.cuda.empty_cache()
-    free = torch.cuda.mem_get_info()[0]
-    return torch.empty(max(free - left, 0), dtype=torch.uint8, device="cuda")
+class _Held:
+    """All of the card's free memory but `left` bytes, through the HIP runtime that the library uses."""
+
+    def __init__(self, ctx, left):
+        gc.collect()
+        ctx.trim()
+        with open("/proc/self/maps") as f:
+            paths = sorted({line.split()[-1] for line in f if "libamdhip64" in line})
+        free, total, self.p = C.c_size_t(), C.c_size_t(), C.c_void_p()
+        self.hip = next(h for h in map(C.CDLL, paths) if h.hipMemGetInfo(C.byref(free), C.byref(total)) == 0)
+        assert self.hip.hipMalloc(C.byref(self.p), C.c_size_t(max(free.value - left, 1 << 20))) == 0
+
+    def free(self):
+        self.hip.hipFree(self.p)
 
 
 def _products(G, mra, fine, n):
@@ -32,7 +40,6 @@ def _products(G, mra, fine, n):
 
 
 def test_products_after_products_that_grew():
-    import torch
     from mrchem_amd import mrcpp as G
     ctx = G.Context(0)
     mra = G.mra_from(configs.BOX20, 9, ctx=ctx)
@@ -45,14 +52,13 @@ def test_products_after_products_that_grew():
     n = int(2.4 * GIB / (nodes * 64000)) + 1
     grown = G.multiply(1e-6, G.FunctionTree(mra), 1.0, coarse, coarse)
     assert grown.getNNodes() > 2 * coarse.getNNodes()
-    held = _hold_all_but(ctx, 4 * GIB)
+    held = _Held(ctx, 4 * GIB)
     try:
         outs = _products(G, mra, fine, n)
         assert all(o.getNNodes() == nodes for o in outs)
         assert np.array_equal(outs[-1].export()[2], one.export()[2])
     finally:
         outs = None
-        del held
-        torch.cuda.empty_cache()
+        held.free()
         gc.collect()
         ctx.trim()
