@@ -38,6 +38,16 @@ __device__ inline int dhash_find(const DHash &h, uint64_t key) {
     return -1;
 }
 
+// The thread's index as a value of its own: addresses made from it are not computed ahead, and held
+// in registers, together with those of another place.  Where that spilled, a kernel needed scratch
+// memory, which the runtime takes from the device when it launches: with the card nearly full
+// it cannot, and ends the process's queue instead of returning an error.
+__device__ inline unsigned thread_here() {
+    unsigned t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 // sums over a block of 256 threads of 8 values per thread in a fixed order (lanes by butterfly,
 // then the waves); thread c < 8 gets the sum of value c
 __device__ inline double block_sum8(double (&ss)[8], double (*wsum)[8]) {

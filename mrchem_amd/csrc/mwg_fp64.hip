@@ -135,7 +135,8 @@ k_contract_slices64(int ntask_arg, const TaskSummary *sum, const SliceTask *task
     // records r0 .. r0 + RB + NS (clamped to the task) into LDS
     auto load_recs = [&](int r0) {
         const int n = 2 * min(RB + NS + 1, count - r0);
-        for (int q = tid; q < n; q += NT) ((uint4 *)recs)[q] = ((const uint4 *)(srec + r0))[q];
+        // (K = 7 has no register to spare for these addresses)
+        for (int q = K == 7 ? (int)thread_here() : tid; q < n; q += NT) ((uint4 *)recs)[q] = ((const uint4 *)(srec + r0))[q];
     };
     auto u = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
     typedef double piece __attribute__((ext_vector_type(D::P)));

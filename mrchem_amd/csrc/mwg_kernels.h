@@ -148,8 +148,6 @@ struct GenState {
     long long *tabcnt;  // per job table: [4 t + 3] counts the generated nodes it inserted
 };
 
-hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
-                         double pre, const DevBasis &B, const double *gx, const double *gw, double *out);
 hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
                              const double *pre, int K, const double *ccoef, const double *gx, const double *gw,
                              double *out);

@@ -14,27 +14,6 @@
 
 namespace mwg {
 
-// ----------------------------------------------------------------- device basis
-
-__device__ inline void d_phi(const DevBasis &B, double x, double *out) {
-    const int K = B.K;
-    double l[MAXK];
-    double t = 2.0 * x - 1.0, p0 = 1.0, p1 = t;
-    l[0] = 1.0;
-    if (K > 1) l[1] = sqrt(3.0) * t;
-    for (int n = 2; n < K; n++) {
-        double p2 = ((2.0 * n - 1.0) * t * p1 - (n - 1.0) * p0) / n;
-        p0 = p1;
-        p1 = p2;
-        l[n] = sqrt(2.0 * n + 1.0) * p2;
-    }
-    for (int i = 0; i < K; i++) {
-        double s = 0.0;
-        for (int j = 0; j < K; j++) s += B.U[i * K + j] * l[j];
-        out[i] = s;
-    }
-}
-
 // global-address-space views: uniform loads through these become scalar loads
 typedef const double __attribute__((address_space(1))) gdouble;
 typedef const float __attribute__((address_space(1))) gfloat;
@@ -60,63 +39,10 @@ __device__ inline double block_sum_256(double v, double *wsum) {
 // ----------------------------------------------------------------- operator blocks
 
 // Scaling-scaling block of one unit Gaussian exp(-b (delta + u - v)^2) at cell scale m:
-// t[i][j] = pre * int_{-1}^{1} exp(-b (delta+z)^2) C_ij(z) dz,
-// C_ij(z) = int phi_i(u) phi_j(u - z) du (K-point rule on the overlap of the two cells),
-// outer integral by 24-point Gauss-Legendre panels of width <= 0.5/sqrt(b) around the peak.
-__global__ void k_tblock(int n, const int *item_term, const long long *item_delta, const double *bvals, double pre,
-                         DevBasis B, const double *gx, const double *gw, double *out) {
-    const int it = blockIdx.x;
-    if (it >= n) return;
-    const int K = B.K, K2 = K * K, tid = threadIdx.x;
-    __shared__ double pu[MAXK * MAXK], pv[MAXK * MAXK], wq[MAXK];
-    const double b = bvals[item_term[it]];
-    const double delta = (double)item_delta[it];
-    const double zc = -delta;
-    const double R = sqrt(GAUSS_CUT_D / b);
-    const double pw = (b > 4.0) ? 0.5 / sqrt(b) : 0.25;
-    double acc = 0.0;
-    for (int half = 0; half < 2; half++) {
-        const double lo = half == 0 ? -1.0 : 0.0, hi = half == 0 ? 0.0 : 1.0;
-        const double a0 = fmax(lo, zc - R), a1 = fmin(hi, zc + R);
-        if (a1 <= a0) continue;
-        int np = (int)ceil((a1 - a0) / pw);
-        if (np < 1) np = 1;
-        const double ph = (a1 - a0) / np;
-        for (int p = 0; p < np; p++) {
-            const double p0 = a0 + p * ph;
-            for (int q = 0; q < 24; q++) {
-                const double z = p0 + ph * gx[q];
-                const double g = exp(-b * (delta + z) * (delta + z)) * ph * gw[q];
-                if (g == 0.0) continue;
-                const double ulo = fmax(0.0, z), uhi = fmin(1.0, 1.0 + z);
-                __syncthreads();
-                if (tid < K) {
-                    double v[MAXK];
-                    d_phi(B, ulo + (uhi - ulo) * B.qx[tid], v);
-                    for (int i = 0; i < K; i++) pu[tid * K + i] = v[i];
-                    wq[tid] = (uhi - ulo) * B.qw[tid];
-                } else if (tid < 2 * K) {
-                    const int q2 = tid - K;
-                    double v[MAXK];
-                    d_phi(B, ulo + (uhi - ulo) * B.qx[q2] - z, v);
-                    for (int i = 0; i < K; i++) pv[q2 * K + i] = v[i];
-                }
-                __syncthreads();
-                if (tid < K2) {
-                    const int i = tid / K, j = tid % K;
-                    double c = 0.0;
-                    for (int qq = 0; qq < K; qq++) c += wq[qq] * pu[qq * K + i] * pv[qq * K + j];
-                    acc += g * c;
-                }
-            }
-        }
-    }
-    if (tid < K2) out[(size_t)it * K2 + tid] = acc * pre;
-}
-
-
-// Same block by moments: t[i][j] = pre * sum_h sum_p ccoef[h][i][j][p] M_h[p] with
-// M_h[p] = int_half exp(-b (delta+z)^2) L_p(t(z)) dz on the same Gauss-Legendre panels.
+// t[i][j] = pre * int_{-1}^{1} exp(-b (delta+z)^2) C_ij(z) dz, C_ij(z) = int phi_i(u) phi_j(u - z) du,
+// by moments: t[i][j] = pre * sum_h sum_p ccoef[h][i][j][p] M_h[p] with
+// M_h[p] = int_half exp(-b (delta+z)^2) L_p(t(z)) dz on 24-point Gauss-Legendre panels of width
+// <= 0.5/sqrt(b) around the peak.
 // One wave per block: lanes take quadrature points independently and keep the 2 x 2K
 // moments in registers; one wave reduction, then the K^2 entries.
 template <int K>
@@ -363,7 +289,8 @@ __global__ void __launch_bounds__(256) k_project_gauss(const MulItem *items, Pro
         for (int e = tid; e < nt * 3 * N; e += 256) {
             const int tt = e / (3 * N), dim = (e / N) % 3, p = e % N, t = t0 + tt;
             const int bit = p / K, q = p % K;
-            const double x0 = geo.lo[dim] + hc * (double)(2 * it.l[dim] + bit);
+            const int l = dim == 0 ? it.l[0] : dim == 1 ? it.l[1] : it.l[2];
+            const double x0 = geo.lo[dim] + hc * (double)(2 * l + bit);
             const double u = x0 + hc * B.qx[q] - center[3 * t + dim];
             double pv = 0.0, up = 1.0;
 #pragma unroll
@@ -1704,13 +1631,6 @@ hipError_t launch_move_groups(hipStream_t s, int npairs, const int *from_to, dou
 }
 
 // ----------------------------------------------------------------- launchers
-
-hipError_t launch_tblock(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
-                         double pre, const DevBasis &B, const double *gx, const double *gw, double *out) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tblock, dim3(n), dim3(128), 0, s, n, item_term, item_delta, b, pre, B, gx, gw, out);
-    return hipGetLastError();
-}
 
 hipError_t launch_tblock_mom(hipStream_t s, int n, const int *item_term, const long long *item_delta, const double *b,
                              const double *pre, int K, const double *ccoef, const double *gx, const double *gw,

@@ -136,10 +136,10 @@ struct NodeRegs {
 #pragma unroll
         for (int w = 0; w < PER; w++) v[w] = *src(min(threadIdx.x + 256u * w, NV - 1u));
     }
-    __device__ inline void store(double *T) const {
+    __device__ inline void store(double *T, unsigned t = threadIdx.x) const {
 #pragma unroll
         for (int w = 0; w < PER; w++) {
-            const int e = threadIdx.x + 256 * w;
+            const int e = t + 256 * w;
             if (NV % 256 == 0 || e < NV) T[padded_index<K>(e / (K * K * K), e % (K * K * K))] = v[w];
         }
     }
@@ -297,7 +297,7 @@ k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B
     constexpr int PER = (N3 + 255) / 256, MP = (3 * N2 + 255) / 256;
     extern __shared__ double smem[];
     __shared__ double wsum[4][8];
-    double *T = smem, *M = T + L::SIZE;  // M: 3 N x N (descents: 2 x 3 K x N on the way)
+    double *T = smem, *M = T + L::SIZE;  // M: 3 N x N
     const MulItem it = items[blockIdx.x];
     const MulJobDev J = jobs[it.job];
     double va[PER];
@@ -307,26 +307,23 @@ k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B
         NodeRegs<K> in;
         in.load([&](unsigned e) { return src + e; });
         if (steps > 0) {
-            double *F = M, *S = M + 3 * KN;
+            double *F = T, *S = T + 3 * KN;  // (the tensor is not there yet)
             descent_matrices<K>(F, S, B.W, it.l[0], it.l[1], it.l[2], steps);
-            double m[MP];  // E (its scaling columns) x descent, in registers until F is no longer read
+            // E (its scaling columns) x descent
 #pragma unroll
             for (int w = 0; w < MP; w++) {
                 const int e = threadIdx.x + 256 * w;
-                double s = 0.0;
                 if (e < 3 * N2) {
                     const int dim = e / N2, r = (e % N2) / N, p = e % N;
+                    double s = 0.0;
 #pragma unroll
                     for (int j = 0; j < K; j++) s += B.E[r * N + j] * F[dim * KN + j * N + p];
+                    M[e] = s;
                 }
-                m[w] = s;
             }
             __syncthreads();
-#pragma unroll
-            for (int w = 0; w < MP; w++)
-                if (threadIdx.x + 256 * w < 3 * N2) M[threadIdx.x + 256 * w] = m[w];
         }
-        in.store(T);
+        in.store(T, K <= 9 ? threadIdx.x : thread_here());  // (K = 10: the registers are full)
         Rows<N, N> m;
         if (steps == 0) m.load(B.E, N);
         __syncthreads();
@@ -336,9 +333,10 @@ k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B
             __syncthreads();
         }
         if (q == 0) {
+            const unsigned t0 = K <= 9 ? threadIdx.x : thread_here();
 #pragma unroll
             for (int w = 0; w < PER; w++) {
-                const int e = threadIdx.x + 256 * w;
+                const int e = t0 + 256 * w;
                 va[w] = N3 % 256 == 0 || e < N3 ? T[(e / N) * P + e % N] : 0.0;
             }
             __syncthreads();
@@ -422,10 +420,11 @@ __global__ void __launch_bounds__(256) k_sum(const SumItem *items, const SumSrc 
         // the next two terms given at the node itself
         while (q < it.nsrc && src[q].steps) q++;
         if (q == it.nsrc) break;
-        const SumSrc ta = src[q++];
+        const int qa = q++;
         while (q < it.nsrc && src[q].steps) q++;
         const bool two = q < it.nsrc;
-        const SumSrc tb = two ? src[q++] : ta;
+        const SumSrc ta = src[qa], tb = src[two ? q : qa];
+        q++;
         NodeRegs<K> va, vb;
         va.load([&](unsigned e) { return ta.p + e; });
         if (two) vb.load([&](unsigned e) { return tb.p + e; });
