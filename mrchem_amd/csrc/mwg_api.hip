@@ -1587,6 +1587,10 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         for (size_t j = 0; j < jobs.size(); j++) scan_input(j);
     else
         for_each_job(jobs.size(), scan_input);
+    bool infinite = false;  // an input with an infinite norm (one that is no number survives no screening)
+    for (const JobH &J : jobs)
+        for (const auto &m : J.fmax)
+            for (double v : m) infinite = infinite || std::isinf(v);
     for (size_t j = 0; j < jobs.size(); j++) {
         JobH &J = jobs[j];
         // output trees reach at most a level or so below their inputs: build one more
@@ -1927,7 +1931,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
             else
                 HC(launch_enum_mixed(s, 1, K, WCAP, 0, dw, djt, C.tabs.p, gs, C.thread_off.p, C.gtotal.p, C.gofs.p,
                                      C.slices64.p, C.slices.p, dsum, C.nodes.p, C.tasks.p, C.stasks.p, nwp, queue + 2));
-            HC(launch_contract_slices64(s, K, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dw, djt, C.slices64.p,
+            HC(launch_contract_slices64(s, K, infinite, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dw, djt, C.slices64.p,
                                         C.genPool.p, C.slots64.p, dts));
             if (mixed) {
                 const int tpb = mfma_tasks_per_block(K);
@@ -2223,7 +2227,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
                                      C.gofs.p, C.slices64.p, C.slices.p, dsum, C.nodes.p, C.tasks.p, C.stasks.p));
             // contraction time: the device clock at the first workgroup of the first and the
             // last workgroup of the last contraction kernel
-            HC(launch_contract_slices64(s, K, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dwork, djobs,
+            HC(launch_contract_slices64(s, K, infinite, 0, dsum, std::max(1, C.caps.tasks), C.tasks.p, dwork, djobs,
                                         C.slices64.p, C.genPool.p, C.slots64.p, dts));
             if (mixed) {
                 const int tpb = mfma_tasks_per_block(K);

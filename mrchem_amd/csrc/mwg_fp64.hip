@@ -10,7 +10,9 @@
 //   pass z  W[gt] += (w Z) V[gt] once per run of equal (dz, ft_z) and gt
 // (the sums are linear, so exactly the surviving combinations enter; only the order of the
 // FP64 additions differs from one combination at a time).  A list in any other order gives
-// the same result with shorter runs.
+// the same result with shorter runs.  INF: the batch has an input of infinite norm; the products with
+// zero that otherwise mask components and row ends would carry it into components that it does not
+// contribute to (they are selects then, which takes 5 to 11 % longer).
 //
 // Every pass runs on v_mfma_f64_4x4x4_4b_f64: four blocks of (4 rows) x (4 columns), 4 products
 // long, in 16 cycles, the full FP64 rate of the chip.  Lane L = 16 kq + 4 blk + r supplies
@@ -93,7 +95,7 @@ __device__ inline int f_place(int q) {
 
 }  // namespace
 
-template <int K>
+template <int K, bool INF>
 __global__ void __launch_bounds__(F64<K>::NA * 64) __attribute__((amdgpu_waves_per_eu(3)))
 k_contract_slices64(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks, const WorkItem *work,
                     const JobTab *jobs, const Slice *slices, const double *genPool, double *slots,
@@ -233,15 +235,25 @@ k_contract_slices64(int ntask_arg, const TaskSummary *sum, const SliceTask *task
                 for (int j = 0; j < G; j++)
 #pragma unroll
                     for (int l = 0; l < G; l++) t1[j][l] = mfma4(f[l][j][s], x[s], t1[j][l]);
-            // added to the components of the mask: a product with 1 or 0 (exact, no branches)
+            // added to the components of the mask: a product with 1 or 0 (exact for finite values, no
+            // branches), a select where there may be others
             const int m = F64<K>::EVEN ? mask >> gxw : mask >> gxl;
+            if constexpr (INF) {
 #pragma unroll
-            for (int p = 0; p < 4; p++) {
-                const double on1 = __hiloint2double((m >> (2 * p)) & 1 ? 0x3ff00000 : 0, 0);
+                for (int p = 0; p < 4; p++)
 #pragma unroll
-                for (int j = 0; j < G; j++)
+                    for (int j = 0; j < G; j++)
 #pragma unroll
-                    for (int l = 0; l < G; l++) U[p][j][l] = fma(t1[j][l], on1, U[p][j][l]);
+                        for (int l = 0; l < G; l++) U[p][j][l] += (m >> (2 * p)) & 1 ? t1[j][l] : 0.0;
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const double on1 = __hiloint2double((m >> (2 * p)) & 1 ? 0x3ff00000 : 0, 0);
+#pragma unroll
+                    for (int j = 0; j < G; j++)
+#pragma unroll
+                        for (int l = 0; l < G; l++) U[p][j][l] = fma(t1[j][l], on1, U[p][j][l]);
+                }
             }
             umask |= mw;
             udiff |= dw;
@@ -397,7 +409,7 @@ struct Wide {
     static constexpr int FC = (K3 / P + NT - 1) / NT, PC = (5 * K2 / P + NT - 1) / NT;
 };
 
-template <int K>
+template <int K, bool INF>
 __global__ void __launch_bounds__(Wide<K>::NT) __attribute__((amdgpu_waves_per_eu(2)))
 k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tasks, const WorkItem *work,
                      const JobTab *jobs, const Slice *slices, const double *genPool, double *slots,
@@ -491,6 +503,15 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
 #pragma unroll
             for (int s = 0; s < KS; s++) a[r][s] = blk[ar[r] + s];
     };
+    // entries of a row beyond K, times a zero of A: what another component left there may be infinite
+    auto row_end = [&](double (&v)[T][KS]) {
+        if constexpr (INF) {
+#pragma unroll
+            for (int t = 0; t < T; t++)
+#pragma unroll
+                for (int s = 0; s < KS; s++) v[t][s] = ib + s < K ? v[t][s] : 0.0;
+        }
+    };
     // zeros behind the rows of f and of the blocks; finite values wherever a row's end is read
     for (int q = tid; q < 2 * ((D::SLOT + 1) & ~1); q += NT) (&stage[0][0])[q] = 0.0;
     for (int q = tid; q < D::XCH + D::AR; q += NT) xch[q] = 0.0;
@@ -529,13 +550,22 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
                 for (int r = 0; r < RG; r++)
 #pragma unroll
                     for (int t = 0; t < T; t++) t1[r][t] = mfma4(X[r][s], f[t][s], t1[r][t]);
+            if constexpr (INF) {  // (as above)
 #pragma unroll
-            for (int p = 0; p < 4; p++) {  // a product with 1 or 0 (exact, no branches)
-                const double on1 = __hiloint2double((mask >> (2 * p)) & 1 ? 0x3ff00000 : 0, 0);
+                for (int p = 0; p < 4; p++)
 #pragma unroll
-                for (int r = 0; r < RG; r++)
+                    for (int r = 0; r < RG; r++)
 #pragma unroll
-                    for (int t = 0; t < T; t++) U[p][r][t] = fma(t1[r][t], on1, U[p][r][t]);
+                        for (int t = 0; t < T; t++) U[p][r][t] += (mask >> (2 * p)) & 1 ? t1[r][t] : 0.0;
+            } else {
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const double on1 = __hiloint2double((mask >> (2 * p)) & 1 ? 0x3ff00000 : 0, 0);
+#pragma unroll
+                    for (int r = 0; r < RG; r++)
+#pragma unroll
+                        for (int t = 0; t < T; t++) U[p][r][t] = fma(t1[r][t], on1, U[p][r][t]);
+                }
             }
             umask |= mask;
         }
@@ -566,6 +596,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
                         for (int t = 0; t < T; t++)
 #pragma unroll
                             for (int s = 0; s < KS; s++) v[t][s] = Ul[p * S * K * ROW + yr[t] + s];
+                        row_end(v);
 #pragma unroll
                         for (int s = 0; s < KS; s++)
 #pragma unroll
@@ -609,6 +640,7 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
                         for (int t = 0; t < T; t++)
 #pragma unroll
                             for (int s = 0; s < KS; s++) v[t][s] = Vl[(p * K2 + zc[t]) * ROW + ib + s];
+                        row_end(v);
 #pragma unroll
                         for (int s = 0; s < KS; s++)
 #pragma unroll
@@ -635,24 +667,27 @@ k_contract_slices64w(int ntask_arg, const TaskSummary *sum, const SliceTask *tas
 }
 
 template <int K>
-static void launch_slices64(hipStream_t s, int ntask, const TaskSummary *sum, int nt, const SliceTask *tasks,
-                            const WorkItem *work, const JobTab *jobs, const Slice *slices, const double *genPool,
-                            double *slots, unsigned long long *ts) {
-    if constexpr (F64<K>::G <= 2)
-        hipLaunchKernelGGL(k_contract_slices64<K>, dim3(nt + (ts ? 1 : 0)), dim3(F64<K>::NA * 64), 0, s, ntask, sum,
-                           tasks, work, jobs, slices, genPool, slots, ts);
-    else
-        hipLaunchKernelGGL(k_contract_slices64w<K>, dim3((nt + 7) / 8 * 16 + (ts ? 1 : 0)), dim3(Wide<K>::NT), 0, s,
-                           ntask, sum, tasks, work, jobs, slices, genPool, slots, ts);
+static void launch_slices64(bool infinite, hipStream_t s, int ntask, const TaskSummary *sum, int nt,
+                            const SliceTask *tasks, const WorkItem *work, const JobTab *jobs, const Slice *slices,
+                            const double *genPool, double *slots, unsigned long long *ts) {
+    if constexpr (F64<K>::G <= 2) {
+        const auto kern = infinite ? k_contract_slices64<K, true> : k_contract_slices64<K, false>;
+        hipLaunchKernelGGL(kern, dim3(nt + (ts ? 1 : 0)), dim3(F64<K>::NA * 64), 0, s, ntask, sum, tasks, work, jobs,
+                           slices, genPool, slots, ts);
+    } else {
+        const auto kern = infinite ? k_contract_slices64w<K, true> : k_contract_slices64w<K, false>;
+        hipLaunchKernelGGL(kern, dim3((nt + 7) / 8 * 16 + (ts ? 1 : 0)), dim3(Wide<K>::NT), 0, s, ntask, sum, tasks,
+                           work, jobs, slices, genPool, slots, ts);
+    }
 }
 
-hipError_t launch_contract_slices64(hipStream_t s, int K, int ntask, const TaskSummary *sum, int grid,
+hipError_t launch_contract_slices64(hipStream_t s, int K, bool infinite, int ntask, const TaskSummary *sum, int grid,
                                     const SliceTask *tasks, const WorkItem *work, const JobTab *jobs,
                                     const Slice *slices, const double *genPool, double *slots,
                                     unsigned long long *ts) {
     const int nt = sum ? grid : ntask;
     if (nt <= 0) return hipSuccess;
-    MWG_DISPATCH_K(K, launch_slices64<KK>(s, ntask, sum, nt, tasks, work, jobs, slices, genPool, slots, ts));
+    MWG_DISPATCH_K(K, (launch_slices64<KK>(infinite, s, ntask, sum, nt, tasks, work, jobs, slices, genPool, slots, ts)));
     return hipGetLastError();
 }
 

@@ -218,8 +218,9 @@ hipError_t launch_enum(hipStream_t s, int mode, int K, int nw, int nparts, const
                        const TaskSummary *sum, const NodeSched *nodes, SliceTask *tasks, const int *nwp = nullptr,
                        int *queue = nullptr);
 // FP64 slice contraction (mwg_fp64.hip).  With sum: the task count is read on the device; grid
-// (tasks) covers the capacity.  With ts: an extra first workgroup stamps the start.
-hipError_t launch_contract_slices64(hipStream_t s, int K, int ntask, const TaskSummary *sum, int grid,
+// (tasks) covers the capacity.  infinite: an input has an infinite norm.  With ts: an extra first
+// workgroup stamps the start.
+hipError_t launch_contract_slices64(hipStream_t s, int K, bool infinite, int ntask, const TaskSummary *sum, int grid,
                                     const SliceTask *tasks, const WorkItem *work, const JobTab *jobs,
                                     const Slice *slices, const double *genPool, double *slots,
                                     unsigned long long *ts = nullptr);
