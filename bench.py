@@ -533,7 +533,8 @@ def main():
             best, dtype = resP, (mixed_dtype(args.k) if mixed_ok else "f64")
 
     # algorithmic flops: the plain FP64 method's surviving tuples x 6 (k+1)^4 (the same work for
-    # every variant); issued flops count what the variant's kernels actually execute
+    # every variant); counted flops: FP64 combinations as three passes each (the FP64 kernels
+    # share passes and issue fewer), MFMA slices as issued
     K = args.k + 1
     F = res64["tuples_per_step"]
     alg = F * 6.0 * K ** 4
@@ -550,7 +551,7 @@ def main():
                     kernel=(kern + " + k_contract_slices64 + k_reduce_slots") if dtype != "f64"
                     else "k_contract_slices64 + k_reduce_slots",
                     plain_tuples_per_step=F, alg_flops_per_tuple=6.0 * K ** 4,
-                    issued_tflops=(best["flops_per_step"] / tc / 1e12) if tc > 0 else None,
+                    counted_tflops=(best["flops_per_step"] / tc / 1e12) if tc > 0 else None,
                     contraction_ms_per_step=1e3 * tc,
                     launches_per_step=best["iters"],
                     traffic_per_step=per_launch * best["iters"] if per_launch else None,

@@ -91,7 +91,7 @@ const char *mwg_last_error(mwg_ctx ctx);
 int mwg_sync(mwg_ctx ctx);
 /* contraction task granularity (no reference counterpart: MRCPP threads over output
  * nodes with OpenMP): at most this many FP64 slices per workgroup task (1..4096; an iteration
- * with fewer than 2048 tasks' worth of slices uses smaller tasks, down to 8; a task size is
+ * with fewer than 1024 tasks' worth of slices uses smaller tasks, down to 8; a task size is
  * raised where the slots of an iteration would exceed 8 GiB) and MFMA slices per
  * workgroup task (0..4096, 0 = automatic; k = 7 uses at most 256, 128 when automatic;
  * k = 9 sizes automatic tasks from each refinement iteration's slice total, 16 to 128

@@ -589,7 +589,7 @@ struct TreeH {
     }
     void refresh_norms() {  // device norms -> host, square norm
         hipStream_t s = mra->ctx->stream;
-        HC(launch_norms(s, n(), nullptr, coef.p, norm.p, K3()));
+        HC(launch_norms(s, n(), coef.p, norm.p, K3()));
         cnorm.resize(8 * (size_t)n());
         norm.download(cnorm.data(), 8 * (size_t)n(), s);
         sqnorm_from_cnorm();
@@ -2265,7 +2265,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         PT.lap("enum_count");
         launch_schedule();
         // A capacity (or the generated-node pool) was too small: grow and run again.  A
-        // partial-slot need beyond SLOT_BUDGET raises this iteration's FP64 task size
+        // need of slots beyond SLOT_BUDGET raises this iteration's FP64 task size
         // instead (fewer, larger tasks: only the summation grouping changes).
         for (int attempt = 0; hsum.overflow; attempt++) {
             if (attempt == 12) throw Error(MWG_ERR_RANGE, "work-list schedule sizing failed");

@@ -10,7 +10,8 @@
 //   pass z  W[gt] += (w Z) V[gt] once per run of equal (dz, ft_z) and gt
 // (the sums are linear, so exactly the surviving combinations enter; only the order of the
 // FP64 additions differs from one combination at a time).  A list in any other order gives
-// the same result with shorter runs.  INF: the batch has an input of infinite norm; the products with
+// the same result with shorter runs: the FP64 slices of a mixed apply come in the order of the
+// candidates, each thread's after another's, and pay all three passes nearly every time.  INF: the batch has an input of infinite norm; the products with
 // zero that otherwise mask components and row ends would carry it into components that it does not
 // contribute to (they are selects then, which takes 5 to 11 % longer).
 //

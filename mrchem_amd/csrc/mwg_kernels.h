@@ -164,7 +164,7 @@ struct NSItems {
 };
 hipError_t launch_nsblocks(hipStream_t s, long long first, long long n, const NSItems &items, const double *t1,
                            const double *W, int K);
-hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3);
+hipError_t launch_norms(hipStream_t s, int n, const double *coef, double *norm, int K3);
 // two nodes' coefficients (skip0: without their scaling parts)
 struct DotPair {
     const double *a, *b;

@@ -14,18 +14,6 @@
 
 namespace mwg {
 
-// global-address-space views: uniform loads through these become scalar loads
-typedef const double __attribute__((address_space(1))) gdouble;
-typedef const float __attribute__((address_space(1))) gfloat;
-
-__device__ inline int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
-
-__device__ inline void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // sum over the block of one value per thread, same order every call (all threads get it)
 __device__ inline double block_sum_256(double v, double *wsum) {
 #pragma unroll
@@ -160,11 +148,10 @@ __global__ void k_nsblocks(long long first, NSItems items, const double *t1, con
     }
 }
 
-// component norms of listed nodes (a workgroup per node, a wave per two components)
-__global__ void __launch_bounds__(256) k_norms(int n, const int *nodes, const double *coef, double *norm, int K3) {
-    const int i = blockIdx.x;
-    if (i >= n) return;
-    const int node = nodes ? nodes[i] : i, lane = threadIdx.x & 63;
+// component norms of a tree's nodes (a workgroup per node, a wave per two components)
+__global__ void __launch_bounds__(256) k_norms(int n, const double *coef, double *norm, int K3) {
+    const int node = blockIdx.x, lane = threadIdx.x & 63;
+    if (node >= n) return;
     const double *p = coef + (size_t)node * 8 * K3;
     for (int c = threadIdx.x >> 6; c < 8; c += 4) {
         double s = 0.0;
@@ -1648,9 +1635,9 @@ hipError_t launch_nsblocks(hipStream_t s, long long first, long long n, const NS
     return hipGetLastError();
 }
 
-hipError_t launch_norms(hipStream_t s, int n, const int *nodes, const double *coef, double *norm, int K3) {
+hipError_t launch_norms(hipStream_t s, int n, const double *coef, double *norm, int K3) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_norms, dim3(n), dim3(256), 0, s, n, nodes, coef, norm, K3);
+    hipLaunchKernelGGL(k_norms, dim3(n), dim3(256), 0, s, n, coef, norm, K3);
     return hipGetLastError();
 }
 

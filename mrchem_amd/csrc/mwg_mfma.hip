@@ -11,7 +11,7 @@
 // survive the screening, is summed over the task's slices (k = 7: FP32 over at most 64
 // slices per wave, then FP64 over the waves; k = 9: FP64 per slice), and a task's sum goes
 // to one node slot (8 K^3 FP64) that k_reduce_slots adds, in slot order, to the
-// node's FP64 tuple partials.  A task is a run of slices of one output node, one task
+// sum of the node's FP64 tasks.  A task is a run of slices of one output node, one task
 // per 256-thread workgroup.
 //
 // Instruction layout of v_mfma_f32_16x16x32_f16 (D = A B + C): lane L supplies A[L % 16]

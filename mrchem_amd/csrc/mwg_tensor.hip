@@ -288,7 +288,9 @@ __global__ void __launch_bounds__(256) k_gen_compute(int first, const int *first
 // quadrature points of the 8 children, product, quadrature projection, compression.
 // Reconstruction and evaluation are one 2K x 2K matrix per dimension (B.E), for an input that
 // ends above the node together with its descent; projection and compression are another (B.C,
-// weights included).  The values of a wait in registers while b uses the tensor.
+// weights included).  The values of a wait in registers while b uses the tensor.  At K = 10 these, a
+// node on its way to LDS and the matrix rows fill the registers: with the addresses of both places
+// held as well it spilled 106 of them (a launch of 21 orbital products 1277 us, 987 now).
 template <int K>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K <= 8 ? 3 : 2)))
 k_multiply(const MulItem *items, const MulJobDev *jobs, ProjGeom geo, DevBasis B, double *compact) {
