@@ -30,12 +30,12 @@
 // with no exchange between waves.  G^3 instructions per pass.
 //
 // What bounds it: the FP64 pipe, which the products share with the other vector instructions
-// (a v_fma_f64 and a product do not overlap).  Per slice and wave at K = 8 about 19 products
-// (304 cycles) and 60 other vector instructions (240 cycles); the counters show the pipe busy
-// about 65 % of the time, the rest are LDS latencies and the barriers with three waves per
-// SIMD.  One combination at a time on v_fma_f64, each with its three passes through LDS, took
+// (a v_fma_f64 and a product do not overlap).  Per slice and wave at K = 8 about 18 products
+// (290 cycles) and 78 other vector instructions (310 cycles), the staging and the schedule among
+// them; the counters show the pipe busy 52 % of the time, the rest are LDS latencies and the
+// barriers with at most three waves per SIMD (2.3 on average, 35 % of their cycles waiting).  One combination at a time on v_fma_f64, each with its three passes through LDS, took
 // 4.29 ms on the contractions of five k = 7 Helmholtz applies at prec 1e-6 (5.55 M combinations
-// in 1.05 M slices, 32 TFLOP/s of 6 K^4 flops each); this takes 2.10 ms (65).  Loading the operands
+// in 1.05 M slices, 32 TFLOP/s of 6 K^4 flops each); this takes 2.06 ms (66).  Loading the operands
 // straight from global memory in their lane layout (a line per lane) took 3.8 ms, four staged
 // slices per buffer (two workgroups per CU instead of three) 2.5.
 #include <hip/hip_ext.h>
@@ -393,8 +393,8 @@ k_contract_slices64(int ntask_arg, const TaskSummary *sum, const SliceTask *task
 // Helmholtz applies at prec 1e-6 (6.6 M combinations in 1.2 M slices): contractions 14.7 ms one
 // combination at a time, 11.2 with the split over rows a' above (one wave per SIMD), 10.1 here with a
 // select per entry of A and a branch per exchanged value, 9.6 with neither: the staged rows end in
-// zeros, and what has no place goes to a row's padding.  Now the FP64 pipe is busy 46 % of the
-// time and LDS 51 %, with the two waves per SIMD that the accumulators leave room for.
+// zeros, and what has no place goes to a row's padding.  Now the FP64 pipe is busy 47 % of the
+// time and LDS 47 %, with the two waves per SIMD that the accumulators leave room for.
 template <int K>
 struct Wide {
     static constexpr int RG = (K + 3) / 4, KS = RG;  // row groups; products per lane group
