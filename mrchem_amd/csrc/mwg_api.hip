@@ -3391,7 +3391,7 @@ int mwg_tree_eval(mwg_tree tree, int64_t n, const double *xyz, double *out) {
             bool inside = true;
             for (int d = 0; d < 3; d++) {
                 u0[d] = (p[d] - M.lo(d)) / (M.sfac * std::ldexp(1.0, -M.n0));
-                if (u0[d] < 0.0 || u0[d] >= M.boxes[d]) inside = false;
+                if (!(u0[d] >= 0.0 && u0[d] < M.boxes[d])) inside = false;  // (or no number)
             }
             if (!inside) {
                 out[pi] = 0.0;
