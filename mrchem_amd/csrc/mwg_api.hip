@@ -1169,6 +1169,17 @@ static void build_oper(OperH &O, MraH *mra, double mu, double prec) {
     }
 }
 
+// The outputs of a call that fails on the way hold nodes but not their coefficients (or no memory
+// at all, which a later kernel would read): they are left empty.
+struct OutGuard {
+    std::vector<TreeH *> outs;
+    bool done = false;
+    ~OutGuard() {
+        if (!done)
+            for (TreeH *t : outs) t->clear();
+    }
+};
+
 // ------------------------------------------------------------------ projection
 
 // read-back of n doubles at the start of the context's device block, through pinned memory
@@ -1223,6 +1234,7 @@ static void project_adaptive(TreeH &T, double prec, LaunchFn launch, const std::
                              const std::vector<double> *gauss_center) {
     MraH &M = *T.mra;
     Ctx &C = *M.ctx;
+    OutGuard guard{{&T}};
     T.make_roots();
     std::vector<int> work = T.roots;
     double sNorm = 0.0, wNorm = 0.0;
@@ -1279,6 +1291,7 @@ static void project_adaptive(TreeH &T, double prec, LaunchFn launch, const std::
         iter++;
     }
     compress_trees(C, M, {&T});
+    guard.done = true;
 }
 
 // ------------------------------------------------------------------ apply
@@ -1587,6 +1600,8 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         for (size_t j = 0; j < jobs.size(); j++) scan_input(j);
     else
         for_each_job(jobs.size(), scan_input);
+    OutGuard guard;
+    for (JobH &J : jobs) guard.outs.push_back(J.out);
     bool infinite = false;  // an input with an infinite norm (one that is no number survives no screening)
     for (const JobH &J : jobs)
         for (const auto &m : J.fmax)
@@ -2556,6 +2571,7 @@ static void apply_jobs(std::vector<JobH> &jobs, int max_iter, unsigned flags, st
         st.device_loop = dl_done ? 1 : 0;
         st.flops = fl * (double)jobs[j].tuples_fp64 + slice_flops(K) * (double)jobs[j].slices;
     }
+    guard.done = true;
 }
 
 
@@ -2658,6 +2674,8 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
         if (J.a->n() == 0 || J.b->n() == 0) throw Error(MWG_ERR_STATE, "multiply: empty input tree");
         nodes += J.a->n() + J.b->n();
     }
+    OutGuard guard;
+    for (MulJob &J : jobs) guard.outs.push_back(J.out);
     for_jobs_of(jobs.size(), nodes, [&](size_t j) { jobs[j].union_grid(M.maxDepth); });
     // room for the refinement that the last batch needed beyond the union grids (a tree that
     // grows level by level is allocated and copied at each), where memory is not short: that batch
@@ -2706,6 +2724,7 @@ static void multiply_batch(std::vector<MulJob> &jobs) {
     }
     C.mul_growth = 1.1 * n_out / n_union;
     compress_trees(C, M, trees);
+    guard.done = true;
 }
 
 // A linear combination out = sum of coef_k f_k on the union grid of its terms.
@@ -2760,9 +2779,12 @@ static void sum_group(SumJob *jobs, size_t njobs) {
     MraH &M = *jobs[0].out->mra;
     Ctx &C = *M.ctx;
     const size_t B8 = 8 * (size_t)M.B.K3;
+    OutGuard guard;
     size_t nodes = 0;
-    for (size_t j = 0; j < njobs; j++)
+    for (size_t j = 0; j < njobs; j++) {
+        guard.outs.push_back(jobs[j].out);
         for (TreeH *t : jobs[j].f) nodes += t->n();
+    }
     for_jobs_of(njobs, nodes, [&](size_t j) { jobs[j].union_grid(); });
     for (size_t j = 0; j < njobs; j++) jobs[j].out->ensure_dev(jobs[j].out->n());
     struct Part {  // nodes i0 .. i1 - 1 of a combination
@@ -2819,6 +2841,7 @@ static void sum_group(SumJob *jobs, size_t njobs) {
         jobs[j].out->sqnorm_from_cnorm();
         std::vector<SumJob::Src>().swap(jobs[j].src);
     }
+    guard.done = true;
 }
 
 // Linear combinations (mrcpp::add): all inputs are checked first, then the combinations are taken in
@@ -3091,6 +3114,7 @@ int mwg_tree_import(mwg_tree tree, int64_t n, const int *depth, const int64_t *l
         const MraH &M = *T.mra;
         const std::string bad = check_tree_layout(M.boxes, M.maxDepth, n, depth, lr);
         if (!bad.empty()) throw Error(MWG_ERR_ARG, "tree import: " + bad);
+        OutGuard guard{{&T}};
         T.reserve_host((size_t)n);
         NodeIndex index;
         for (int64_t i = 0; i < n; i++) {
@@ -3105,6 +3129,7 @@ int mwg_tree_import(mwg_tree tree, int64_t n, const int *depth, const int64_t *l
         HC(hipMemcpyAsync(T.coef.p, coefs, (size_t)n * 8 * T.K3() * sizeof(double), hipMemcpyHostToDevice,
                           C->stream));
         T.refresh_norms();
+        guard.done = true;
     });
 }
 

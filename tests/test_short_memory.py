@@ -1,4 +1,4 @@
-"""Products on a card whose memory is nearly used up.
+"""Calls on a card whose memory is nearly used up.
 
 A batch of products that fits at its own size runs, whatever ran on the context before it.  Most of
 the card is held by an allocation that no kernel touches; the calls that run out of memory fail
@@ -62,3 +62,33 @@ def test_products_after_products_that_grew():
         held.free()
         gc.collect()
         ctx.trim()
+
+
+def test_outputs_of_a_call_that_runs_out_of_memory_are_empty():
+    """(they would hold nodes without coefficients, which the next kernel reads)"""
+    from mrchem_amd import mrcpp as G
+    ctx = G.Context(0)
+    mra = G.mra_from(configs.BOX20, 9, ctx=ctx)
+    orbs, _, _ = configs.orbitals(3, n_orb=2)
+    fine = G.project(1e-8, G.FunctionTree(mra), orbs[0])
+    one = _products(G, mra, fine, 1)[0]
+    n = int(2.4 * GIB / (one.getNNodes() * 64000)) + 1
+    held = _Held(ctx, GIB)
+    try:
+        for call in (lambda o: G.multiply_batch(0.5, o, 1.0, [fine] * n, [fine] * n),
+                     lambda o: G.add_batch(o, [[(1.0, fine)]] * n)):
+            outs = [G.FunctionTree(mra) for _ in range(n)]
+            with pytest.raises(G.MwgError, match="allocation"):
+                call(outs)
+            assert all(o.getNNodes() == 0 for o in outs)
+            with pytest.raises(G.MwgError, match="empty"):
+                G.add(G.FunctionTree(mra), 1.0, outs[0], 1.0, fine)
+            outs = None
+            gc.collect()
+            ctx.trim()
+    finally:
+        held.free()
+        gc.collect()
+        ctx.trim()
+    two = _products(G, mra, fine, 2)
+    assert all(np.array_equal(t.export()[2], one.export()[2]) for t in two)
