@@ -33,7 +33,8 @@
 // (a v_fma_f64 and a product do not overlap).  Per slice and wave at K = 8 about 18 products
 // (290 cycles) and 78 other vector instructions (310 cycles), the staging and the schedule among
 // them; the counters show the pipe busy 52 % of the time, the rest are LDS latencies and the
-// barriers with at most three waves per SIMD (2.3 on average, 35 % of their cycles waiting).  One combination at a time on v_fma_f64, each with its three passes through LDS, took
+// barriers with at most three waves per SIMD (2.3 on average, 35 % of their cycles waiting).
+// One combination at a time on v_fma_f64, each with its three passes through LDS, took
 // 4.29 ms on the contractions of five k = 7 Helmholtz applies at prec 1e-6 (5.55 M combinations
 // in 1.05 M slices, 32 TFLOP/s of 6 K^4 flops each); this takes 2.06 ms (66).  Loading the operands
 // straight from global memory in their lane layout (a line per lane) took 3.8 ms, four staged
